@@ -2,7 +2,7 @@
 //
 // Layout in HBM (structure of arrays, element arrays in Hilbert order, river
 // arrays in the caller's order):
-//   element statics   18 x double[ne]      area .. rzd
+//   element statics   17 x double[ne]      area .. rzd
 //   edge statics       4 x double[3*ne]    edge, nabrdist, nabr_x, nabr_y  (index j*ne+p)
 //   edge codes         int32[3*ne]         nb (neighbour code, boundary type folded in)
 //   per-step inputs    4 x double[ne] + double[3*ne]
@@ -43,7 +43,7 @@ struct alignas(64) NbrRec {
 
 struct ElemDev {
   double *area, *zmin, *zmax, *depth, *ksath, *ksatv, *kinfv, *dinf, *alpha,
-      *beta, *porosity, *dmac, *kmach, *kmacv, *areafv, *areafh, *rough, *rzd;
+      *beta, *porosity, *dmac, *kmac, *kmacv, *areafh, *rough, *rzd;   // kmac: kmach areafv + ksath (1 - areafv)
   double *edge, *nabrdist, *nabr_x, *nabr_y;  // [3*ne]
   int32_t *nb;                                // [3*ne]
   // per-step inputs

@@ -80,26 +80,43 @@ __global__ __launch_bounds__(kBlock) void k_soil_prev(int ne, SoilDev s, const d
   s.prev[ne + p] = y[2L * ne + p];
 }
 
+// KrFunc (src/soil.c:8-13) and the retention curve's slope dpsi/dtheta of
+// WDfCnd at relative saturation f in (0, 1).  With m = 1 - 1/beta and
+// A = f^(1/m), the reference's product of powers
+//   (f^(-1/m) - 1)^(-m) f^(-(1/m + 1)) = ((1 - A) / A)^(-m) / (A f)
+// is 1 / (A (1 - A)^m), whose (1 - A)^m is also KrFunc's: two logarithms and
+// two exponentials for both instead of five of each.
+__device__ __forceinline__ void kr_slope(double f, double e1, double m, double scale, double *kr, double *slope) {
+  double lo, tlo;
+  const double hi = ln_pos(f, &lo);
+  double thi = mul_pair(e1, hi, lo, &tlo);
+  const double A = exp_pair(thi, tlo);
+  const double qm = xpow(1.0 - A, m);
+  const double g = 1.0 - qm;
+  *kr = sqrt(f) * g * g;
+  *slope = scale / (A * qm);
+}
+
+// What WDfCnd (src/noah/noah.c:2813-2861) takes from the soil alone, the same
+// in every layer of a column.
+struct WdfSoil {
+  double range, e1, m, scale, ksatv, smcmin, sicemax, vkwgt;
+};
+
 // WDfCnd: src/noah/noah.c:2813-2861
-__device__ void wdf_cnd(double *wdf, double *wcnd, double smc, double sicemax, double smcmax, double smcmin,
-                        double ksatv, double alpha, double beta) {
-  double factr1 = 0.05 / (smcmax - smcmin);
-  double factr2 = (smc - smcmin) / (smcmax - smcmin);
+__device__ __forceinline__ void wdf_cnd(double *wdf, double *wcnd, double smc, const WdfSoil &w) {
+  double factr1 = 0.05 / w.range;
+  double factr2 = (smc - w.smcmin) / w.range;
   factr2 = (factr2 > 1.0 - 5.0e-4) ? 1.0 - 5.0e-4 : factr2;
   factr2 = (factr2 < 0.0 + 5.0e-4) ? 5.0e-4 : factr2;
   factr1 = (factr1 < factr2) ? factr1 : factr2;
-  const double expon = 1.0 - 1.0 / beta;
-  double satkfunc = kr_func(beta, factr2);
-  double dpsidsm = (1.0 - expon) / alpha / expon / (smcmax - smcmin) *
-                   xpow(xpow(factr2, -1.0 / expon) - 1.0, -expon) * xpow(factr2, -(1.0 / expon + 1.0));
-  *wcnd = ksatv * satkfunc;
+  double satkfunc, dpsidsm;
+  kr_slope(factr2, w.e1, w.m, w.scale, &satkfunc, &dpsidsm);
+  *wcnd = w.ksatv * satkfunc;
   *wdf = *wcnd * dpsidsm;
-  if (sicemax > 0.0) {
-    const double vkwgt = 1.0 / (1.0 + xpow(500.0 * sicemax, 3.0));
-    satkfunc = kr_func(beta, factr1);
-    dpsidsm = (1.0 - expon) / alpha / expon / (smcmax - smcmin) *
-              xpow(xpow(factr1, -1.0 / expon) - 1.0, -expon) * xpow(factr1, -(1.0 / expon + 1.0));
-    *wdf = vkwgt * *wdf + (1.0 - vkwgt) * dpsidsm * satkfunc * ksatv;
+  if (w.sicemax > 0.0) {
+    kr_slope(factr1, w.e1, w.m, w.scale, &satkfunc, &dpsidsm);
+    *wdf = w.vkwgt * *wdf + (1.0 - w.vkwgt) * dpsidsm * satkfunc * w.ksatv;
   }
 }
 
@@ -223,9 +240,23 @@ __global__ __launch_bounds__(kBlock) void k_noah_soil(int ne, SoilDev s, ElemDev
         fcr = 1.0 - exp(-acrt) * sum;
       }
       const double pddum = s.infil[p];
+      WdfSoil ws;
+      ws.range = smcmax - smcmin;
+      ws.e1 = beta / (beta - 1.0);
+      ws.m = (beta - 1.0) / beta;
+      const double expon = 1.0 - 1.0 / beta;
+      ws.scale = (1.0 - expon) / alpha / expon / ws.range;
+      ws.ksatv = ksatv;
+      ws.smcmin = smcmin;
+      ws.sicemax = sicemax;
+      ws.vkwgt = 1.0;
+      if (sicemax > 0.0) {
+        const double i500 = 500.0 * sicemax;
+        ws.vkwgt = 1.0 / (1.0 + i500 * i500 * i500);
+      }
       double wdf, wcnd;
       double dsmdz = (sh2o[0] - sh2o[1]) / (-0.5 * zsoil[1]);
-      wdf_cnd(&wdf, &wcnd, sh2o[0], sicemax, smcmax, smcmin, ksatv, alpha, beta);
+      wdf_cnd(&wdf, &wcnd, sh2o[0], ws);
       double ddz = 1.0 / (-0.5 * zsoil[1]);
       ai[0] = 0.0;
       bi[0] = wdf * ddz / (-zsoil[0]);
@@ -241,7 +272,7 @@ __global__ __launch_bounds__(kBlock) void k_noah_soil(int ne, SoilDev s, ElemDev
           if (k + 1 < ML && k < nsoil - 1) {
             const double denom = zsoil[k - 1] - zsoil[k + 1];
             dsmdz2 = (sh2o[k] - sh2o[k + 1]) / (denom * 0.5);
-            wdf_cnd(&wdf2, &wcnd2, sh2o[k], sicemax, smcmax, smcmin, ksatv, alpha, beta);
+            wdf_cnd(&wdf2, &wcnd2, sh2o[k], ws);
             ddz2 = 2.0 / denom;
             ci[k] = -wdf2 * ddz2 / denom2;
           } else {

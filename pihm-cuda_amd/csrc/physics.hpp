@@ -37,7 +37,7 @@ PIHM_DEV double clamp0(double v) { return (v >= 0.0) ? v : 0.0; }
 PIHM_DEV double surf_h(double surfeqv) {
   double surfh;
   if (surfeqv < 0.0) surfh = 0.0;
-  else if (surfeqv <= 0.5 * DEPRSTG) surfh = sqrt(2.0 * DEPRSTG * surfeqv);
+  else if (surfeqv <= 0.5 * DEPRSTG) surfh = sqrt_pos(2.0 * DEPRSTG * surfeqv);
   else surfh = DEPRSTG + (surfeqv - 0.5 * DEPRSTG);
   return surfh;
 }
@@ -56,17 +56,39 @@ PIHM_DEV double psi_vg(double satn, double alpha, double beta) {
   return -xpow(xpow(1.0 / satn, beta / (beta - 1.0)) - 1.0, 1.0 / beta) / alpha;
 }
 
-// EffKh: src/lat_flow.c:248-277
-PIHM_DEV double eff_kh(double depth, double dmac, double kmach, double areafv,
-                       double ksath, double gw) {
+// Psi and KrFunc of one saturation in [SATMIN, 1], the powers and their order
+// those of psi_vg and kr_func, in two chains side by side.  Exponents that no
+// soil has (beta <= 1.0034) take the functions one by one.
+PIHM_DEV void psi_kr(double satn, double alpha, double beta, double *psi, double *kr) {
+  const double e1 = fdiv(beta, beta - 1.0);
+  if (!(e1 > 1.0 && e1 < 300.0)) {
+    *psi = psi_vg(satn, alpha, beta);
+    *kr = kr_func(beta, satn);
+    return;
+  }
+  const Recip rb = recip_of(beta);
+  const double s[2] = {satn, fdiv(1.0, satn)}, e[2] = {e1, e1};
+  double ab[2], r[2];
+  xpow_n<2>(s, e, ab);
+  const double x[2] = {1.0 - ab[0], ab[1] - 1.0};
+  const double y[2] = {quot(beta - 1.0, rb), quot(1.0, rb)};
+  xpow_n<2>(x, y, r);
+  const double f = 1.0 - r[0];
+  *psi = fdiv(-r[1], alpha);
+  *kr = sqrt_mid(satn) * f * f;
+}
+
+// EffKh: src/lat_flow.c:248-277; kmac = kmach * areafv + ksath * (1 - areafv),
+// which is static, comes from the mesh upload
+PIHM_DEV double eff_kh(double depth, double dmac, double kmac, double ksath, double gw) {
   gw = (gw > 0.0) ? gw : 0.0;
   if (gw > depth - dmac) {
-    double k1 = kmach * areafv + ksath * (1.0 - areafv);
+    double k1 = kmac;
     double k2 = ksath;
     double d1, d2;
     if (gw > depth) { d1 = dmac; d2 = depth - dmac; }
     else { d1 = gw - (depth - dmac); d2 = depth - dmac; }
-    return (k1 * d1 + k2 * d2) / (d1 + d2);
+    return fdiv(k1 * d1 + k2 * d2, d1 + d2);
   }
   return ksath;
 }
@@ -85,7 +107,7 @@ PIHM_DEV double avg_kv(double dmac, double ksatv, double kmacv, double areafh,
     d2 = dmac - deficit;
     k3 = ksatv; d3 = gw - (dmac - deficit);
   }
-  return (k1 * d1 + k2 * d2 + k3 * d3) / (d1 + d2 + d3);
+  return fdiv(k1 * d1 + k2 * d2 + k3 * d3, d1 + d2 + d3);
 }
 
 // EffKinf: src/vert_flow.c:211-270
@@ -114,8 +136,8 @@ PIHM_DEV double eff_kinf(double kinfv, double kmacv, double areafh, double dh_by
 // DhByDl: src/lat_flow.c:239-246
 PIHM_DEV double dh_by_dl(double a0, double a1, double a2, double b0, double b1,
                          double b2, double h0, double h1, double h2) {
-  return -1.0 * (a2 * (h1 - h0) + a1 * (h0 - h2) + a0 * (h2 - h1)) /
-         (b2 * (a1 - a0) + b1 * (a0 - a2) + b0 * (a2 - a1));
+  return fdiv(-1.0 * (a2 * (h1 - h0) + a1 * (h0 - h2) + a0 * (h2 - h1)),
+              b2 * (a1 - a0) + b1 * (a0 - a2) + b0 * (a2 - a1));
 }
 
 // OverLandFlow: src/lat_flow.c:279-283 (literal exponent 0.6666667)
@@ -138,23 +160,18 @@ PIHM_DEV double avg_h_sub(double diff, double hsub, double hnabr) {
   return avg_h;
 }
 
-// RiverCroSectArea: src/river_flow.c:520-548 (unknown shapes are rejected
-// when the context is built, where the reference exits at run time)
-PIHM_DEV double riv_cs_area(int order, double depth, double coeff) {
-  depth = (depth > 0.0) ? depth : 0.0;
+// Sections other than rectangles, kept out of line: their powers and
+// logarithms, inlined at every use, were four fifths of the one-launch RHS's
+// code.
+__device__ __attribute__((noinline)) inline double riv_cs_area_other(int order, double depth, double coeff) {
   switch (order) {
-    case RECTANGLE: return depth * coeff;
     case TRIANGLE: return depth * depth / coeff;
     case QUADRATIC: return 4.0 * depth * sqrt(depth) / (3.0 * sqrt(coeff));
     default: return 3.0 * xpow(depth, 4.0 / 3.0) / (2.0 * xpow(coeff, 1.0 / 3.0));
   }
 }
-
-// RiverPerim: src/river_flow.c:550-583
-PIHM_DEV double riv_perim(int order, double depth, double coeff) {
-  depth = (depth > 0.0) ? depth : 0.0;
+__device__ __attribute__((noinline)) inline double riv_perim_other(int order, double depth, double coeff) {
   switch (order) {
-    case RECTANGLE: return 2.0 * depth + coeff;
     case TRIANGLE: return 2.0 * depth * sqrt(1.0 + coeff * coeff) / coeff;
     case QUADRATIC:
       return sqrt(depth * (1.0 + 4.0 * coeff * depth) / coeff) +
@@ -166,6 +183,19 @@ PIHM_DEV double riv_perim(int order, double depth, double coeff) {
                          xpow(1.0 + 9.0 * xpow(coeff, 2.0 / 3.0) * depth, 0.5)) /
                      (9.0 * xpow(coeff, 1.0 / 3.0))));
   }
+}
+
+// RiverCroSectArea: src/river_flow.c:520-548 (unknown shapes are rejected
+// when the context is built, where the reference exits at run time)
+PIHM_DEV double riv_cs_area(int order, double depth, double coeff) {
+  depth = (depth > 0.0) ? depth : 0.0;
+  return (order == RECTANGLE) ? depth * coeff : riv_cs_area_other(order, depth, coeff);
+}
+
+// RiverPerim: src/river_flow.c:550-583
+PIHM_DEV double riv_perim(int order, double depth, double coeff) {
+  depth = (depth > 0.0) ? depth : 0.0;
+  return (order == RECTANGLE) ? 2.0 * depth + coeff : riv_perim_other(order, depth, coeff);
 }
 
 // OvlFlowElemToRiver: src/river_flow.c:185-255

@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(RhsArgs a, int nbe) {
   // first group of loads
   const double ys = y[lp], yg = y[2 * ix.ne + lp];
   const double zmax = e.zmax[p], zmin = e.zmin[p], depth = e.depth[p], dmac = e.dmac[p];
-  const double kmach = e.kmach[p], areafv = e.areafv[p], ksath = e.ksath[p];
+  const double kmac = e.kmac[p], ksath = e.ksath[p];
   int c[3] = {0, 0, 0};
   double nx[3] = {0.0, 0.0, 0.0}, ny[3] = {0.0, 0.0, 0.0};
   if (diff) {
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(RhsArgs a, int nbe) {
   const double surfh = surf_h(s);
   const double head = zmax + surfh;
   const double gwz = g + zmin;
-  const double effkh = eff_kh(depth, dmac, kmach, areafv, ksath, g);
+  const double effkh = eff_kh(depth, dmac, kmac, ksath, g);
 
   double sfmag = 0.0;
   if (diff) {
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kBlock) void k_prep(RhsArgs a, int nbe) {
     }
     const double dhdx = dh_by_dl(ny[0], ny[1], ny[2], nx[0], nx[1], nx[2], h[0], h[1], h[2]);
     const double dhdy = dh_by_dl(nx[0], nx[1], nx[2], ny[0], ny[1], ny[2], h[0], h[1], h[2]);
-    sfmag = sqrt(dhdx * dhdx + dhdy * dhdy);
+    sfmag = sqrt_pos(dhdx * dhdx + dhdy * dhdy);
   }
   // the six per-call fields of the record, as three 16-byte stores
   double2 *rp = reinterpret_cast<double2 *>(&a.e.rec[p]);
@@ -230,7 +230,7 @@ template <bool B>
 __device__ __forceinline__ double effkh_of(const RhsArgs &a, const Ix &ix, int q) {
   const ElemDev &e = a.e;
   const double g = clamp0(ix.y[2 * ix.ne + (q - ix.eoff)]);
-  return eff_kh(e.depth[q], e.dmac[q], e.kmach[q], e.areafv[q], e.ksath[q], g);
+  return eff_kh(e.depth[q], e.dmac[q], e.kmac[q], e.ksath[q], g);
 }
 
 // Where an element's per-call neighbour values come from.
@@ -239,9 +239,9 @@ __device__ __forceinline__ double effkh_of(const RhsArgs &a, const Ix &ix, int q
 //   TileSrc:   the tile's records in LDS (codes: LDS slots) and the bank
 //              fluxes evaluated here, from the element's own record.
 struct GlobalSrc {
-  static constexpr bool kGatherFirst = true;   // neighbour records from HBM: all three loads at once
   const RhsArgs &a;
   int p;
+  __device__ __forceinline__ int own() const { return p; }
   __device__ __forceinline__ NbrRec self() const { return a.e.rec[p]; }
   __device__ __forceinline__ int code(int j) const { return a.e.nb[j * a.ne + p]; }
   __device__ __forceinline__ NbrRec nbr(int c) const { return a.e.rec[c]; }
@@ -274,13 +274,13 @@ struct LdsRecs {
 constexpr int kTile = 128;            // elements per tile = threads per block of the one-launch RHS (two wavefronts)
 
 struct TileSrc {
-  static constexpr bool kGatherFirst = false;  // from LDS: each edge's record when its turn comes
   const RhsArgs &a;
   LdsRecs srec;         // LDS records of the tile and its halo
   const int32_t *lnb;   // neighbour slots of the tile's elements
   int p, i;
   const double *bk;     // LDS: the bank fluxes of each tile element's first river edge (ovl, then sub)
   const int *bkj;       // LDS: that edge (-1: none)
+  __device__ __forceinline__ int own() const { return i; }
   __device__ __forceinline__ NbrRec self() const { return srec.get(i); }
   __device__ __forceinline__ int code(int j) const { return lnb[j * a.ne + p]; }
   __device__ __forceinline__ NbrRec nbr(int c) const { return srec.get(c); }
@@ -323,25 +323,35 @@ struct ElemIn {
   double bcv[3], hov[3];
 };
 
+// What the unsaturated zone's terms read, loaded ahead of the rest.
+struct SoilIn {
+  double yu, depth, dinf, dmac, alpha, beta;
+};
+__device__ __forceinline__ SoilIn load_soil_in(const RhsArgs &a, int p, const Ix &ix) {
+  const ElemDev &e = a.e;
+  return SoilIn{ix.y[ix.ne + (p - ix.eoff)], e.depth[p], e.dinf[p], e.dmac[p], e.alpha[p], e.beta[p]};
+}
+
 // Loads in two groups: the element's own entries and edge codes, then what the
 // codes point at (a wavefront waits for memory twice, not once per edge).
 template <bool N, class Src>
-__device__ __forceinline__ ElemIn load_elem_in(const RhsArgs &a, int p, const Ix &ix, const Src &src) {
+__device__ __forceinline__ ElemIn load_elem_in(const RhsArgs &a, int p, const Ix &ix, const Src &src,
+                                               const SoilIn &so) {
   const int ne = a.ne;
   const ElemDev &e = a.e;
   ElemIn in;
-  in.yu = ix.y[ix.ne + (p - ix.eoff)];
-  in.area = e.area[p]; in.zmax = e.zmax[p]; in.zmin = e.zmin[p];
-  in.depth = e.depth[p]; in.dinf = e.dinf[p]; in.rzd = e.rzd[p];
+  in.yu = so.yu; in.depth = so.depth; in.dinf = so.dinf; in.dmac = so.dmac; in.alpha = so.alpha; in.beta = so.beta;
+#pragma unroll
+  for (int j = 0; j < 3; j++) in.c[j] = src.code(j);
+  in.area = e.area[p]; in.zmax = e.zmax[p]; in.zmin = e.zmin[p]; in.rzd = e.rzd[p];
   in.edir = e.edir[p]; in.ett = e.ett[p]; in.pcpdrp = e.pcpdrp[p]; in.ws0 = e.ws0s[p];
-  in.alpha = e.alpha[p]; in.beta = e.beta[p]; in.kinfv = e.kinfv[p]; in.kmacv = e.kmacv[p];
-  in.areafh = e.areafh[p]; in.dmac = e.dmac[p]; in.ksatv = e.ksatv[p]; in.porosity = e.porosity[p];
+  in.kinfv = e.kinfv[p]; in.kmacv = e.kmacv[p];
+  in.areafh = e.areafh[p]; in.ksatv = e.ksatv[p]; in.porosity = e.porosity[p];
   if (N) {
     in.gwet = e.gwet[p]; in.sh2o0 = e.sh2o0[p]; in.smcmin = e.smcmin[p]; in.fcr = e.fcr[p];
   }
 #pragma unroll
   for (int j = 0; j < 3; j++) {
-    in.c[j] = src.code(j);
     in.dist[j] = e.nabrdist[j * ne + p];
     in.edge[j] = e.edge[j * ne + p];
   }
@@ -359,105 +369,104 @@ __device__ __forceinline__ ElemIn load_elem_in(const RhsArgs &a, int p, const Ix
   return in;
 }
 
-// An element's fluxes come in three parts, which the two-kernel RHS runs one
-// after the other in one thread and the one-launch RHS in two wavefronts:
+// An element's fluxes come in three parts:
 //   elem_lateral   LateralFlow over the three edges (src/lat_flow.c:29-63),
 //                  with the overland flux carried from the previous call on
 //                  river edges, the sum Infil's application rate starts from,
 //                  then this call's bank fluxes on river edges;
-//   elem_vert_pre  EtExtract's split and the unsaturated zone's saturation,
-//                  pressure head and conductivity;
-//   elem_vert_post Infil, Recharge and the element ODEs.
+//   elem_soil      the unsaturated zone's saturation, pressure head and
+//                  conductivity;
+//   elem_vert      EtExtract's split, Infil, Recharge and the element ODEs.
 // N: the reference built with _NOAH_ (src/hydrol.c:43-56,79-84;
 // src/vert_flow.c:16-19,94-98), single solves only.
 struct LatOut {
-  double ovl[3], sub[3];   // this call's edge fluxes
   double asum;             // sum of -ovl / area with the carried fluxes on river edges
+  double qo[3], qs[3];     // this call's ovl / area and sub / area
   double out;              // ovl + sub over the domain-boundary edges (closure)
 };
 
+// The three faces are worked in step and without branches, an edge that is
+// not an element neighbour as a face to the element itself; boundary and river
+// edges then replace theirs.  A wavefront alone on its SIMD (small meshes)
+// waits for each result of a dependent chain, and three chains side by side
+// wait once; with more wavefronts the three share the polynomials' scalar
+// operands.  Quotients by one distance, and by the area, share the reciprocal.
+// Every value is that of the reference's expressions, rounding included.
 template <bool B, class Src>
 __device__ __forceinline__ LatOut elem_lateral(const RhsArgs &a, int p, const Ix &ix, const Src &src,
                                                const ElemIn &in, const NbrRec &me) {
   const int ne = a.ne;
-  NbrRec nrec[3];
-  if constexpr (Src::kGatherFirst) {
-#pragma unroll
-    for (int j = 0; j < 3; j++)
-      if (in.c[j] >= 0) nrec[j] = src.nbr(in.c[j]);
-  }
-  const double area = in.area, zmax = in.zmax, zmin = in.zmin;
-  const double g = me.gw;
-  const double surfh = me.surfh;
-  LatOut o;
-  double *ovl = o.ovl, *sub = o.sub;
-  bool bank = false;
-  bool bnd[3] = {false, false, false};
+  const bool kin = a.surf_mode == KINEMATIC;
+  double ovl[3], sub[3], hs[3], gh[3], den[3];
 #pragma unroll
   for (int j = 0; j < 3; j++) {
-    const int c = in.c[j];
-    bnd[j] = nb_is_bound(c);
-    if (c >= 0) {
-      if constexpr (!Src::kGatherFirst) nrec[j] = src.nbr(c);
-      const NbrRec &nr = nrec[j];
-      // SubFlowElemToElem: src/lat_flow.c:285-309
-      {
-        const double diff_h = me.gwz - nr.gwz;
-        const double avg_h = avg_h_sub(diff_h, g, nr.gw);
-        const double grad_h = diff_h / in.dist[j];
-        const double avg_ksat = 0.5 * (me.effkh + nr.effkh);
-        sub[j] = avg_ksat * grad_h * avg_h * in.edge[j];
-      }
-      // OvlFlowElemToElem: src/lat_flow.c:311-338
-      {
-        double avg_sf = 0.5 * (me.sfmag + nr.sfmag);
-        const double diff_h = (a.surf_mode == KINEMATIC) ? zmax - nr.zmax : me.head - nr.head;
-        const double avg_h = avg_hsurf(diff_h, surfh, nr.surfh);
-        const double grad_h = diff_h / in.dist[j];
-        if (a.surf_mode == KINEMATIC) avg_sf = (grad_h > 0.0) ? grad_h : GRADMIN;
-        else avg_sf = (avg_sf > GRADMIN) ? avg_sf : GRADMIN;
-        const double avg_rough = 0.5 * (me.rough + nr.rough);
-        const double crossa = avg_h * in.edge[j];
-        ovl[j] = overland_flow(avg_h, grad_h, avg_sf, crossa, avg_rough);
-      }
-    } else if (nb_is_bound(c)) {
-      // BoundFluxElem: src/lat_flow.c:340-382
-      ovl[j] = 0.0;
-      const int bt = nb_bc_sign(c);
-      if (bt == 0) {
-        sub[j] = 0.0;
-      } else if (bt > 0) {
-        const double diff_h = me.gwz - in.bcv[j];
-        const double avg_h = avg_h_sub(diff_h, g, in.bcv[j] - zmin);
-        const double grad_h = diff_h / in.dist[j];
-        sub[j] = me.effkh * grad_h * avg_h * in.edge[j];
+    const NbrRec nr = src.nbr(in.c[j] >= 0 ? in.c[j] : src.own());
+    const Recip rd = recip_of(in.dist[j]);
+    // SubFlowElemToElem: src/lat_flow.c:285-309
+    const double dg = me.gwz - nr.gwz;
+    const double avg_ksat = 0.5 * (me.effkh + nr.effkh);
+    sub[j] = avg_ksat * quot(dg, rd) * avg_h_sub(dg, me.gw, nr.gw) * in.edge[j];
+    // OvlFlowElemToElem: src/lat_flow.c:311-338
+    const double dh = kin ? in.zmax - nr.zmax : me.head - nr.head;
+    hs[j] = avg_hsurf(dh, me.surfh, nr.surfh);
+    gh[j] = quot(dh, rd);
+    double avg_sf = 0.5 * (me.sfmag + nr.sfmag);
+    if (kin) avg_sf = (gh[j] > 0.0) ? gh[j] : GRADMIN;
+    else avg_sf = (avg_sf > GRADMIN) ? avg_sf : GRADMIN;
+    den[j] = sqrt_pos(avg_sf) * (0.5 * (me.rough + nr.rough));
+    ovl[j] = 0.0;
+  }
+  if (hs[0] > 0.0 || hs[1] > 0.0 || hs[2] > 0.0) {
+    // OverLandFlow: src/lat_flow.c:279-283 (literal exponent 0.6666667)
+    const double ex[3] = {0.6666667, 0.6666667, 0.6666667};
+    double pw[3];
+    xpow_n<3>(hs, ex, pw);
+#pragma unroll
+    for (int j = 0; j < 3; j++) ovl[j] = fdiv((hs[j] * in.edge[j]) * pw[j] * gh[j], den[j]);
+  }
+  const Recip ra = recip_of(in.area);
+  LatOut o;
+  o.out = 0.0;
+  double first[3];                                 // what Infil's application rate reads, over the area
+#pragma unroll
+  for (int j = 0; j < 3; j++) first[j] = o.qo[j] = quot(ovl[j], ra);
+  if (in.c[0] < 0 || in.c[1] < 0 || in.c[2] < 0) {
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+      const int c = in.c[j];
+      if (c >= 0) continue;
+      if (nb_is_bound(c)) {
+        // BoundFluxElem: src/lat_flow.c:340-382
+        ovl[j] = first[j] = 0.0;
+        const int bt = nb_bc_sign(c);
+        if (bt == 0) {
+          sub[j] = 0.0;
+        } else if (bt > 0) {
+          const double diff_h = me.gwz - in.bcv[j];
+          sub[j] = me.effkh * fdiv(diff_h, in.dist[j]) * avg_h_sub(diff_h, me.gw, in.bcv[j] - in.zmin) * in.edge[j];
+        } else {
+          sub[j] = -in.bcv[j];
+        }
+        o.out += ovl[j] + sub[j];      // volume rates crossing the element's outer boundary
       } else {
-        sub[j] = -in.bcv[j];
+        // river edge: Infil reads the overland flux carried from the previous
+        // call (src/vert_flow.c:59-62); this call's bank fluxes
+        // (src/river_flow.c:113-183) replace it, and the new overland flux is
+        // carried to the next call (src/river_flow.c:159-182)
+        const int slot = -c - 1;
+        first[j] = quot(in.hov[j], ra);
+        src.bank(ix, j, slot, me, in.zmax, in.zmin, ovl[j], sub[j]);
+        a.r.hid_ovl[slot] = ovl[j];
       }
-    } else {
-      // river edge: the overland flux carried from the previous call is what
-      // Infil reads (src/vert_flow.c:59-62); both fluxes are replaced below.
-      bank = true;
-      ovl[j] = in.hov[j];
-      sub[j] = 0.0;
+      o.qo[j] = quot(ovl[j], ra);
     }
   }
   // Infil's application rate starts from the lateral inflow (src/vert_flow.c:56-66)
   o.asum = 0.0;
 #pragma unroll
-  for (int j = 0; j < 3; j++) o.asum += -ovl[j] / area;
-  // River edges: this call's bank fluxes (src/river_flow.c:113-183) replace
-  // the carried overland flux that Infil uses, and the new overland flux is
-  // carried to the next call (src/river_flow.c:159-182).
-  if (bank) {
-#pragma unroll
-    for (int j = 0; j < 3; j++) {
-      if (nb_is_river(in.c[j])) {
-        const int slot = -in.c[j] - 1;
-        src.bank(ix, j, slot, me, zmax, zmin, ovl[j], sub[j]);
-        a.r.hid_ovl[slot] = ovl[j];
-      }
-    }
+  for (int j = 0; j < 3; j++) {
+    o.asum += -first[j];
+    o.qs[j] = quot(sub[j], ra);
   }
   if (a.record) {
 #pragma unroll
@@ -466,69 +475,41 @@ __device__ __forceinline__ LatOut elem_lateral(const RhsArgs &a, int p, const Ix
       a.rec.sub[j * ne + p] = sub[j];
     }
   }
-  // volume rates crossing the element's outer boundary
-  o.out = 0.0;
-#pragma unroll
-  for (int j = 0; j < 3; j++)
-    if (bnd[j]) o.out += ovl[j] + sub[j];
   return o;
 }
 
-struct VertPre {
-  double edir_s, edir_u, edir_g, ett_u, ett_g;
+// Unsaturated-zone terms shared by Infil and Recharge (same deficit and
+// saturation in both, src/vert_flow.c:93-102 and :149-156); g is the clamped
+// groundwater.
+struct SoilTerms {
   double deficit, satn, psi_raw, kr;
   bool wet_bottom;
 };
 
-template <bool N>
-__device__ __forceinline__ VertPre elem_vert_pre(const ElemIn &in, const NbrRec &me) {
-  const double depth = in.depth, dinf = in.dinf, rzd = in.rzd;
-  const double edir = in.edir, ett = in.ett;
-  const double u = clamp0(in.yu);
-  const double g = me.gw;
-  const double surfh = me.surfh;
-  VertPre v;
-  // EtExtract: src/hydrol.c:33-97
-  if (N) {
-    // no direct evaporation from ponded water; the saturated zone's share of
-    // transpiration, GwTransp (src/noah/lsm_func.c:163-185), is fixed per step
-    v.edir_s = 0.0;
-    if (g > depth - dinf) { v.edir_u = 0.0; v.edir_g = edir; }
-    else { v.edir_u = edir; v.edir_g = 0.0; }
-    const double gwet = in.gwet;
-    v.ett_u = (1.0 - gwet) * ett;
-    v.ett_g = gwet * ett;
-  } else {
-    if (surfh >= DEPRSTG) { v.edir_s = edir; v.edir_u = 0.0; v.edir_g = 0.0; }
-    else if (g > depth - dinf) { v.edir_s = 0.0; v.edir_u = 0.0; v.edir_g = edir; }
-    else { v.edir_s = 0.0; v.edir_u = edir; v.edir_g = 0.0; }
-    if (g > depth - rzd) { v.ett_u = 0.0; v.ett_g = ett; }
-    else { v.ett_u = ett; v.ett_g = 0.0; }
-  }
-  // Unsaturated-zone terms shared by Infil and Recharge (same deficit and
-  // saturation in both, src/vert_flow.c:93-102 and :149-156).
-  v.wet_bottom = g > depth - dinf;
+__device__ __forceinline__ SoilTerms elem_soil(const SoilIn &in, double g) {
+  SoilTerms v;
+  v.wet_bottom = g > in.depth - in.dinf;
   v.deficit = 0.0; v.satn = 0.0; v.psi_raw = 0.0; v.kr = 0.0;
   if (!v.wet_bottom) {
-    v.deficit = depth - g;
-    double satn = u / v.deficit;
+    v.deficit = in.depth - g;
+    double satn = fdiv(clamp0(in.yu), v.deficit);
     satn = (satn > 1.0) ? 1.0 : satn;
     satn = (satn < SATMIN) ? SATMIN : satn;
     v.satn = satn;
-    v.psi_raw = psi_vg(satn, in.alpha, in.beta);
-    v.kr = kr_func(in.beta, satn);
+    psi_kr(satn, in.alpha, in.beta, &v.psi_raw, &v.kr);
   }
   return v;
 }
 
 template <bool B, bool N>
-__device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix &ix, const ElemIn &in,
-                                               const NbrRec &me, const VertPre &v, const LatOut &lat) {
+__device__ __forceinline__ void elem_vert(const RhsArgs &a, int p, const Ix &ix, const ElemIn &in,
+                                          const NbrRec &me, const SoilTerms &v, const LatOut &lat) {
   const int ne = a.ne;
   const int lp = p - ix.eoff;
   double *ydot = ix.ydot;
-  const double area = in.area, zmax = in.zmax, zmin = in.zmin;
-  const double depth = in.depth, dinf = in.dinf;
+  const double area = in.area, zmax = in.zmax;
+  const double depth = in.depth, dinf = in.dinf, rzd = in.rzd;
+  const double edir = in.edir, ett = in.ett;
   const double pcpdrp = in.pcpdrp, ws0 = in.ws0;
   const double beta = in.beta, kinfv = in.kinfv, kmacv = in.kmacv;
   const double areafh = in.areafh, dmac = in.dmac, ksatv = in.ksatv, porosity = in.porosity;
@@ -538,6 +519,25 @@ __device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix
   const bool wet_bottom = v.wet_bottom;
   const double deficit = v.deficit, satn = v.satn, psi_raw = v.psi_raw, kr = v.kr;
 
+  // EtExtract: src/hydrol.c:33-97
+  double edir_s, edir_u, edir_g, ett_u, ett_g;
+  if (N) {
+    // no direct evaporation from ponded water; the saturated zone's share of
+    // transpiration, GwTransp (src/noah/lsm_func.c:163-185), is fixed per step
+    edir_s = 0.0;
+    if (wet_bottom) { edir_u = 0.0; edir_g = edir; }
+    else { edir_u = edir; edir_g = 0.0; }
+    const double gwet = in.gwet;
+    ett_u = (1.0 - gwet) * ett;
+    ett_g = gwet * ett;
+  } else {
+    if (surfh >= DEPRSTG) { edir_s = edir; edir_u = 0.0; edir_g = 0.0; }
+    else if (wet_bottom) { edir_s = 0.0; edir_u = 0.0; edir_g = edir; }
+    else { edir_s = 0.0; edir_u = edir; edir_g = 0.0; }
+    if (g > depth - rzd) { ett_u = 0.0; ett_g = ett; }
+    else { ett_u = ett; ett_g = 0.0; }
+  }
+
   // Infil: src/vert_flow.c:33-130
   double infil;
   if (u + g > depth) {
@@ -546,12 +546,12 @@ __device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix
     double applrate = lat.asum;
     applrate = (applrate > 0.0) ? applrate : 0.0;
     applrate += pcpdrp;
-    double wetfrac = surfh / DEPRSTG;
+    double wetfrac = fdiv(surfh, DEPRSTG);
     wetfrac = (wetfrac > 0.0) ? wetfrac : 0.0;
     wetfrac = (wetfrac < 1.0) ? wetfrac : 1.0;
     double dh_by_dz, kinf;
     if (wet_bottom) {
-      dh_by_dz = (surfh + zmax - (g + zmin)) / (0.5 * (surfh + dinf));
+      dh_by_dz = fdiv(surfh + zmax - me.gwz, 0.5 * (surfh + dinf));
       dh_by_dz = (surfh <= 0.0 && dh_by_dz > 0.0) ? 0.0 : dh_by_dz;
       // KrFunc(beta, 1) is exactly 1 for beta > 1 (1^m = 1, 0^(1/m) = 0)
       const double satkfunc = (beta > 1.0) ? 1.0 : kr_func(beta, 1.0);
@@ -562,21 +562,20 @@ __device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix
       if (N) {
         // saturation of the top soil layer; smcmax - smcmin is the porosity
         // (src/init_soil.c:34-36)
-        isatn = (in.sh2o0 - in.smcmin) / porosity;
+        isatn = fdiv(in.sh2o0 - in.smcmin, porosity);
         isatn = (isatn > 1.0) ? 1.0 : isatn;
         isatn = (isatn < SATMIN) ? SATMIN : isatn;
-        ipsi = psi_vg(isatn, in.alpha, beta);
-        ikr = kr_func(beta, isatn);
+        psi_kr(isatn, in.alpha, beta, &ipsi, &ikr);
       }
       const double psi_u = (ipsi > PSIMIN) ? ipsi : PSIMIN;
       const double h_u = psi_u + zmax - 0.5 * dinf;
-      dh_by_dz = (surfh + zmax - h_u) / (0.5 * (surfh + dinf));
+      dh_by_dz = fdiv(surfh + zmax - h_u, 0.5 * (surfh + dinf));
       dh_by_dz = (surfh <= 0.0 && dh_by_dz > 0.0) ? 0.0 : dh_by_dz;
       kinf = eff_kinf(kinfv, kmacv, areafh, dh_by_dz, ikr, isatn, applrate, surfh);
       infil = kinf * dh_by_dz;
       infil = (infil > 0.0) ? infil : 0.0;
     }
-    const double infil_max = applrate + ((ws0 > 0.0) ? ws0 / ix.dt : 0.0);
+    const double infil_max = applrate + ((ws0 > 0.0) ? fdiv(ws0, ix.dt) : 0.0);
     infil = (infil > infil_max) ? infil_max : infil;
     infil *= wetfrac;
   }
@@ -587,7 +586,7 @@ __device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix
   if (wet_bottom) {
     rechg = infil;
   } else {
-    const double dh_by_dz = (0.5 * deficit + psi_raw) / (0.5 * (deficit + g));
+    const double dh_by_dz = fdiv(0.5 * deficit + psi_raw, 0.5 * (deficit + g));
     const double kavg = avg_kv(dmac, ksatv, kmacv, areafh, deficit, g, kr);
     rechg = kavg * dh_by_dz;
     rechg = (rechg > 0.0 && u <= 0.0) ? 0.0 : rechg;
@@ -600,33 +599,34 @@ __device__ __forceinline__ void elem_vert_post(const RhsArgs &a, int p, const Ix
 
   // element ODEs: src/ode.c:121-149
   double dys = 0.0, dyu = 0.0, dyg = 0.0;
-  dys += pcpdrp - infil - v.edir_s;
-  dyu += infil - rechg - v.edir_u - v.ett_u;
-  dyg += rechg - v.edir_g - v.ett_g;
-  dyu /= porosity;
+  dys += pcpdrp - infil - edir_s;
+  dyu += infil - rechg - edir_u - ett_u;
+  dyg += rechg - edir_g - ett_g;
+  const Recip rp = recip_of(porosity);
+  dyu = quot(dyu, rp);
 #pragma unroll
   for (int j = 0; j < 3; j++) {
-    dys -= lat.ovl[j] / area;
-    dyg -= lat.sub[j] / area;
+    dys -= lat.qo[j];
+    dyg -= lat.qs[j];
   }
-  dyg /= porosity;
+  dyg = quot(dyg, rp);
   ydot[lp] = dys;
   ydot[ix.ne + lp] = dyu;
   ydot[2 * ix.ne + lp] = dyg;
   if (isnan(dys) || isnan(dyu) || isnan(dyg)) flag_nan<B>(a, ix);
   if (!B && a.closure) {
     a.cl_e[p] = pcpdrp * area;
-    a.cl_e[ne + p] = ((((v.edir_s + v.edir_u) + v.edir_g) + v.ett_u) + v.ett_g) * area;
+    a.cl_e[ne + p] = ((((edir_s + edir_u) + edir_g) + ett_u) + ett_g) * area;
     a.cl_e[2L * ne + p] = lat.out;
   }
 }
 
 template <bool B, bool N, class Src>
-__device__ __forceinline__ void elem_core(const RhsArgs &a, int p, const Ix &ix, const Src &src, const ElemIn &in) {
+__device__ __forceinline__ void elem_core(const RhsArgs &a, int p, const Ix &ix, const Src &src, const ElemIn &in,
+                                          const SoilTerms &v) {
   const NbrRec me = src.self();
   const LatOut lat = elem_lateral<B>(a, p, ix, src, in, me);
-  const VertPre v = elem_vert_pre<N>(in, me);
-  elem_vert_post<B, N>(a, p, ix, in, me, v, lat);
+  elem_vert<B, N>(a, p, ix, in, me, v, lat);
 }
 
 template <bool B, bool N = false>
@@ -635,7 +635,9 @@ __device__ __forceinline__ void elem_flux(const RhsArgs &a, int p) {
   if (!ix.active) return;
   if (B && p - ix.eoff >= ix.ne) return;     // unused capacity of a slot
   const GlobalSrc src{a, p};
-  elem_core<B, N>(a, p, ix, src, load_elem_in<N>(a, p, ix, src));
+  const SoilIn so = load_soil_in(a, p, ix);
+  const ElemIn in = load_elem_in<N>(a, p, ix, src, so);
+  elem_core<B, N>(a, p, ix, src, in, elem_soil(so, src.self().gw));
 }
 
 template <bool B>
@@ -649,7 +651,7 @@ __device__ __forceinline__ BankView bank_view(const RhsArgs &a, const Ix &ix, in
   v.gw = g;
   v.zmin = e.zmin[q];
   v.gwz = g + v.zmin;
-  v.effkh = eff_kh(e.depth[q], e.dmac[q], e.kmach[q], e.areafv[q], e.ksath[q], g);
+  v.effkh = eff_kh(e.depth[q], e.dmac[q], e.kmac[q], e.ksath[q], g);
   v.zmax = e.zmax[q];
   return v;
 }
@@ -992,7 +994,7 @@ __device__ __forceinline__ void river_parts(const RhsArgs &a, int rb, double *xr
 // A halo or tile entry's record fields (all but the FrictSlope gradient) and
 // its head, as k_prep evaluates them.
 __device__ __forceinline__ NbrRec tile_rec(double ys, double yg, double zmax, double zmin, double depth,
-                                           double dmac, double kmach, double areafv, double ksath, double rough) {
+                                           double dmac, double kmac, double ksath, double rough) {
   const double surfh = surf_h(clamp0(ys));
   const double g = clamp0(yg);
   NbrRec r;
@@ -1000,7 +1002,7 @@ __device__ __forceinline__ NbrRec tile_rec(double ys, double yg, double zmax, do
   r.head = zmax + surfh;
   r.gw = g;
   r.gwz = g + zmin;
-  r.effkh = eff_kh(depth, dmac, kmach, areafv, ksath, g);
+  r.effkh = eff_kh(depth, dmac, kmac, ksath, g);
   r.sfmag = 0.0;
   r.rough = rough;
   r.zmax = zmax;
@@ -1028,33 +1030,42 @@ __device__ __forceinline__ double tile_sfmag(const RhsArgs &a, int s, long q, co
   }
   const double dhdx = dh_by_dl(ny[0], ny[1], ny[2], nx[0], nx[1], nx[2], h[0], h[1], h[2]);
   const double dhdy = dh_by_dl(nx[0], nx[1], nx[2], ny[0], ny[1], ny[2], h[0], h[1], h[2]);
-  return sqrt(dhdx * dhdx + dhdy * dhdy);
+  return sqrt_pos(dhdx * dhdx + dhdy * dhdy);
 }
 
 // One RHS call of a single solve in one launch.  Grid: river blocks
 // (river_parts, kRivSeg segments each), then one block per tile of kTile
 // consecutive elements (Hilbert order), two wavefronts per block: blocks run
 // independently, hiding each other's memory latency, and a tile of 128 has a
-// smaller halo per element than one of 64 (at the 200,000- and
-// 100,000-triangle meshes 128 measured 2% and 7% faster than 64; 192 and 256
-// were no better).  Each element block stages in LDS what its elements'
-// fluxes read: the heads of the tile and of its halo (the first ring of
-// outside neighbours and their outside neighbours), and the records of the
-// tile and the first ring, whose FrictSlope gradients need those heads; then
-// it runs the element fluxes from them (elem_core with TileSrc).  The loads
-// for the staging (its element's and its halo entry's record inputs, and the
-// bank fluxes of its first river edge) are issued at the start, the element's
-// flux inputs after the barriers, and each edge reads its neighbour's record
-// from LDS when its turn comes: the kernel stays within 128 VGPRs, four
-// wavefronts per SIMD, so that a 200,000-triangle RHS (3,381 wavefronts of
-// element and river blocks) runs in one round of 4,096 wavefront slots
-// instead of spilling into a second round of 3,072.  With the _NOAH_ branches
-// the cap is three wavefronts (140 VGPRs): four would spill in the element
-// path.  The halo's records are evaluated again by every tile that borders
-// them, from the same operands: every output keeps one writer, and the
-// arithmetic is that of k_prep + k_flux, bit for bit.
+// smaller halo per element than one of 64.  Each element block stages in LDS
+// what its elements' fluxes read: the heads of the tile and of its halo (the
+// first ring of outside neighbours and their outside neighbours), and the
+// records of the tile and the first ring, whose FrictSlope gradients need
+// those heads; then it runs the element fluxes from them (elem_core with
+// TileSrc).  The loads for the staging (its element's and its halo entry's
+// record inputs, and the bank fluxes of its first river edge) are issued at
+// the start, the element's flux inputs after the barriers.  The halo's records
+// are evaluated again by every tile that borders them, from the same operands:
+// every output keeps one writer, and the arithmetic is that of k_prep + k_flux,
+// bit for bit.
+//
+// What bounds it: at 200,000 triangles the phases run one after the other on
+// every SIMD, memory (about 14 us of the time, 430 B per element) and then the
+// FP64 issue of the fluxes; on small meshes the one wavefront of a SIMD walks
+// its chain of dependent operations alone.  Measured (us per evaluation, wet
+// state, 535 / 6,000 / 20,011 / 100,000 / 200,000 triangles): 14.5 / 15.3 /
+// 15.3 / 20.3 / 31.0 with one edge after the other and the compiler's
+// divisions; 11.7 / 12.6 / 12.6 / 16.9 / 27.3 with the faces and powers in
+// step, divisions that share reciprocals, and nothing spilled (157 VGPRs,
+// three wavefronts per SIMD).  Held to 128 VGPRs for a fourth wavefront it
+// spills, and a kernel with any scratch memory costs more than the wavefront
+// gives (28.1 against 25.3 in an otherwise equal pair).  Tiles of 64 / 256
+// elements: 7% / 12% slower at 20,011, equal / 4% slower at 200,000.
+//
+// The river blocks read their own copy of the arguments (ra): with one copy
+// the compiler keeps both paths' pointers in vector lanes from the start.
 template <bool N>
-__global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileArgs t, int nbe) {
+__global__ __launch_bounds__(kTile, 3) void k_rhs_tile(RhsArgs a, TileArgs t, int nbe, RhsArgs ra) {
   extern __shared__ double tile_lds[];
   const LdsRecs srec{tile_lds, t.s1cap};
   double *shead = tile_lds + 8 * t.s1cap;
@@ -1062,7 +1073,7 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   int *sbankj = reinterpret_cast<int *>(sbank + 2 * kTile);   // [kTile]
   const int nrb = (int)gridDim.x - nbe;
   if ((int)blockIdx.x < nrb) {
-    river_parts(a, (int)blockIdx.x, tile_lds);
+    river_parts(ra, (int)blockIdx.x, tile_lds);
     return;
   }
   const int tile = xcd_tile((int)blockIdx.x - nrb, nbe, a.tile_span);
@@ -1080,14 +1091,16 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   // through the staging)
   const bool own = p < ne;
   double ys = 0.0, yg = 0.0, zmax = 0.0, zmin = 0.0, depth = 0.0, dmac = 0.0;
-  double kmach = 0.0, areafv = 0.0, ksath = 0.0, rough = 0.0;
+  double kmac = 0.0, ksath = 0.0, rough = 0.0;
   int oc[3] = {0, 0, 0};
   double nx[3] = {0.0, 0.0, 0.0}, ny[3] = {0.0, 0.0, 0.0};
+  SoilIn so{0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
   if (own) {
-    zmax = e.zmax[p]; zmin = e.zmin[p]; depth = e.depth[p]; dmac = e.dmac[p];
+    so = load_soil_in(a, p, ix);
+    zmax = e.zmax[p]; zmin = e.zmin[p]; depth = so.depth; dmac = so.dmac;
     ys = y[p];
     yg = y[2 * ne + p];
-    kmach = e.kmach[p]; areafv = e.areafv[p]; ksath = e.ksath[p]; rough = e.rough[p];
+    kmac = e.kmac[p]; ksath = e.ksath[p]; rough = e.rough[p];
 #pragma unroll
     for (int j = 0; j < 3; j++) oc[j] = src.code(j);
     if (diff) {
@@ -1103,7 +1116,7 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   const bool hv = i < nh, h1 = i < n1;
   long hq = 0;
   double hys = 0.0, hyg = 0.0, hzmax = 0.0, hzmin = 0.0, hdepth = 0.0, hdmac = 0.0;
-  double hkmach = 0.0, hareafv = 0.0, hksath = 0.0, hrough = 0.0;
+  double hkmac = 0.0, hksath = 0.0, hrough = 0.0;
   int hc[3] = {0, 0, 0};
   double hnx[3] = {0.0, 0.0, 0.0}, hny[3] = {0.0, 0.0, 0.0};
   if (hv) {
@@ -1113,7 +1126,7 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
     if (h1) {
       hyg = y[2 * ne + hq];
       hzmin = e.zmin[hq]; hdepth = e.depth[hq]; hdmac = e.dmac[hq];
-      hkmach = e.kmach[hq]; hareafv = e.areafv[hq]; hksath = e.ksath[hq]; hrough = e.rough[hq];
+      hkmac = e.kmac[hq]; hksath = e.ksath[hq]; hrough = e.rough[hq];
       if (diff) {
 #pragma unroll
         for (int j = 0; j < 3; j++) {
@@ -1128,7 +1141,7 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   // records and heads; the bank fluxes of the element's first river edge,
   // whose gathers (segment, then the other bank) then overlap the halo's
   if (own) {
-    const NbrRec r = tile_rec(ys, yg, zmax, zmin, depth, dmac, kmach, areafv, ksath, rough);
+    const NbrRec r = tile_rec(ys, yg, zmax, zmin, depth, dmac, kmac, ksath, rough);
     srec.put(i, r);
     shead[i] = r.head;
     int bj = -1;
@@ -1143,7 +1156,7 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   }
   if (hv) {
     if (h1) {
-      const NbrRec r = tile_rec(hys, hyg, hzmax, hzmin, hdepth, hdmac, hkmach, hareafv, hksath, hrough);
+      const NbrRec r = tile_rec(hys, hyg, hzmax, hzmin, hdepth, hdmac, hkmac, hksath, hrough);
       srec.put(kTile + i, r);
       shead[kTile + i] = r.head;
     } else {
@@ -1153,8 +1166,8 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
   for (int h = i + kTile; h < nh; h += kTile) {
     const long q = t.hidx[hb + h];
     if (h < n1) {
-      const NbrRec r = tile_rec(y[q], y[2 * ne + q], e.zmax[q], e.zmin[q], e.depth[q], e.dmac[q], e.kmach[q],
-                                e.areafv[q], e.ksath[q], e.rough[q]);
+      const NbrRec r = tile_rec(y[q], y[2 * ne + q], e.zmax[q], e.zmin[q], e.depth[q], e.dmac[q], e.kmac[q],
+                                e.ksath[q], e.rough[q]);
       srec.put(kTile + h, r);
       shead[kTile + h] = r.head;
     } else {
@@ -1180,7 +1193,8 @@ __global__ __launch_bounds__(kTile, N ? 3 : 4) void k_rhs_tile(RhsArgs a, TileAr
     __syncthreads();
   }
   if (!own) return;
-  elem_core<false, N>(a, p, ix, src, load_elem_in<N>(a, p, ix, src));
+  const ElemIn in = load_elem_in<N>(a, p, ix, src, so);
+  elem_core<false, N>(a, p, ix, src, in, elem_soil(so, srec.get(i).gw));
 }
 
 // k_flux of a single solve, with the _NOAH_ branches when the context has them.
@@ -1196,9 +1210,9 @@ static void launch_single(const pihm_ctx *c, const RhsArgs &a) {
   if (c->rhs_path == PIHM_RHS_ONE_LAUNCH) {
     const int nt = div_up(c->ne, kTile), nrb = div_up(c->nr, kRivSeg);
     if (c->noah)
-      hipLaunchKernelGGL((k_rhs_tile<true>), dim3(nt + nrb), dim3(kTile), c->tile_lds, c->stream, a, c->tiles, nt);
+      hipLaunchKernelGGL((k_rhs_tile<true>), dim3(nt + nrb), dim3(kTile), c->tile_lds, c->stream, a, c->tiles, nt, a);
     else
-      hipLaunchKernelGGL((k_rhs_tile<false>), dim3(nt + nrb), dim3(kTile), c->tile_lds, c->stream, a, c->tiles, nt);
+      hipLaunchKernelGGL((k_rhs_tile<false>), dim3(nt + nrb), dim3(kTile), c->tile_lds, c->stream, a, c->tiles, nt, a);
     return;
   }
   hipLaunchKernelGGL(k_prep<false>, dim3(nbe + 3 * nbr), dim3(kBlock), 0, c->stream, a, nbe);
@@ -1396,7 +1410,7 @@ int ctx_alloc(const std::vector<SlotCap> &caps, int surf_mode, int riv_mode, pih
   RiverDev &R = A.r;
   Arena ar;
   double **ed[] = {&E.area, &E.zmin, &E.zmax, &E.depth, &E.ksath, &E.ksatv, &E.kinfv, &E.dinf,
-                   &E.alpha, &E.beta, &E.porosity, &E.dmac, &E.kmach, &E.kmacv, &E.areafv,
+                   &E.alpha, &E.beta, &E.porosity, &E.dmac, &E.kmac, &E.kmacv,
                    &E.areafh, &E.rough, &E.rzd, &E.pcpdrp, &E.edir, &E.ett, &E.ws0s};
   for (auto p : ed) ar.add(p, ne);
   double **ed3[] = {&E.edge, &E.nabrdist, &E.nabr_x, &E.nabr_y, &E.ebc};
@@ -1571,12 +1585,20 @@ int ctx_load(pihm_ctx *c, int k, const pihm_mesh_desc *m) {
   std::vector<double> hd(3L * cap.ne, 0.0);
   const double *es[] = {m->area, m->zmin, m->zmax, m->depth, m->ksath, m->ksatv, m->kinfv,
                         m->dinf, m->alpha, m->beta, m->porosity, m->dmac, m->kmach, m->kmacv,
-                        m->areafv, m->areafh, m->rough, m->rzd};
+                        m->areafh, m->rough, m->rzd};
   double *ed[] = {E.area, E.zmin, E.zmax, E.depth, E.ksath, E.ksatv, E.kinfv, E.dinf,
-                  E.alpha, E.beta, E.porosity, E.dmac, E.kmach, E.kmacv, E.areafv,
+                  E.alpha, E.beta, E.porosity, E.dmac, E.kmac, E.kmacv,
                   E.areafh, E.rough, E.rzd};
-  for (int f = 0; f < 18; f++) {
-    for (int lp = 0; lp < n; lp++) hd[lp] = es[f][order[lp]];
+  for (int f = 0; f < 17; f++) {
+    if (es[f] == m->kmach) {
+      // EffKh's conductivity with macropores (src/lat_flow.c:258), static
+      for (int lp = 0; lp < n; lp++) {
+        const int i = order[lp];
+        hd[lp] = m->kmach[i] * m->areafv[i] + m->ksath[i] * (1.0 - m->areafv[i]);
+      }
+    } else {
+      for (int lp = 0; lp < n; lp++) hd[lp] = es[f][order[lp]];
+    }
     PIHM_HIP_TRY(hipMemcpyAsync(ed[f] + off, hd.data(), n * sizeof(double), hipMemcpyHostToDevice, st));
     PIHM_HIP_TRY(hipStreamSynchronize(st));
   }
