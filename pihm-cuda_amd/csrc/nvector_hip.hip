@@ -33,6 +33,8 @@ constexpr int kMaxMulti = PIHM_RED_MAXSUMS;
 
 using RedWork = pihm_redwork;
 
+constexpr int kMaxPool = 32;   // a BDF/SPGMR integrator holds 6 + 5 + maxl + 5 clones (21 by default)
+
 // One workspace per device vector family (clones share the parent's).
 struct Aux {
   RedWork w;
@@ -90,46 +92,30 @@ __global__ void k_unary(long n, int op, double c, const double *x, const double 
 // reduction kinds
 enum RedKind { R_DOT = 0, R_WSQ, R_WSQMASK, R_MAXABS, R_MIN, R_ABSSUM, R_MINQ, R_INVTEST, R_CONSTR };
 
-__device__ __forceinline__ double red_identity(int kind) {
-  switch (kind) {
-    case R_MAXABS: return 0.0;
-    case R_MIN: case R_MINQ: return DBL_MAX;
-    default: return 0.0;
-  }
-}
-__device__ __forceinline__ double red_combine(int kind, double a, double b) {
-  switch (kind) {
-    case R_MAXABS: return fmax(a, b);
-    case R_MIN: case R_MINQ: return fmin(a, b);
-    case R_INVTEST: case R_CONSTR: return fmax(a, b);
-    default: return a + b;
-  }
+// how the partials of a reduction kind combine
+__host__ __device__ constexpr unsigned red_comb(int kind) {
+  return (kind == R_MAXABS || kind == R_INVTEST || kind == R_CONSTR) ? COMB_MAX
+         : (kind == R_MIN || kind == R_MINQ)                         ? COMB_MIN
+                                                                     : COMB_SUM;
 }
 
-__device__ __forceinline__ double wave_reduce(int kind, double v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v = red_combine(kind, v, __shfl_xor(v, off, 64));
-  return v;
-}
-
-// Block reduction in a fixed order: wavefront butterfly, then wave 0 over
-// the 4 wave sums.
-__device__ __forceinline__ double block_reduce(int kind, double v, double *lds) {
-  v = wave_reduce(kind, v);
+// Block reduction in a fixed order: wavefront butterfly, then the 4 wave
+// values in order (from the combination's identity).  Valid in thread 0.
+__device__ __forceinline__ double block_reduce(unsigned c, double v, double *lds) {
+  v = wave_comb(c, v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) lds[wave] = v;
   __syncthreads();
-  double r = red_identity(kind);
+  double r = comb_ident(c);
   if (threadIdx.x == 0) {
-    for (int w = 0; w < (int)(blockDim.x >> 6); w++) r = red_combine(kind, r, lds[w]);
+    for (int w = 0; w < kRedBlock / 64; w++) r = comb(c, r, lds[w]);
   }
   __syncthreads();
-  return r;  // valid in thread 0
+  return r;
 }
 
 struct RedArgs {
   long n;
-  int kind;
   int nvec;                    // number of simultaneous reductions (dot-multi)
   const double *x;
   const double *w;             // weights / second operand
@@ -140,54 +126,70 @@ struct RedArgs {
   RedWork work;
 };
 
-__device__ __forceinline__ double red_elem(const RedArgs &a, long i, int k) {
-  switch (a.kind) {
-    case R_DOT: return a.x[i] * a.ys[k][i];
-    case R_WSQ: { double p = a.x[i] * a.w[i]; return p * p; }
-    case R_WSQMASK: { if (a.id[i] > 0.0) { double p = a.x[i] * a.w[i]; return p * p; } return 0.0; }
-    case R_MAXABS: return fabs(a.x[i]);
-    case R_MIN: return a.x[i];
-    case R_ABSSUM: return fabs(a.x[i]);
-    case R_MINQ: { double d = a.w[i]; return (d == 0.0) ? DBL_MAX : a.x[i] / d; }
-    case R_INVTEST: {
-      double xv = a.x[i];
-      if (xv == 0.0) return 1.0;
-      a.z[i] = 1.0 / xv;
-      return 0.0;
-    }
-    case R_CONSTR: {
-      const double c = a.id[i], xv = a.x[i];
-      double bad = 0.0;
-      if (c != 0.0) {
-        if (c > 1.5 || c < -1.5) { if (xv * c <= 0.0) bad = 1.0; }
-        else if (c > 0.5 || c < -0.5) { if (xv * c < 0.0) bad = 1.0; }
-      }
-      a.m[i] = bad;
-      return bad;
-    }
+// Entry i of a reduction in two parts: its loads, then its value (and, for the
+// two tests, its store).
+struct RedIn { double x, o; };
+template <int KIND>
+__device__ __forceinline__ RedIn red_load(const RedArgs &a, const double *y, long i) {
+  RedIn in{a.x[i], 0.0};
+  if constexpr (KIND == R_DOT) in.o = y[i];
+  if constexpr (KIND == R_WSQ || KIND == R_MINQ) in.o = a.w[i];
+  if constexpr (KIND == R_WSQMASK) in.o = (a.id[i] > 0.0) ? a.w[i] : 0.0;
+  if constexpr (KIND == R_CONSTR) in.o = a.id[i];
+  return in;
+}
+template <int KIND>
+__device__ __forceinline__ double red_elem(const RedArgs &a, const RedIn &in, long i) {
+  const double xv = in.x;
+  if constexpr (KIND == R_DOT) return xv * in.o;
+  if constexpr (KIND == R_WSQ) { const double p = xv * in.o; return p * p; }
+  if constexpr (KIND == R_WSQMASK) {
+    if (a.id[i] > 0.0) { const double p = xv * in.o; return p * p; }
+    return 0.0;
   }
-  return 0.0;
+  if constexpr (KIND == R_MAXABS || KIND == R_ABSSUM) return fabs(xv);
+  if constexpr (KIND == R_MIN) return xv;
+  if constexpr (KIND == R_MINQ) return (in.o == 0.0) ? DBL_MAX : xv / in.o;
+  if constexpr (KIND == R_INVTEST) {
+    if (xv == 0.0) return 1.0;
+    a.z[i] = 1.0 / xv;
+    return 0.0;
+  }
+  if constexpr (KIND == R_CONSTR) {
+    const double c = in.o;
+    double bad = 0.0;
+    if (c != 0.0) {
+      if (c > 1.5 || c < -1.5) { if (xv * c <= 0.0) bad = 1.0; }
+      else if (c > 0.5 || c < -0.5) { if (xv * c < 0.0) bad = 1.0; }
+    }
+    a.m[i] = bad;
+    return bad;
+  }
 }
 
+// First pass (and the second, as k_fused_sum): two entries' loads before
+// either is combined, in the order of the entries.
+template <int KIND>
 __global__ __launch_bounds__(kRedBlock) void k_reduce(RedArgs a) {
   __shared__ double lds[4];
+  constexpr unsigned c = red_comb(KIND);
   const long stride = (long)gridDim.x * blockDim.x;
+  const bool ends = a.nvec == 1 && a.work.ticket && (int)gridDim.x <= kTicketBlocks;
   for (int k = 0; k < a.nvec; k++) {
-    double v = red_identity(a.kind);
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < a.n; i += stride)
-      v = red_combine(a.kind, v, red_elem(a, i, k));
-    const double r = block_reduce(a.kind, v, lds);
-    if (threadIdx.x == 0) a.work.partials[(long)k * kMaxRedBlocks + blockIdx.x] = r;
+    const double *y = a.ys[k];
+    double v = comb_ident(c);
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (; i + stride < a.n; i += 2 * stride) {
+      const RedIn p = red_load<KIND>(a, y, i), q = red_load<KIND>(a, y, i + stride);
+      v = comb(c, v, red_elem<KIND>(a, p, i));
+      v = comb(c, v, red_elem<KIND>(a, q, i + stride));
+    }
+    if (i < a.n) v = comb(c, v, red_elem<KIND>(a, red_load<KIND>(a, y, i), i));
+    const double r = block_reduce(c, v, lds);
+    if (threadIdx.x == 0) store_partial(&a.work.partials[(long)k * kMaxRedBlocks + blockIdx.x], r, ends);
   }
-}
-
-// how the second pass combines the partials of a reduction kind
-unsigned red_comb(int kind) {
-  switch (kind) {
-    case R_MAXABS: case R_INVTEST: case R_CONSTR: return COMB_MAX;
-    case R_MIN: case R_MINQ: return COMB_MIN;
-    default: return COMB_SUM;
-  }
+  if (ends && last_workgroup(a.work.ticket, gridDim.x))
+    second_pass<1, c, true>(gridDim.x, a.work.partials, a.work.result, nullptr, a.work.ctr, a.work.flag, nullptr, 0.0);
 }
 
 // fused ops ------------------------------------------------------------------
@@ -258,6 +260,7 @@ __global__ void k_correct(long n, int q, ZnPtrs z, const double *acor, double l0
   }
 }
 
+constexpr unsigned kEwtCombs = COMB_MIN | (COMB_SUM << 2);
 __global__ __launch_bounds__(kRedBlock) void k_ewt(long n, const double *y, double rtol, double atol,
                                                   double *ewt, RedWork work) {
   __shared__ double lds[4];
@@ -279,12 +282,15 @@ __global__ __launch_bounds__(kRedBlock) void k_ewt(long n, const double *y, doub
     one(i + stride, y1);
   }
   if (i < n) one(i, y[i]);
-  const double r0 = block_reduce(R_MIN, mn, lds);
-  const double r1 = block_reduce(R_DOT, sq, lds);
+  const double r0 = block_reduce(COMB_MIN, mn, lds);
+  const double r1 = block_reduce(COMB_SUM, sq, lds);
+  const bool ends = (int)gridDim.x <= kTicketBlocks;
   if (threadIdx.x == 0) {
-    work.partials[blockIdx.x] = r0;
-    work.partials[kMaxRedBlocks + blockIdx.x] = r1;
+    store_partial(&work.partials[blockIdx.x], r0, ends);
+    store_partial(&work.partials[kMaxRedBlocks + blockIdx.x], r1, ends);
   }
+  if (ends && last_workgroup(work.ticket, gridDim.x))
+    second_pass<2, kEwtCombs, true>(gridDim.x, work.partials, work.result, nullptr, work.ctr, work.flag, nullptr, 0.0);
 }
 
 __global__ void k_newton_rhs(long n, double rl1, const double *zn1, const double *acor, double gamma,
@@ -317,8 +323,10 @@ int aux_new(Aux **out) {
   if (!x) return -1;
   HostBlock *hb = nullptr;
   if (hipMalloc(&x->w.partials, sizeof(double) * kMaxRedBlocks * kMaxMulti) != hipSuccess) return -1;
-  if (hipMalloc(&x->w.ctr, sizeof(unsigned)) != hipSuccess) return -1;
-  if (hipMemset(x->w.ctr, 0, sizeof(unsigned)) != hipSuccess) return -1;
+  // the count of second passes and, a cache line away, the ticket
+  if (hipMalloc(&x->w.ctr, 256) != hipSuccess) return -1;
+  if (hipMemset(x->w.ctr, 0, 256) != hipSuccess) return -1;
+  x->w.ticket = x->w.ctr + 32;
   if (hipHostMalloc((void **)&hb, sizeof(HostBlock), hipHostMallocCoherent) != hipSuccess) return -1;
   std::memset(hb, 0, sizeof(HostBlock));
   x->w.result = hb->result;
@@ -337,16 +345,35 @@ void aux_release(Aux *x) {
   std::free(x);
 }
 
-bool reduce(N_Vector v, RedArgs &a, double *out, int nout) {
-  a.work = X(v)->w;
-  const int nb = red_blocks(a.n);
-  hipLaunchKernelGGL(k_reduce, dim3(nb), dim3(kRedBlock), 0, S(v), a);
-  unsigned combs = 0;
-  for (int k = 0; k < a.nvec; k++) combs |= red_comb(a.kind) << (2 * k);
-  launch_final(nb, a.nvec, combs, a.work, S(v), nullptr);
+template <int KIND>
+void launch_reduce(const RedArgs &a, int nb, hipStream_t st) {
+  hipLaunchKernelGGL(k_reduce<KIND>, dim3(nb), dim3(kRedBlock), 0, st, a);
+  if (a.nvec == 1) launch_final<1, red_comb(KIND)>(nb, a.work, st, nullptr);
+}
+
+// Second pass of nvec dot products at once.
+template <int NV>
+void launch_multi_final(int nvec, int nb, RedWork w, hipStream_t st) {
+  if constexpr (NV <= kMaxMulti) {
+    if (nvec == NV) {
+      hipLaunchKernelGGL((k_partials_final<NV, 0u>), dim3(1), dim3(kRedThreads), 0, st, nb, w.partials, w.result,
+                         (double *)nullptr, w.ctr, w.flag, (double *)nullptr, 0.0);
+    } else {
+      launch_multi_final<NV + 1>(nvec, nb, w, st);
+    }
+  }
+}
+
+bool reduce_wait(N_Vector v, const RedArgs &a, double *out) {
   if (pihm_red_wait(a.work, S(v))) return false;
-  for (int k = 0; k < nout; k++) out[k] = a.work.result[k];
+  for (int k = 0; k < a.nvec; k++) out[k] = a.work.result[k];
   return true;
+}
+template <int KIND>
+bool reduce(N_Vector v, RedArgs &a, double *out) {
+  a.work = X(v)->w;
+  launch_reduce<KIND>(a, red_blocks(a.n), S(v));
+  return reduce_wait(v, a, out);
 }
 
 void launch_unary(N_Vector x, int op, double c, N_Vector y, N_Vector z) {
@@ -486,83 +513,82 @@ void N_VInv_Hip(N_Vector x, N_Vector z) { launch_unary(x, 4, 0.0, nullptr, z); }
 void N_VAddConst_Hip(N_Vector x, double b, N_Vector z) { launch_unary(x, 5, b, nullptr, z); }
 void N_VCompare_Hip(double c, N_Vector x, N_Vector z) { launch_unary(x, 6, c, nullptr, z); }
 
-static RedArgs red_init(N_Vector x, int kind) {
+static RedArgs red_init(N_Vector x) {
   RedArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = L(x);
-  a.kind = kind;
   a.nvec = 1;
   a.x = D(x);
   return a;
 }
 
 double N_VDotProd_Hip(N_Vector x, N_Vector y) {
-  RedArgs a = red_init(x, R_DOT);
+  RedArgs a = red_init(x);
   a.ys[0] = D(y);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_DOT>(x, a, &r);
   return r;
 }
 double N_VMaxNorm_Hip(N_Vector x) {
-  RedArgs a = red_init(x, R_MAXABS);
+  RedArgs a = red_init(x);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_MAXABS>(x, a, &r);
   return r;
 }
 double N_VWrmsNorm_Hip(N_Vector x, N_Vector w) {
-  RedArgs a = red_init(x, R_WSQ);
+  RedArgs a = red_init(x);
   a.w = D(w);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_WSQ>(x, a, &r);
   return std::sqrt(r / (double)L(x));
 }
 double N_VWrmsNormMask_Hip(N_Vector x, N_Vector w, N_Vector id) {
-  RedArgs a = red_init(x, R_WSQMASK);
+  RedArgs a = red_init(x);
   a.w = D(w);
   a.id = D(id);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_WSQMASK>(x, a, &r);
   return std::sqrt(r / (double)L(x));
 }
 double N_VMin_Hip(N_Vector x) {
-  RedArgs a = red_init(x, R_MIN);
+  RedArgs a = red_init(x);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_MIN>(x, a, &r);
   return r;
 }
 double N_VWL2Norm_Hip(N_Vector x, N_Vector w) {
-  RedArgs a = red_init(x, R_WSQ);
+  RedArgs a = red_init(x);
   a.w = D(w);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_WSQ>(x, a, &r);
   return std::sqrt(r);
 }
 double N_VL1Norm_Hip(N_Vector x) {
-  RedArgs a = red_init(x, R_ABSSUM);
+  RedArgs a = red_init(x);
   double r = NAN;
-  reduce(x, a, &r, 1);
+  reduce<R_ABSSUM>(x, a, &r);
   return r;
 }
 booleantype N_VInvTest_Hip(N_Vector x, N_Vector z) {
-  RedArgs a = red_init(x, R_INVTEST);
+  RedArgs a = red_init(x);
   a.z = D(z);
   double r = 1.0;
-  reduce(x, a, &r, 1);
+  reduce<R_INVTEST>(x, a, &r);
   return r == 0.0;
 }
 booleantype N_VConstrMask_Hip(N_Vector c, N_Vector x, N_Vector m) {
-  RedArgs a = red_init(x, R_CONSTR);
+  RedArgs a = red_init(x);
   a.id = D(c);
   a.m = D(m);
   double r = 1.0;
-  reduce(x, a, &r, 1);
+  reduce<R_CONSTR>(x, a, &r);
   return r == 0.0;
 }
 double N_VMinQuotient_Hip(N_Vector num, N_Vector denom) {
-  RedArgs a = red_init(num, R_MINQ);
+  RedArgs a = red_init(num);
   a.w = D(denom);
   double r = DBL_MAX;
-  reduce(num, a, &r, 1);
+  reduce<R_MINQ>(num, a, &r);
   return r;
 }
 
@@ -577,10 +603,15 @@ int N_VLinearCombination_Hip(int nvec, const double *c, N_Vector *Xv, N_Vector z
 
 int N_VDotProdMulti_Hip(int nvec, N_Vector x, N_Vector *Y, double *d) {
   if (nvec < 1 || nvec > kMaxMulti) return -1;
-  RedArgs a = red_init(x, R_DOT);
+  RedArgs a = red_init(x);
   a.nvec = nvec;
   for (int k = 0; k < nvec; k++) a.ys[k] = D(Y[k]);
-  return reduce(x, a, d, nvec) ? 0 : -2;
+  if (nvec == 1) return reduce<R_DOT>(x, a, d) ? 0 : -2;
+  a.work = X(x)->w;
+  const int nb = red_blocks(a.n);
+  launch_reduce<R_DOT>(a, nb, S(x));
+  launch_multi_final<2>(nvec, nb, a.work, S(x));
+  return reduce_wait(x, a, d) ? 0 : -2;
 }
 
 double N_VLinearSumWrms_Hip(double a, N_Vector x, double b, N_Vector y, N_Vector z, N_Vector w) {
@@ -627,7 +658,7 @@ int pihm_nv_ewt_ss(N_Vector y, double rtol, double atol, N_Vector ewt, double *m
   RedWork w = X(y)->w;
   const int nb = red_blocks(n);
   hipLaunchKernelGGL(k_ewt, dim3(nb), dim3(kRedBlock), 0, S(y), n, D(y), rtol, atol, D(ewt), w);
-  launch_final(nb, 2, COMB_MIN | (COMB_SUM << 2), w, S(y), nullptr);
+  launch_final<2, kEwtCombs>(nb, w, S(y), nullptr);
   if (pihm_red_wait(w, S(y))) return -2;
   *mn = w.result[0];
   *ynrm = std::sqrt(w.result[1] / (double)n);
@@ -686,19 +717,17 @@ int pihm_nv_dotprod_noalloc(long int n, const double *x_dev, const double *y_dev
   RedArgs a;
   std::memset(&a, 0, sizeof(a));
   a.n = n;
-  a.kind = R_DOT;
   a.nvec = 1;
   a.x = x_dev;
   a.ys[0] = y_dev;
-  a.work.partials = ws;
+  a.work.partials = ws;   // no ticket: always two launches
   const int nb = red_blocks(n);
-  hipLaunchKernelGGL(k_reduce, dim3(nb), dim3(kRedBlock), 0, st, a);
+  hipLaunchKernelGGL(k_reduce<R_DOT>, dim3(nb), dim3(kRedBlock), 0, st, a);
   // second pass: the same tree as N_VDotProd_Hip's; its counters live in the
   // last slot of the array, the result goes to the caller's device memory
   unsigned *ctr = reinterpret_cast<unsigned *>(ws + PIHM_RED_MAXBLOCKS);
-  hipLaunchKernelGGL(k_partials_final, dim3(1), dim3(kRedThreads), 0, st, nb, 1, (unsigned)COMB_SUM,
-                     (const double *)ws, result_dev, (double *)nullptr, ctr, (volatile unsigned *)(ctr + 1),
-                     (double *)nullptr, 0.0);
+  hipLaunchKernelGGL((k_partials_final<1, 0u>), dim3(1), dim3(kRedThreads), 0, st, nb, (const double *)ws, result_dev,
+                     (double *)nullptr, ctr, (volatile unsigned *)(ctr + 1), (double *)nullptr, 0.0);
   return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 

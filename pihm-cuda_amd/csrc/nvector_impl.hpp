@@ -16,8 +16,11 @@ typedef struct pihm_redwork {
   unsigned *ctr;             // device: second passes completed
   volatile unsigned *flag;   // pinned host (coherent): copy of *ctr
   unsigned *expect;          // host: second passes launched and awaited
+  unsigned *ticket;          // device: workgroups of the running first pass that are done
+                             // (nullptr: the second pass is always a launch of its own)
 } pihm_redwork;
 #define PIHM_RED_MAXBLOCKS 1024
+#define PIHM_RED_TICKETS 64    // workgroups up to which the last one does the second pass
 #define PIHM_RED_MAXSUMS 16
 pihm_redwork pihm_nv_redwork(N_Vector v);
 void *pihm_nv_stream(N_Vector v);
