@@ -217,6 +217,10 @@ struct pihm_ctx {
   pihm::TileArgs tiles;
   size_t tile_lds;               // dynamic LDS bytes per element block
   void *tile_arena;
+  // State vector of model runs on this context and, through its family's pool,
+  // the integrator's vectors (22 vectors, 8 neq bytes each): kept from the
+  // first run to the next and freed with the context.
+  N_Vector run_vec;
 };
 
 // Caller-order index of device element p / device river r (the loaded slots

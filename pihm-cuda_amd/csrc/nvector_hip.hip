@@ -39,6 +39,12 @@ constexpr int kMaxPool = 32;   // a BDF/SPGMR integrator holds 6 + 5 + maxl + 5 
 struct Aux {
   RedWork w;
   int refs;
+  // Buffers of destroyed clones, kept for later clones when the family was
+  // made by pihm_nv_new_pooled; freed with the family's last vector.
+  int pooled;
+  long pool_len;      // entries per buffer
+  int npool;
+  double *pool[kMaxPool];
 };
 
 inline N_VectorContent_Hip C(N_Vector v) { return (N_VectorContent_Hip)v->content; }
@@ -339,6 +345,7 @@ int aux_new(Aux **out) {
 void aux_release(Aux *x) {
   if (!x) return;
   if (--x->refs > 0) return;
+  for (int k = 0; k < x->npool; k++) (void)hipFree(x->pool[k]);
   (void)hipFree(x->w.partials);
   (void)hipFree(x->w.ctr);
   (void)hipHostFree(x->w.result);   // first member of the host block
@@ -444,6 +451,15 @@ N_Vector N_VNew_Hip(long int length) {
   return v;
 }
 
+N_Vector pihm_nv_new_pooled(long int length) {
+  N_Vector v = N_VNew_Hip(length);
+  if (v) {
+    X(v)->pooled = 1;
+    X(v)->pool_len = length;
+  }
+  return v;
+}
+
 N_Vector N_VMake_Hip(long int length, double *device_data) {
   N_Vector v = N_VNewEmpty_Hip(length);
   if (v) C(v)->data = device_data;
@@ -452,7 +468,11 @@ N_Vector N_VMake_Hip(long int length, double *device_data) {
 
 void N_VDestroy_Hip(N_Vector v) {
   if (!v) return;
-  if (C(v)->own_data && C(v)->data) (void)hipFree(C(v)->data);
+  if (C(v)->own_data && C(v)->data) {
+    Aux *x = X(v);
+    if (x->pooled && L(v) == x->pool_len && x->refs > 1 && x->npool < kMaxPool) x->pool[x->npool++] = C(v)->data;
+    else (void)hipFree(C(v)->data);
+  }
   aux_release(X(v));
   std::free(v->content);
   std::free(v);
@@ -466,6 +486,12 @@ N_Vector N_VCloneEmpty_Hip(N_Vector w) {
 N_Vector N_VClone_Hip(N_Vector w) {
   N_Vector v = N_VCloneEmpty_Hip(w);
   double *d = nullptr;
+  Aux *x = X(w);
+  if (x->pooled && L(w) == x->pool_len && x->npool > 0) {
+    C(v)->data = x->pool[--x->npool];
+    C(v)->own_data = 1;
+    return v;
+  }
   if (hipMalloc(&d, sizeof(double) * std::max<long>(L(w), 1)) != hipSuccess) {
     N_VDestroy_Hip(v);
     return nullptr;

@@ -24,6 +24,11 @@ typedef struct pihm_redwork {
 #define PIHM_RED_MAXSUMS 16
 pihm_redwork pihm_nv_redwork(N_Vector v);
 void *pihm_nv_stream(N_Vector v);
+// N_VNew_Hip whose family keeps the buffers of destroyed clones (at most 32)
+// for later clones and frees them with its last vector.  A buffer may be
+// reused at once, on any stream: the caller waits for the family's queued work
+// between destroying clones and making new ones.
+N_Vector pihm_nv_new_pooled(long int length);
 // Wait until the most recently launched second pass of w has written its
 // results (spins on the pinned flag; falls back to synchronising the stream).
 int pihm_red_wait(pihm_redwork w, void *stream);

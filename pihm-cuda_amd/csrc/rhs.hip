@@ -1397,6 +1397,7 @@ int ctx_alloc(const std::vector<SlotCap> &caps, int surf_mode, int riv_mode, pih
   c->tiles = TileArgs{};
   c->tile_lds = 0;
   c->tile_arena = nullptr;
+  c->run_vec = nullptr;
   PIHM_HIP_TRY(hipGetDevice(&c->device));
   c->perm.assign(ne, -1);
   c->iperm.assign(ne, -1);
@@ -1829,6 +1830,7 @@ extern "C" int pihm_ctx_load_member(pihm_ctx *c, int k, const pihm_mesh_desc *m)
 
 extern "C" void pihm_ctx_destroy(pihm_ctx *c) {
   if (!c) return;
+  if (c->run_vec) N_VDestroy_Hip(c->run_vec);
   if (c->arena) (void)hipFree(c->arena);
   if (c->noah_arena) (void)hipFree(c->noah_arena);
   if (c->tile_arena) (void)hipFree(c->tile_arena);
