@@ -60,6 +60,10 @@ struct Mem {
   long rp_n = 0;
   int att_it[PIHM_REC_ITERS] = {};   // Newton and Krylov counts of the step attempt in progress
   bool fused = false;
+  // fused: the rescaling that the next predict applies (factors of zn[1..q])
+  bool scale_pending = false;
+  int scale_q = 0;
+  double scale_f[6] = {};
   // Krylov iterations replayed from graphs (device vectors on a non-null
   // stream and an RHS declared capturable, PihmCVodeSetGraphRhs)
   bool graph_rhs = false, graph_off = false;
@@ -186,11 +190,25 @@ int ewt_set(Mem *m, N_Vector ycur, double *ynrm) {
 }
 
 // ---------------------------------------------------------------- Nordsieck
+// Applies a rescaling that no prediction has taken up (an error return, or
+// anything else that reads zn first).
+void flush_scale(Mem *m) {
+  if (!m->scale_pending) return;
+  m->scale_pending = false;
+  for (int j = 1; j <= m->scale_q; j++) VScale(m->scale_f[j], m->zn[j], m->zn[j]);
+}
+
 void rescale(Mem *m) {   // cvode.c:2251-2275
   double f[6] = {1, 1, 1, 1, 1, 1};
   double factor = m->eta;
   for (int j = 1; j <= m->q; j++) { f[j] = factor; factor *= m->eta; }
-  if (m->fused) pihm_nv_rescale(m->q, f, m->zn);
+  if (m->fused) {
+    // the prediction that follows applies it
+    flush_scale(m);
+    m->scale_pending = true;
+    m->scale_q = m->q;
+    for (int j = 0; j < 6; j++) m->scale_f[j] = f[j];
+  }
   else for (int j = 1; j <= m->q; j++) VScale(f[j], m->zn[j], m->zn[j]);
   m->h = m->hscale * m->eta;
   m->next_h = m->h;
@@ -201,13 +219,23 @@ void rescale(Mem *m) {   // cvode.c:2251-2275
 void predict(Mem *m) {   // cvode.c:2277-2306
   m->tn += m->h;
   if (m->tstopset && (m->tn - m->tstop) * m->h > 0.0) m->tn = m->tstop;
-  if (m->fused) { pihm_nv_predict(m->q, m->zn); return; }
+  if (m->fused) {
+    // without a preconditioner setup, which borrows them, y and acor start the
+    // Newton iteration in the same launch
+    const bool start = !setup_nonnull(m);
+    if (m->scale_q != m->q) flush_scale(m);
+    pihm_nv_predict(m->q, m->zn, m->scale_pending ? m->scale_f : nullptr, start ? m->y : nullptr,
+                    start ? m->acor : nullptr);
+    m->scale_pending = false;
+    return;
+  }
   for (int k = 1; k <= m->q; k++)
     for (int j = m->q; j >= k; j--) VLin(1.0, m->zn[j - 1], 1.0, m->zn[j], m->zn[j - 1]);
 }
 
 void restore(Mem *m, double saved_t) {   // cvode.c:2882-2913
   m->tn = saved_t;
+  flush_scale(m);
   if (m->fused) { pihm_nv_restore(m->q, m->zn); return; }
   for (int k = 1; k <= m->q; k++)
     for (int j = m->q; j >= k; j--) VLin(1.0, m->zn[j - 1], -1.0, m->zn[j], m->zn[j - 1]);
@@ -250,6 +278,7 @@ void decrease_bdf(Mem *m) {   // cvode.c:2225-2249
 
 void adjust_order(Mem *m, int deltaq) {   // cvode.c:2099-2118, 2165-2187
   if (m->q == 2 && deltaq != 1) return;
+  flush_scale(m);
   if (deltaq == 1) increase_bdf(m);
   else if (deltaq == -1) decrease_bdf(m);
 }
@@ -669,8 +698,10 @@ int nls_newton(Mem *m, int nflag) {   // cvode.c:2651-2727
       if (ier < 0) return PIHM_CV_LSETUP_FAIL;
       if (ier > 0) return CONV_FAIL;
     }
-    VConst(0.0, m->acor);
-    VScale(1.0, m->zn[0], m->y);
+    if (!m->fused || setup_nonnull(m)) {   // otherwise predict has done it
+      VConst(0.0, m->acor);
+      VScale(1.0, m->zn[0], m->y);
+    }
     const int ier = m->fused ? newton_iteration_fused(m) : newton_iteration(m);
     if (ier != TRY_AGAIN) return ier;
     call_setup = true;
@@ -788,6 +819,32 @@ double compute_etaqp1(Mem *m) {   // cvode.c:3110-3135
   return m->etaqp1;
 }
 
+// The two estimates above with both norms from one launch.
+void order_etas_fused(Mem *m) {
+  m->etaqm1 = m->etaqp1 = 0.0;
+  const bool lower = m->q > 1, higher = m->q != m->qmax && m->saved_tq5 != 0.0;
+  if (!lower && !higher) return;
+  double cquot = 0.0, sq = 0.0, sp = 0.0;
+  if (higher) {
+    double pw = 1.0;
+    const double r = m->h / m->tau[2];
+    for (int i = 0; i < m->L; i++) pw *= r;
+    cquot = (m->tq[5] / m->saved_tq5) * pw;
+  }
+  if (pihm_nv_order_sums(lower ? m->zn[m->q] : nullptr, -cquot, higher ? m->zn[m->qmax] : nullptr, m->acor, m->ewt,
+                         &sq, &sp))
+    sq = sp = NAN;
+  const double N = (double)m->neq;
+  if (lower) {
+    const double ddn = std::sqrt(sq / N) * m->tq[1];
+    m->etaqm1 = 1.0 / (std::pow(BIAS1 * ddn, 1.0 / m->q) + ADDON);
+  }
+  if (higher) {
+    const double dup = std::sqrt(sp / N) * m->tq[3];
+    m->etaqp1 = 1.0 / (std::pow(BIAS3 * dup, 1.0 / (m->L + 1)) + ADDON);
+  }
+}
+
 void choose_eta(Mem *m) {   // cvode.c:3137-3184
   const double etam = std::fmax(m->etaqm1, std::fmax(m->etaq, m->etaqp1));
   if (etam < THRESH) {
@@ -824,8 +881,12 @@ void prepare_next_step(Mem *m, double dsm) {   // cvode.c:3029-3066
     return;
   }
   m->qwait = 2;
-  m->etaqm1 = compute_etaqm1(m);
-  m->etaqp1 = compute_etaqp1(m);
+  if (m->fused) {
+    order_etas_fused(m);
+  } else {
+    m->etaqm1 = compute_etaqm1(m);
+    m->etaqp1 = compute_etaqp1(m);
+  }
   choose_eta(m);
   set_eta(m);
 }
@@ -870,7 +931,9 @@ int step(Mem *m) {   // cvode.c:2005-2066
     m->eta = m->hprime / m->h;
   }
   m->etamax = (m->nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
-  VScale(m->tq[2], m->acor, m->acor);
+  // CVODE leaves the local error estimate tq[2]*acor in acor for its getter; this
+  // integrator has no such getter, and the next step starts acor at zero
+  if (!m->fused) VScale(m->tq[2], m->acor, m->acor);
   return PIHM_CV_SUCCESS;
 }
 
@@ -882,6 +945,11 @@ int get_dky(Mem *m, double t, int k, N_Vector dky) {   // cvode.c:1509-1569
   const double tn1 = m->tn + tfuzz;
   if ((t - tp) * (t - tn1) > 0.0) return PIHM_CV_BAD_T;
   const double s = (t - m->tn) / m->h;
+  flush_scale(m);
+  if (m->fused && k == 0) {
+    pihm_nv_dky(m->q, s, m->zn, dky);
+    return PIHM_CV_SUCCESS;
+  }
   for (int j = m->q; j >= k; j--) {
     double c = 1.0;
     for (int i = j; i >= j - k + 1; i--) c *= i;
@@ -921,6 +989,7 @@ int PihmCVodeInit(void *mem, PihmRhsFn f, realtype t0, N_Vector y0) {   // cvode
   m->q = 1; m->L = 2; m->qwait = m->L; m->etamax = ETAMX1;
   m->qu = 0; m->hu = 0.0; m->tolsf = 1.0;
   VScale(1.0, y0, m->zn[0]);
+  m->scale_pending = false;
   m->nst = m->nfe = m->ncfn = m->netf = m->nni = m->nli = m->nfes = m->nhnil = m->nscon = 0;
   m->nstlp = m->nstlpre = m->npe = m->nps = m->nsetups = 0;
   m->jcur = false;
@@ -942,6 +1011,7 @@ int PihmCVodeReInit(void *mem, realtype t0, N_Vector y0) {   // cvode.c:580-675
   m->q = 1; m->L = 2; m->qwait = m->L; m->etamax = ETAMX1;
   m->qu = 0; m->hu = 0.0; m->tolsf = 1.0;
   VScale(1.0, y0, m->zn[0]);
+  m->scale_pending = false;
   m->nst = m->nfe = m->ncfn = m->netf = m->nni = m->nli = m->nfes = m->nhnil = m->nscon = 0;
   m->nstlp = m->nstlpre = m->npe = m->nps = m->nsetups = 0;
   m->jcur = false;

@@ -188,6 +188,32 @@ struct FFinish {
   __device__ __forceinline__ void operator()(long i, double (&acc)[2]) const { apply(i, load(i), acc); }
 };
 
+// The two norms of the order selection, from N_VLinearSum and N_VWrmsNorm's
+// expressions (the linear sum is not stored: nothing else reads it).
+struct FOrder {
+  const double *znq, *znm, *acor, *ewt;
+  double a;
+  struct In { double q, m, ac, w; };
+  __device__ __forceinline__ In load(long i) const {
+    In in{0.0, 0.0, 0.0, ewt[i]};
+    if (znq) in.q = znq[i];
+    if (znm) { in.m = znm[i]; in.ac = acor[i]; }
+    return in;
+  }
+  __device__ __forceinline__ void apply(long, const In &in, double (&acc)[2]) const {
+    if (znq) { const double p = in.q * in.w; acc[0] += p * p; }
+    if (znm) {
+      double t;
+      if (a == 1.0) t = a * (in.m + in.ac);
+      else if (a == -1.0) t = a * (in.m - in.ac);
+      else t = (a * in.m) + (1.0 * in.ac);
+      const double p = t * in.w;
+      acc[1] += p * p;
+    }
+  }
+  __device__ __forceinline__ void operator()(long i, double (&acc)[2]) const { apply(i, load(i), acc); }
+};
+
 // xcor = sum_j y_j V_j (LinearSum(y_j, V_j, 1, xcor, xcor) from xcor = 0), then
 // Div(xcor, s2): the operand of the right preconditioner's final solve.
 struct CombineArgs {
@@ -318,6 +344,16 @@ int pihm_gm_finish(int mode, int k, const double *ycoef, N_Vector *V, N_Vector s
   for (int j = 0; j < k; j++) { f.yc[j] = ycoef[j]; f.vk[j] = D(V[j]); }
   f.s = D(s); f.b = D(b); f.zn0 = D(zn0); f.acor = D(acor); f.y = D(y); f.xsrc = xsrc;
   return fused_sum<2>(L(s), f, pihm_nv_redwork(s), S(s), sums);
+}
+
+int pihm_nv_order_sums(N_Vector znq, double a, N_Vector znmax, N_Vector acor, N_Vector ewt, double *sumq,
+                       double *sump) {
+  FOrder f{znq ? D(znq) : nullptr, znmax ? D(znmax) : nullptr, D(acor), D(ewt), a};
+  double sums[2];
+  const int rc = fused_sum<2>(L(ewt), f, pihm_nv_redwork(ewt), S(ewt), sums);
+  *sumq = sums[0];
+  *sump = sums[1];
+  return rc;
 }
 
 int pihm_gm_combine(int k, const double *ycoef, N_Vector *V, N_Vector s, N_Vector out) {

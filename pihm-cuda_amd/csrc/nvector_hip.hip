@@ -201,13 +201,24 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce(RedArgs a) {
 // fused ops ------------------------------------------------------------------
 struct ZnPtrs { double *p[7]; };
 
+// A step's start in one launch: the pending rescaling zn[j] *= f[j] (when
+// scale), the Pascal update, and with y and acor the Newton iteration's start
+// y = zn[0], acor = 0.  sign < 0: the inverse update alone.  One launch instead
+// of four, each 1 to 2 passes over the vectors (20 us of a step at 200,000
+// triangles; 9 us of launches on small meshes).
+struct Factors { double f[6]; };
 template <int Q>
-__global__ void k_predict(long n, ZnPtrs z, int sign) {
+__global__ void k_predict(long n, ZnPtrs z, int sign, bool scale, Factors fs, double *y, double *acor) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   double v[Q + 1];
 #pragma unroll
   for (int j = 0; j <= Q; j++) v[j] = z.p[j][i];
+  if (scale) {
+#pragma unroll
+    for (int j = 1; j <= Q; j++) v[j] = fs.f[j] * v[j];
+    z.p[Q][i] = v[Q];
+  }
 #pragma unroll
   for (int k = 1; k <= Q; k++)
 #pragma unroll
@@ -217,31 +228,44 @@ __global__ void k_predict(long n, ZnPtrs z, int sign) {
     }
 #pragma unroll
   for (int j = 0; j < Q; j++) z.p[j][i] = v[j];
-}
-
-void launch_predict(long n, int q, ZnPtrs z, int sign, hipStream_t st) {
-  const dim3 g(ew_blocks(n)), b(kBlock);
-  switch (q) {
-    case 1: hipLaunchKernelGGL(k_predict<1>, g, b, 0, st, n, z, sign); break;
-    case 2: hipLaunchKernelGGL(k_predict<2>, g, b, 0, st, n, z, sign); break;
-    case 3: hipLaunchKernelGGL(k_predict<3>, g, b, 0, st, n, z, sign); break;
-    case 4: hipLaunchKernelGGL(k_predict<4>, g, b, 0, st, n, z, sign); break;
-    default: hipLaunchKernelGGL(k_predict<5>, g, b, 0, st, n, z, sign); break;
+  if (y) {
+    y[i] = v[0];
+    acor[i] = 0.0;
   }
 }
 
-__global__ void k_rescale(long n, int q, ZnPtrs z, double f1, double f2, double f3, double f4, double f5) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+void launch_predict(long n, int q, ZnPtrs z, int sign, const double *f, double *y, double *acor, hipStream_t st) {
+  const dim3 g(ew_blocks(n)), b(kBlock);
+  Factors fs{};
+  for (int j = 0; f && j <= q && j < 6; j++) fs.f[j] = f[j];
+  const bool sc = f != nullptr;
+  switch (q) {
+    case 1: hipLaunchKernelGGL(k_predict<1>, g, b, 0, st, n, z, sign, sc, fs, y, acor); break;
+    case 2: hipLaunchKernelGGL(k_predict<2>, g, b, 0, st, n, z, sign, sc, fs, y, acor); break;
+    case 3: hipLaunchKernelGGL(k_predict<3>, g, b, 0, st, n, z, sign, sc, fs, y, acor); break;
+    case 4: hipLaunchKernelGGL(k_predict<4>, g, b, 0, st, n, z, sign, sc, fs, y, acor); break;
+    default: hipLaunchKernelGGL(k_predict<5>, g, b, 0, st, n, z, sign, sc, fs, y, acor); break;
+  }
+}
+
+// zn interpolated at a time: out = zn[q]; out = LinearSum(1, zn[j], s, out) for
+// j = q-1 .. 0, one launch instead of q + 1.
+__global__ void k_dky(long n, int q, ZnPtrs z, double s, double *out) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const double f[6] = {1.0, f1, f2, f3, f4, f5};
-  // every entry loaded before any is stored (a store would keep the next
-  // array's load behind it)
   double v[6];
 #pragma unroll
-  for (int j = 1; j < 6; j++) v[j] = (j <= q) ? z.p[j][i] : 0.0;
+  for (int j = 0; j < 6; j++) v[j] = (j <= q) ? z.p[j][i] : 0.0;
+  double r = 0.0;
 #pragma unroll
-  for (int j = 1; j < 6; j++)
-    if (j <= q) z.p[j][i] = f[j] * v[j];
+  for (int j = 5; j >= 0; j--) {
+    if (j > q) continue;
+    if (j == q) r = v[j];
+    else if (s == 1.0) r = v[j] + r;
+    else if (s == -1.0) r = v[j] - r;
+    else r = v[j] + (s * r);
+  }
+  out[i] = r;
 }
 
 __global__ void k_correct(long n, int q, ZnPtrs z, const double *acor, double l0, double l1, double l2,
@@ -645,28 +669,25 @@ double N_VLinearSumWrms_Hip(double a, N_Vector x, double b, N_Vector y, N_Vector
   return N_VWrmsNorm_Hip(z, w);
 }
 
-int pihm_nv_predict(int q, N_Vector *zn) {
+int pihm_nv_predict(int q, N_Vector *zn, const double *factors, N_Vector y, N_Vector acor) {
   ZnPtrs z;
   for (int j = 0; j <= q; j++) z.p[j] = D(zn[j]);
   const long n = L(zn[0]);
-  launch_predict(n, q, z, 1, S(zn[0]));
+  launch_predict(n, q, z, 1, factors, y ? D(y) : nullptr, acor ? D(acor) : nullptr, S(zn[0]));
   return 0;
 }
 int pihm_nv_restore(int q, N_Vector *zn) {
   ZnPtrs z;
   for (int j = 0; j <= q; j++) z.p[j] = D(zn[j]);
   const long n = L(zn[0]);
-  launch_predict(n, q, z, -1, S(zn[0]));
+  launch_predict(n, q, z, -1, nullptr, nullptr, nullptr, S(zn[0]));
   return 0;
 }
-int pihm_nv_rescale(int q, const double *f, N_Vector *zn) {
+int pihm_nv_dky(int q, double s, N_Vector *zn, N_Vector out) {
   ZnPtrs z;
   for (int j = 0; j <= q; j++) z.p[j] = D(zn[j]);
   const long n = L(zn[0]);
-  double ff[6] = {1, 1, 1, 1, 1, 1};
-  for (int j = 1; j <= q && j <= 5; j++) ff[j] = f[j];
-  hipLaunchKernelGGL(k_rescale, dim3(ew_blocks(n)), dim3(kBlock), 0, S(zn[0]), n, q, z, ff[1], ff[2],
-                     ff[3], ff[4], ff[5]);
+  hipLaunchKernelGGL(k_dky, dim3(ew_blocks(n)), dim3(kBlock), 0, S(zn[0]), n, q, z, s, D(out));
   return 0;
 }
 int pihm_nv_correct(int q, const double *l, N_Vector acor, N_Vector *zn) {

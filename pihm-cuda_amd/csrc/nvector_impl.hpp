@@ -76,14 +76,21 @@ int pihm_gm_combine(int k, const double *ycoef, N_Vector *V, N_Vector s, N_Vecto
 
 // Fused Nordsieck-array updates used by the integrator (one launch each).
 // zn holds q+1 (or more) device vectors of equal length.
-//   predict:  for k=1..q, j=q..k: zn[j-1] += zn[j]        (cvode.c:2277-2306)
+//   predict:  zn[j] *= factors[j], j=1..q (cvode.c:2251-2275), when factors is
+//             not NULL; for k=1..q, j=q..k: zn[j-1] += zn[j] (cvode.c:2277-2306);
+//             y = zn[0], acor = 0 when y is not NULL (cvode.c:2710-2712)
 //   restore:  for k=1..q, j=q..k: zn[j-1] -= zn[j]        (cvode.c:2882-2913)
-//   rescale:  zn[j] *= eta^j, j=1..q                      (cvode.c:2251-2275)
 //   correct:  zn[j] += l[j]*acor, j=0..q                  (cvode.c:3010-3011)
-int pihm_nv_predict(int q, N_Vector *zn);
+//   dky:      out = zn[q], then out = zn[j] + s*out, j=q-1..0 (cvode.c:1550-1560)
+int pihm_nv_predict(int q, N_Vector *zn, const double *factors, N_Vector y, N_Vector acor);
 int pihm_nv_restore(int q, N_Vector *zn);
-int pihm_nv_rescale(int q, const double *factors, N_Vector *zn);
 int pihm_nv_correct(int q, const double *l, N_Vector acor, N_Vector *zn);
+int pihm_nv_dky(int q, double s, N_Vector *zn, N_Vector out);
+// Order selection (cvode.c:3091-3135), one launch and one wait: *sumq = sum
+// (znq*ewt)^2 when znq is not NULL, *sump = sum (LinearSum(a, znmax, 1, acor) *
+// ewt)^2 when znmax is not NULL.
+int pihm_nv_order_sums(N_Vector znq, double a, N_Vector znmax, N_Vector acor, N_Vector ewt, double *sumq,
+                       double *sump);
 // ewt = 1/(rtol*|y| + atol); returns min(rtol*|y|+atol) in *mn and
 // WRMS(y, ewt) in *ynrm (cvode.c:4081-4098 and :1377-1378) in one pass.
 int pihm_nv_ewt_ss(N_Vector y, double rtol, double atol, N_Vector ewt, double *mn, double *ynrm);
