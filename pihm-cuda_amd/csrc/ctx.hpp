@@ -146,6 +146,11 @@ struct RhsArgs {
 }  // namespace pihm
 
 namespace pihm {
+// What pihm_ctx_poll_nan's kernel hands to the host.
+struct NanReport {
+  int flag;
+  volatile unsigned count;
+};
 // Capacity of one slot of a context: the largest mesh it can hold.
 struct SlotCap {
   int ne, nr;
@@ -207,8 +212,9 @@ struct pihm_ctx {
   pihm::RhsArgs args;            // pointers filled at creation
   void *arena;                   // one device allocation for everything
   size_t arena_bytes;
-  int *nanflag_dev;
-  int *nanflag_host;             // pinned
+  int *nanflag_dev;              // the flag, then the count of its reports
+  pihm::NanReport *nan_host;     // pinned (coherent)
+  unsigned nan_expect;           // reports awaited so far
   double *stage_host;            // scratch for host-side permutations
   int noah;                      // RHS with the reference's _NOAH_ branches
   void *noah_arena;              // the Noah fields of ElemDev
