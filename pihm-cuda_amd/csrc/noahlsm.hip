@@ -69,10 +69,12 @@ struct ColDev {
   double *pcpdrp, *edir, *ett, *et, *sh2o0;    // context step inputs and Noah hand-over
 };
 
-// One element's working record: the reference's ps/ws/wf/es/ef fields the step touches.
+// One element's working record: the reference's ps/ws/wf/es/ef fields the step
+// touches.  The layer arrays are the kernel's own locals: an array inside the
+// record, indexed at run time, would keep the whole record in scratch memory.
 struct Col {
   int nsoil, nroot;
-  double zsoil[ML], rtdis[ML], smc[ML], sh2o[ML], stc[ML], et[ML];
+  double *zsoil, *rtdis, *smc, *sh2o, *stc, *et;   // [ML]
   // parameters
   double shdfac, cmcfactr, laimin, laimax, emissmin, emissmax, albedomin, albedomax, z0min, z0max, snup, cfactr;
   double rgl, rsmin, rsmax, topt, hs, smcmax, smcmin, smcref, smcwlt, smcdry, quartz, alpha, beta, zlvl_wind;
@@ -88,7 +90,7 @@ struct Col {
 };
 
 // CalHum: src/noah/noah.c:659-702
-__device__ void cal_hum(Col &c, const NoahUni &u) {
+__device__ __forceinline__ void cal_hum(Col &c, const NoahUni &u) {
   const double A2 = 17.67, A3 = 273.15, A4 = 29.65, ELWV = 2.501e6, E0 = 611.0, RVV = 461.0, EPSILON = 0.622;
   const double SVP1 = 611.2, SVP2 = 17.67, SVP3 = 29.65, SVPT0 = 273.15;
   const double rh = c.rh / 100.0;
@@ -103,14 +105,14 @@ __device__ void cal_hum(Col &c, const NoahUni &u) {
 }
 
 // CSnow: src/noah/noah.c:811-839
-__device__ double c_snow(double dsnow) {
+__device__ __forceinline__ double c_snow(double dsnow) {
   const double UNIT = 0.11631;
   const double cc = 0.328 * pow(10.0, 2.25 * dsnow);
   return 2.0 * UNIT * cc;
 }
 
 // SnowNew: src/noah/noah.c:2222-2268
-__device__ void snow_new(Col &c, double newsn) {
+__device__ __forceinline__ void snow_new(Col &c, double newsn) {
   double snowhc = c.snowh * 100.0;
   const double newsnc = newsn * 100.0;
   const double tempc = c.sfctmp - 273.15;
@@ -123,7 +125,7 @@ __device__ void snow_new(Col &c, double newsn) {
 }
 
 // SnFrac: src/noah/noah.c:1713-1744
-__device__ double sn_frac(double sneqv, double snup, double salp) {
+__device__ __forceinline__ double sn_frac(double sneqv, double snup, double salp) {
   if (sneqv < snup) {
     const double rsnow = sneqv / snup;
     return 1.0 - (exp(-salp * rsnow) - rsnow * exp(-salp));
@@ -132,7 +134,7 @@ __device__ double sn_frac(double sneqv, double snup, double salp) {
 }
 
 // AlCalc: src/noah/noah.c:610-657
-__device__ void al_calc(Col &c, const NoahUni &u, double dt, int snowng) {
+__device__ __forceinline__ void al_calc(Col &c, const NoahUni &u, double dt, int snowng) {
   const double SNACCA = 0.94, SNACCB = 0.58;
   const double snoalb = u.snoalb;
   c.albedo = c.alb + c.sncovr * (snoalb - c.alb);
@@ -151,7 +153,7 @@ __device__ void al_calc(Col &c, const NoahUni &u, double dt, int snowng) {
 }
 
 // TDfCnd: src/noah/noah.c:2520-2619
-__device__ double tdf_cnd(double smc, double qz, double smcmax, double smcmin, double sh2o) {
+__device__ __forceinline__ double tdf_cnd(double smc, double qz, double smcmax, double smcmin, double sh2o) {
   const double THKICE = 2.2, THKQTZ = 7.7, THKW = 0.57;
   const double satratio = (smc - smcmin) / (smcmax - smcmin);
   const double thko = 2.0;
@@ -169,7 +171,7 @@ __device__ double tdf_cnd(double smc, double qz, double smcmax, double smcmin, d
 }
 
 // Snowz0: src/noah/noah.c:2202-2220
-__device__ double snow_z0(double sncovr, double z0brd, double snowh) {
+__device__ __forceinline__ double snow_z0(double sncovr, double z0brd, double snowh) {
   const double Z0S = 0.001;
   const double burial = 7.0 * z0brd - snowh;
   const double z0eff = (burial <= 0.0007) ? Z0S : (burial / 7.0);
@@ -177,14 +179,14 @@ __device__ double snow_z0(double sncovr, double z0brd, double snowh) {
 }
 
 // Paulson's stability functions: src/noah/noah.c:3204-3222
-__device__ double psp_mu(double xx) {
+__device__ __forceinline__ double psp_mu(double xx) {
   return -2.0 * log((xx + 1.0) * 0.5) - log((xx * xx + 1.0) * 0.5) + 2.0 * atan(xx) - NPI * 0.5;
 }
-__device__ double psp_hu(double xx) { return -2.0 * log((xx * xx + 1.0) * 0.5); }
+__device__ __forceinline__ double psp_hu(double xx) { return -2.0 * log((xx * xx + 1.0) * 0.5); }
 
 // SfcDifOff: src/noah/noah.c:2862-3079 with iz0tlnd = 0 and Paulson's
 // functions (ilech = 0; the Lech branches are never taken)
-__device__ void sfc_dif_off(double zlvl, double zlvl_wind, double z0, double czil, double sfcspd, double t1v,
+__device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, double z0, double czil, double sfcspd, double t1v,
                             double th2v, double &cm, double &ch) {
   const double WWST = 1.2, VKRM = 0.40, EXCM = 0.001, BETA = 1.0 / 270.0;
   const double WOLD = 0.15;
@@ -256,7 +258,7 @@ __device__ void sfc_dif_off(double zlvl, double zlvl_wind, double z0, double czi
 }
 
 // Penman: src/noah/noah.c:1508-1570
-__device__ void penman(Col &c, double &t24, double t2v, int snowng, int frzgra) {
+__device__ __forceinline__ void penman(Col &c, double &t24, double t2v, int snowng, int frzgra) {
   const double ELCP = 2.4888e+3, LSUBC = 2.501000e+6;
   const double emissi = c.emissi;
   const double elcp1 = (1.0 - c.sncovr) * ELCP + c.sncovr * ELCP * LSUBS / LSUBC;
@@ -284,7 +286,7 @@ __device__ void penman(Col &c, double &t24, double t2v, int snowng, int frzgra) 
 }
 
 // CanRes: src/noah/noah.c:704-809
-__device__ void can_res(Col &c) {
+__device__ __forceinline__ void can_res(Col &c) {
   const double SLV = 2.501000e6;
   c.rc = 0.0;
   const double ff = 0.55 * 2.0 * c.soldn / (c.rgl * c.proj_lai);
@@ -315,7 +317,7 @@ __device__ void can_res(Col &c) {
 }
 
 // DEvap: src/noah/noah.c:841-870
-__device__ void d_evap(Col &c, const NoahUni &u) {
+__device__ __forceinline__ void d_evap(Col &c, const NoahUni &u) {
   const double sratio = (c.sh2o[0] - c.smcdry) / (c.smcmax - c.smcdry);
   double fx = 0.0;
   if (sratio > 0.0) {
@@ -327,7 +329,7 @@ __device__ void d_evap(Col &c, const NoahUni &u) {
 }
 
 // Transp: src/noah/noah.c:2725-2811
-__device__ void transp(Col &c) {
+__device__ __forceinline__ void transp(Col &c) {
   for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
   double etpa;
   if (c.cmc != 0.0) etpa = c.shdfac * c.pc * c.etp * (1.0 - pow(c.cmc / c.cmcmax, c.cfactr));
@@ -352,7 +354,7 @@ __device__ void transp(Col &c) {
 }
 
 // Evapo: src/noah/noah.c:872-959
-__device__ void evapo(Col &c, const NoahUni &u, double dt) {
+__device__ __forceinline__ void evapo(Col &c, const NoahUni &u, double dt) {
   c.edir = 0.0;
   c.ec = 0.0;
   c.ett = 0.0;
@@ -374,7 +376,7 @@ __device__ void evapo(Col &c, const NoahUni &u, double dt) {
 }
 
 // PcpDrp: src/noah/noah.c:1451-1506
-__device__ void pcp_drp(Col &c, double prcp, double dt) {
+__device__ __forceinline__ void pcp_drp(Col &c, double prcp, double dt) {
   const double KD = 6.54e-7, BFACTR = 3.89;
   double rhsct = c.shdfac * prcp - c.ec;
   c.drip = 0.0;
@@ -393,14 +395,14 @@ __device__ void pcp_drp(Col &c, double prcp, double dt) {
 }
 
 // TBnd: src/noah/noah.c:2482-2518
-__device__ double t_bnd(double tu, double tb, const double *zsoil, double zbot, int k, int nsoil) {
+__device__ __forceinline__ double t_bnd(double tu, double tb, const double *zsoil, double zbot, int k, int nsoil) {
   const double zup = (k == 0) ? 0.0 : zsoil[k - 1];
   const double zb = (k == nsoil - 1) ? 2.0 * zbot - zsoil[k] : zsoil[k + 1];
   return tu + (tb - tu) * (zup - zsoil[k]) / (zup - zb);
 }
 
 // TmpAvg: src/noah/noah.c:2621-2723
-__device__ double tmp_avg(double tup, double tm, double tdn, const double *zsoil, int k) {
+__device__ __forceinline__ double tmp_avg(double tup, double tm, double tdn, const double *zsoil, int k) {
   const double dz = (k == 0) ? -zsoil[0] : zsoil[k - 1] - zsoil[k];
   const double dzh = dz * 0.5;
   double tavg;
@@ -445,7 +447,7 @@ __device__ double tmp_avg(double tup, double tm, double tdn, const double *zsoil
 }
 
 // FrH2O: src/noah/noah.c:978-1090 (van Genuchten form)
-__device__ double fr_h2o(double tkelv, double smc, double sh2o, double smcmax, double smcmin, double alpha,
+__device__ __forceinline__ double fr_h2o(double tkelv, double smc, double sh2o, double smcmax, double smcmin, double alpha,
                          double beta) {
   const double CK = 8.0, ERROR = 0.005;
   if (tkelv > (TFREEZ - 1.0e-3)) return smc;
@@ -480,7 +482,7 @@ __device__ double fr_h2o(double tkelv, double smc, double sh2o, double smcmax, d
 }
 
 // SnkSrc: src/noah/noah.c:1746-1811 (updates sh2o[k])
-__device__ double snk_src(Col &c, double tavg, int k, double dt, double qtot) {
+__device__ __forceinline__ double snk_src(Col &c, double tavg, int k, double dt, double qtot) {
   const double DH2O = 1.0000e3;
   const double dz = (k == 0) ? -c.zsoil[0] : c.zsoil[k - 1] - c.zsoil[k];
   const double sh2o = c.sh2o[k], smc = c.smc[k];
@@ -497,7 +499,7 @@ __device__ double snk_src(Col &c, double tavg, int k, double dt, double qtot) {
 
 // ShFlx: src/noah/noah.c:1621-1652 with HRT (:1092-1299, itavg on), HStep
 // (:1301-1340) and Rosr12 (:1572-1620) inline
-__device__ void sh_flx(Col &c, const NoahUni &u, double dt, double yy, double zz1, double df1) {
+__device__ __forceinline__ void sh_flx(Col &c, const NoahUni &u, double dt, double yy, double zz1, double df1) {
   const double CH2O = 4.2e6;
   const int nsoil = c.nsoil;
   const double csoil_loc = u.csoil;
@@ -558,28 +560,23 @@ __device__ void sh_flx(Col &c, const NoahUni &u, double dt, double yy, double zz
     dtsdz = dtsdz2;
     ddz = ddz2;
   }
-  // HStep
-  double rin[ML], cin[ML];
-  for (int k = 0; k < nsoil; k++) {
-    rhsts[k] *= dt;
-    ai[k] *= dt;
-    bi[k] = 1.0 + bi[k] * dt;
-    ci[k] *= dt;
-  }
-  for (int k = 0; k < nsoil; k++) rin[k] = rhsts[k];
-  for (int k = 0; k < nsoil; k++) cin[k] = ci[k];
-  // Rosr12 (p = ci, a = ai, b = bi, c = cin, d = rin, delta = rhsts)
+  // HStep and Rosr12 in place, layer by layer: ci becomes p, rhsts becomes
+  // delta; each entry is read before it is overwritten, so the arithmetic is
+  // the reference's, which works on copies
   {
-    double *p = ci, *delta = rhsts;
-    cin[nsoil - 1] = 0.0;
-    p[0] = -cin[0] / bi[0];
-    delta[0] = rin[0] / bi[0];
+    double bk = 1.0 + bi[0] * dt, ck = (nsoil == 1) ? 0.0 : ci[0] * dt;
+    ci[0] = -ck / bk;
+    rhsts[0] = (rhsts[0] * dt) / bk;
     for (int k = 1; k < nsoil; k++) {
-      p[k] = -cin[k] * (1.0 / (bi[k] + ai[k] * p[k - 1]));
-      delta[k] = (rin[k] - ai[k] * delta[k - 1]) * (1.0 / (bi[k] + ai[k] * p[k - 1]));
+      const double ak = ai[k] * dt;
+      bk = 1.0 + bi[k] * dt;
+      ck = (k == nsoil - 1) ? 0.0 : ci[k] * dt;
+      const double inv = 1.0 / (bk + ak * ci[k - 1]);
+      ci[k] = -ck * inv;
+      rhsts[k] = (rhsts[k] * dt - ak * rhsts[k - 1]) * inv;
     }
-    p[nsoil - 1] = delta[nsoil - 1];
-    for (int k = nsoil - 2; k >= 0; k--) p[k] = p[k] * p[k + 1] + delta[k];
+    ci[nsoil - 1] = rhsts[nsoil - 1];
+    for (int k = nsoil - 2; k >= 0; k--) ci[k] = ci[k] * ci[k + 1] + rhsts[k];
   }
   for (int k = 0; k < nsoil; k++) c.stc[k] += ci[k];
   c.t1 = (yy + (zz1 - 1.0) * c.stc[0]) / zz1;
@@ -587,7 +584,7 @@ __device__ void sh_flx(Col &c, const NoahUni &u, double dt, double yy, double zz
 }
 
 // NoPac: src/noah/noah.c:1343-1449
-__device__ void no_pac(Col &c, const NoahUni &u, double dt, double t24) {
+__device__ __forceinline__ void no_pac(Col &c, const NoahUni &u, double dt, double t24) {
   double prcpf = c.prcp;
   c.dew = 0.0;
   c.edir = 0.0;
@@ -620,7 +617,7 @@ __device__ void no_pac(Col &c, const NoahUni &u, double dt, double t24) {
 }
 
 // SnowPack: src/noah/noah.c:2100-2200
-__device__ void snow_pack(double esd, double dtsec, double &snowh, double &sndens, double tsnow, double tsoil) {
+__device__ __forceinline__ void snow_pack(double esd, double dtsec, double &snowh, double &sndens, double tsnow, double tsoil) {
   const double C1 = 0.01, C2 = 21.0;
   const double esdc = esd * 100.0;
   const double dthr = dtsec / 3600.0;
@@ -646,7 +643,7 @@ __device__ void snow_pack(double esd, double dtsec, double &snowh, double &snden
 }
 
 // SnoPac: src/noah/noah.c:1813-2098
-__device__ void sno_pac(Col &c, const NoahUni &u, int snowng, double dt, double t24, double prcpf, double df1) {
+__device__ __forceinline__ void sno_pac(Col &c, const NoahUni &u, int snowng, double dt, double t24, double prcpf, double df1) {
   const double ESDMIN = 1.0e-6, SNOEXP = 2.0;
   c.dew = 0.0;
   c.edir = 0.0;
@@ -747,7 +744,7 @@ __device__ void sno_pac(Col &c, const NoahUni &u, int snowng, double dt, double 
 }
 
 // SFlx: src/noah/noah.c:166-609
-__device__ void s_flx(Col &c, const NoahUni &u, double dt) {
+__device__ __forceinline__ void s_flx(Col &c, const NoahUni &u, double dt) {
   const double shdfac = c.shdfac;
   double t24 = 0.0;
   c.snomlt = 0.0;
@@ -860,11 +857,26 @@ __global__ __launch_bounds__(kBlock) void k_noah_meteo(int nstation, int nrec, c
 }
 
 // Noah(): src/noah/noah.c:3-55, one element per thread.
-__global__ __launch_bounds__(kBlock) void k_noah(int ne, int nstation, NoahDev d, NoahUni u, ColDev s, double dt) {
-  const int p = blockIdx.x * kBlock + threadIdx.x;
+//
+// What bounds it: one column's chain of dependent FP64 work (the whole step is
+// one wavefront's latency up to some 20,000 columns), and at 100,000 columns
+// the chain times the few wavefronts a SIMD holds.  So the functions are
+// inlined, which lets the column's record live in registers (256, two
+// wavefronts per SIMD) with only the layer arrays and the largest branches'
+// overflow in scratch memory, and a workgroup is one wavefront, which spreads
+// 20,000 columns over every CU.  Measured (us per step, 6,000 / 20,011 /
+// 100,000 columns): 122 / 139 / 233 with calls and the record in scratch;
+// inlined 74.9 / 85.3 / 181.8 at one wavefront per SIMD, 80.9 / 101.1 / 170.8
+// at two, 94.8 / 124.7 / 208.1 at three; two and the heat solve in place
+// 77.9 / 92.8 / 147.7.
+constexpr int kNoahBlock = 64;
+__global__ __launch_bounds__(kNoahBlock, 2) void k_noah(int ne, int nstation, NoahDev d, NoahUni u, ColDev s, double dt) {
+  const int p = blockIdx.x * kNoahBlock + threadIdx.x;
   if (p >= ne) return;
   auto at = [ne, p](double *f, int k) -> double & { return f[(long)k * ne + p]; };
+  double zsoil[ML], rtdis[ML], smc[ML], sh2o[ML], stc[ML], et[ML];
   Col c;
+  c.zsoil = zsoil; c.rtdis = rtdis; c.smc = smc; c.sh2o = sh2o; c.stc = stc; c.et = et;
   c.nsoil = s.nsoil[p];
   c.nroot = d.nroot[p];
   for (int k = 0; k < ML; k++) {
@@ -1142,7 +1154,7 @@ int pihm_noah_lsm_step(pihm_noah_lsm *n, double t, double dt) {
   hipStream_t st = n->ctx->stream;
   hipLaunchKernelGGL(k_noah_meteo, dim3(div_up(n->nstation, kBlock)), dim3(kBlock), 0, st, n->nstation, n->nrec,
                      n->ftime, n->data, t, n->d.met);
-  hipLaunchKernelGGL(k_noah, dim3(div_up(n->ne, kBlock)), dim3(kBlock), 0, st, n->ne, n->nstation, n->d, n->u, n->s,
+  hipLaunchKernelGGL(k_noah, dim3(div_up(n->ne, kNoahBlock)), dim3(kNoahBlock), 0, st, n->ne, n->nstation, n->d, n->u, n->s,
                      dt);
   PIHM_HIP_TRY(hipGetLastError());
   return pihm_ctx_noah_refresh(n->ctx);
