@@ -120,46 +120,82 @@ __device__ __forceinline__ void wdf_cnd(double *wdf, double *wcnd, double smc, c
   }
 }
 
-// Every loop over the layers runs over the fixed 11 with a test for the
-// column's own nsoil, so each array index is a constant after unrolling and
-// the column stays in registers.  The water table, the lateral split and the
-// layer fluxes go straight to their HBM fields, which the thread reads back
-// where the reference reads them again.
-__global__ __launch_bounds__(kBlock) void k_noah_soil(int ne, SoilDev s, ElemDev e, const double *y, double dt) {
-  const int p = blockIdx.x * kBlock + threadIdx.x;
-  if (p >= ne) return;
+// Block shape of the soil-water step: 64 columns (one per lane) and four
+// wavefronts.  The layers' conductivities and diffusivities, two logarithms
+// and two exponentials each, depend on nothing but the layer and are dealt to
+// the wavefronts; the water table and the lateral split go to the last one,
+// which has the fewest layers; the recurrences down and up the column then run
+// in the first, from LDS, while other blocks' wavefronts fill the SIMD.
+//
+// What bounds it: the chain of one column, some 11 layers of dependent FP64
+// divisions, and 932 B per column of memory.  Measured (us per step, 6,000 /
+// 20,011 / 100,000 columns of 11 layers): 42.4 / 46.8 / 104.6 with one thread
+// per column, the column in registers (316 VGPRs, one wavefront per SIMD) and
+// five powers per layer; 32.5 / 37.0 / 85.2 with the powers shared; this form 17.8 / 22.6 / 52.0.
+constexpr int kSoilCols = 64, kSoilWaves = 4;
+
+__global__ __launch_bounds__(kSoilCols * kSoilWaves, 4) void k_noah_soil(int ne, SoilDev s, ElemDev e,
+                                                                         const double *y, double dt) {
+  __shared__ double lsh[ML][kSoilCols];    // liquid water after the clamps
+  __shared__ double lic[ML][kSoilCols];    // ice
+  __shared__ double lz[ML][kSoilCols];     // layer bottoms below the surface (negative)
+  __shared__ double lsat[ML][kSoilCols];   // saturated depth per layer
+  __shared__ double la[ML][kSoilCols];     // diffusivity; then Rosr12's p; then the moisture
+  __shared__ double lb[ML][kSoilCols];     // conductivity; then Rosr12's delta
+  __shared__ double lmax[kSoilWaves][kSoilCols];
+  __shared__ int ltbl[kSoilCols];
+  const int lane = (int)threadIdx.x % kSoilCols, wave = (int)threadIdx.x / kSoilCols;
+  const int q = blockIdx.x * kSoilCols + lane;
+  const bool own = q < ne;
+  const int p = own ? q : ne - 1;          // lanes past the end repeat the last column and store nothing
   const int nsoil = s.nsoil[p];
   const double smcmax = s.smcmax[p], smcmin = e.smcmin[p];
-  const double ksatv = e.ksatv[p], alpha = e.alpha[p], beta = e.beta[p];
-  const double gw = y[2L * ne + p];
   auto at = [ne, p](double *f, int k) -> double & { return f[(long)k * ne + p]; };
-  double zsoil[ML], smc[ML], sh2o[ML], sice[ML], ai[ML], bi[ML], ci[ML], rhstt[ML];
-  // layer depths below the surface (src/noah/lsm_func.c:150-160)
-#pragma unroll
-  for (int k = 0; k < ML; k++) {
-    zsoil[k] = 0.0;
-    if (k < nsoil) zsoil[k] = (k == 0) ? -at(s.sldpth, 0) : -at(s.sldpth, k) + zsoil[k - 1];
-    smc[k] = at(s.smc, k);
-    sh2o[k] = at(s.sh2o, k);
-  }
-  double fcr = e.fcr[p];
+  auto put = [&](double *f, int k, double v) {
+    if (own) f[(long)k * ne + p] = v;
+  };
 
-  // FindWaterTable (src/noah/lsm_func.c:4-55); Summary and NoahHydrol call it
-  // with the same arguments (src/update.c:40, src/noah/noah.c:72), so once
-  int nwtbl = -999;
-  {
-    double depth = 0.0;
+  // NoahHydrol's clamps (src/noah/noah.c:74-83) and the ice of each layer
+  // (SmFlx: src/noah/noah.c:1676-1679)
+  double icemax = 0.0;
+  for (int k = wave; k < nsoil; k += kSoilWaves) {
+    double smc = at(s.smc, k), sh2o = at(s.sh2o, k);
+    smc = (smc > smcmin + SH2OMIN) ? smc : smcmin + SH2OMIN;
+    smc = (smc < smcmax) ? smc : smcmax;
+    sh2o = (sh2o < smc) ? sh2o : smc;
+    const double sice = smc - sh2o;
+    lsh[k][lane] = sh2o;
+    lic[k][lane] = sice;
+    icemax = (sice > icemax) ? sice : icemax;
+  }
+  lmax[wave][lane] = icemax;
+  if (wave == kSoilWaves - 1) {
+    // layer depths (src/noah/lsm_func.c:150-160), FindWaterTable (:4-55;
+    // Summary and NoahHydrol call it with the same arguments, src/update.c:40,
+    // src/noah/noah.c:72, so once) and CalcLatFlx (:226-255; runoff2 is
+    // MassBalance's subsurface runoff)
+    const double gw = y[2L * ne + p];
+    double sl[ML], z = 0.0, depth = 0.0;
 #pragma unroll
-    for (int k = 0; k < ML; k++)
-      if (k < nsoil) depth += at(s.sldpth, k);
+    for (int k = 0; k < ML; k++) sl[k] = at(s.sldpth, k);
+#pragma unroll
+    for (int k = 0; k < ML; k++) {
+      if (k < nsoil) {
+        z = (k == 0) ? -sl[0] : -sl[k] + z;
+        lz[k][lane] = z;
+        depth += sl[k];
+      }
+    }
+    int nwtbl = -999;
+    double sat[ML];
     if (gw <= 0.0) {
       nwtbl = nsoil;
 #pragma unroll
-      for (int k = 0; k < ML; k++) at(s.satdpth, k) = (k == nsoil - 1) ? 1.0E-3 : 0.0;
+      for (int k = 0; k < ML; k++) sat[k] = (k == nsoil - 1) ? 1.0E-3 : 0.0;
     } else if (gw > depth) {
       nwtbl = 0;
 #pragma unroll
-      for (int k = 0; k < ML; k++) at(s.satdpth, k) = (k < nsoil) ? at(s.sldpth, k) : 0.0;
+      for (int k = 0; k < ML; k++) sat[k] = (k < nsoil) ? sl[k] : 0.0;
     } else {
       double dsum = 0.0;
       bool found = false;
@@ -167,67 +203,81 @@ __global__ __launch_bounds__(kBlock) void k_noah_soil(int ne, SoilDev s, ElemDev
       for (int k = ML - 1; k >= 0; k--) {
         double v = 0.0;
         if (k < nsoil && !found) {
-          const double sl = at(s.sldpth, k);
-          if (dsum + sl > gw) {
+          if (dsum + sl[k] > gw) {
             v = gw - dsum;
             nwtbl = k + 1;
             found = true;
           } else {
-            v = sl;
-            dsum += sl;
+            v = sl[k];
+            dsum += sl[k];
           }
         }
-        at(s.satdpth, k) = v;
+        sat[k] = v;
       }
     }
-  }
-  // CalcLatFlx: src/noah/lsm_func.c:226-255 (runoff2 is MassBalance's subsurface runoff)
-  {
     double sattot = 0.0;
 #pragma unroll
-    for (int k = 0; k < ML; k++)
-      if (k < nsoil) sattot += at(s.satdpth, k);
+    for (int k = 0; k < ML; k++) {
+      lsat[k][lane] = sat[k];
+      put(s.satdpth, k, sat[k]);
+      if (k < nsoil) sattot += sat[k];
+    }
     const double runoff2 = s.runoff2[p];
 #pragma unroll
     for (int k = 0; k < ML; k++) {
       if (sattot <= 0.0) {
-        if (k == nsoil - 1) at(s.runoff2_lyr, k) = runoff2;
+        if (k == nsoil - 1) put(s.runoff2_lyr, k, runoff2);
       } else if (k < nsoil) {
-        at(s.runoff2_lyr, k) = at(s.satdpth, k) / sattot * runoff2;
+        put(s.runoff2_lyr, k, sat[k] / sattot * runoff2);
       }
     }
+    ltbl[lane] = nwtbl;
   }
-  // NoahHydrol's clamps: src/noah/noah.c:74-83
-#pragma unroll
-  for (int k = 0; k < ML; k++) {
-    if (k < nsoil) {
-      smc[k] = (smc[k] > smcmin + SH2OMIN) ? smc[k] : smcmin + SH2OMIN;
-      smc[k] = (smc[k] < smcmax) ? smc[k] : smcmax;
-      sh2o[k] = (sh2o[k] < smc[k]) ? sh2o[k] : smc[k];
+  __syncthreads();
+
+  const int nwtbl = ltbl[lane];
+  const double sicemax = fmax(fmax(lmax[0][lane], lmax[1][lane]), fmax(lmax[2][lane], lmax[3][lane]));
+  if (nwtbl != 0) {
+    const double alpha = e.alpha[p], beta = e.beta[p];
+    WdfSoil ws;
+    ws.range = smcmax - smcmin;
+    ws.e1 = beta / (beta - 1.0);
+    ws.m = (beta - 1.0) / beta;
+    const double expon = 1.0 - 1.0 / beta;
+    ws.scale = (1.0 - expon) / alpha / expon / ws.range;
+    ws.ksatv = e.ksatv[p];
+    ws.smcmin = smcmin;
+    ws.sicemax = sicemax;
+    ws.vkwgt = 1.0;
+    if (sicemax > 0.0) {
+      const double i500 = 500.0 * sicemax;
+      ws.vkwgt = 1.0 / (1.0 + i500 * i500 * i500);
     }
-    sice[k] = smc[k] - sh2o[k];   // SmFlx: src/noah/noah.c:1676-1679
+    for (int k = wave; k < nsoil - 1; k += kSoilWaves) {
+      double wdf, wcnd;
+      wdf_cnd(&wdf, &wcnd, lsh[k][lane], ws);
+      la[k][lane] = wdf;
+      lb[k][lane] = wcnd;
+    }
   }
+  __syncthreads();
+  if (wave != 0) return;
+
+  double fcr = e.fcr[p], top;
   if (0 == nwtbl) {
-#pragma unroll
-    for (int k = 0; k < ML; k++) {
-      if (k < nsoil) {
-        smc[k] = smcmax;
-        sh2o[k] = smc[k] - sice[k];
-      }
+    for (int k = 0; k < nsoil; k++) {
+      put(s.smc, k, smcmax);
+      put(s.sh2o, k, smcmax - lic[k][lane]);
     }
+    top = smcmax - lic[0][lane];
   } else {
     // SRT: src/noah/noah.c:2315-2425
-    {
-      const double CVFRZ = 3.0;
-      double sicemax = 0.0, dice = 0.0;
-#pragma unroll
-      for (int k = 0; k < ML; k++) {
-        if (k < nsoil) {
-          sicemax = (sice[k] > sicemax) ? sice[k] : sicemax;
-          dice = (k == 0) ? -zsoil[0] * sice[0] : dice + (zsoil[k - 1] - zsoil[k]) * sice[k];
-        }
-      }
-      fcr = 1.0;
+    const double CVFRZ = 3.0;
+    fcr = 1.0;
+    if (sicemax > 0.0) {   // without ice dice is 0
+      double dice = 0.0;
+      for (int k = 0; k < nsoil; k++)
+        dice = (k == 0) ? -lz[0][lane] * lic[0][lane] : dice + (lz[k - 1][lane] - lz[k][lane]) * lic[k][lane];
       if (dice > 1.0e-2) {
         const double acrt = CVFRZ * s.frzx[p] / dice;
         double sum = 1.0;
@@ -239,164 +289,120 @@ __global__ __launch_bounds__(kBlock) void k_noah_soil(int ne, SoilDev s, ElemDev
         }
         fcr = 1.0 - exp(-acrt) * sum;
       }
-      const double pddum = s.infil[p];
-      WdfSoil ws;
-      ws.range = smcmax - smcmin;
-      ws.e1 = beta / (beta - 1.0);
-      ws.m = (beta - 1.0) / beta;
-      const double expon = 1.0 - 1.0 / beta;
-      ws.scale = (1.0 - expon) / alpha / expon / ws.range;
-      ws.ksatv = ksatv;
-      ws.smcmin = smcmin;
-      ws.sicemax = sicemax;
-      ws.vkwgt = 1.0;
-      if (sicemax > 0.0) {
-        const double i500 = 500.0 * sicemax;
-        ws.vkwgt = 1.0 / (1.0 + i500 * i500 * i500);
-      }
-      double wdf, wcnd;
-      double dsmdz = (sh2o[0] - sh2o[1]) / (-0.5 * zsoil[1]);
-      wdf_cnd(&wdf, &wcnd, sh2o[0], ws);
-      double ddz = 1.0 / (-0.5 * zsoil[1]);
-      ai[0] = 0.0;
-      bi[0] = wdf * ddz / (-zsoil[0]);
-      ci[0] = -bi[0];
-      rhstt[0] = (wdf * dsmdz + wcnd - pddum + e.edir[p] + at(e.et, 0)) / zsoil[0];
-      rhstt[0] += at(s.runoff2_lyr, 0) / zsoil[0];
-#pragma unroll
-      for (int k = 1; k < ML; k++) {
-        ai[k] = bi[k] = ci[k] = rhstt[k] = 0.0;
-        if (k < nsoil) {
-          const double denom2 = (zsoil[k - 1] - zsoil[k]);
-          double wdf2 = 0.0, wcnd2 = 0.0, dsmdz2 = 0.0, ddz2 = 0.0;
-          if (k + 1 < ML && k < nsoil - 1) {
-            const double denom = zsoil[k - 1] - zsoil[k + 1];
-            dsmdz2 = (sh2o[k] - sh2o[k + 1]) / (denom * 0.5);
-            wdf_cnd(&wdf2, &wcnd2, sh2o[k], ws);
-            ddz2 = 2.0 / denom;
-            ci[k] = -wdf2 * ddz2 / denom2;
-          } else {
-            ci[k] = 0.0;
-          }
-          double numer = (wdf2 * dsmdz2) + wcnd2 - (wdf * dsmdz) - wcnd + at(e.et, k);
-          numer += at(s.runoff2_lyr, k);
-          rhstt[k] = numer / (-denom2);
-          ai[k] = -wdf * ddz / denom2;
-          bi[k] = -(ai[k] + ci[k]);
-          if (k != nsoil - 1) {
-            wdf = wdf2;
-            wcnd = wcnd2;
-            dsmdz = dsmdz2;
-            ddz = ddz2;
-          }
-        }
-      }
     }
-    // SStep: src/noah/noah.c:2437-2480
-#pragma unroll
-    for (int k = 0; k < ML; k++) {
-      if (k < nsoil) {
-        rhstt[k] *= dt;
-        ai[k] *= dt;
-        bi[k] = 1.0 + bi[k] * dt;
-        ci[k] *= dt;
-        at(s.smflxv, k) = 0.0;
-      }
-    }
-    // Rosr12 (src/noah/noah.c:1572-1620) in place: ci becomes p, rhstt becomes
-    // delta; each entry is read before it is overwritten, so the arithmetic is
-    // the reference's, which works on copies
-#pragma unroll
-    for (int k = 0; k < ML; k++)
-      if (k == nsoil - 1) ci[k] = 0.0;
-    ci[0] = -ci[0] / bi[0];
-    rhstt[0] = rhstt[0] / bi[0];
-#pragma unroll
-    for (int k = 1; k < ML; k++) {
-      if (k < nsoil) {
-        const double inv = 1.0 / (bi[k] + ai[k] * ci[k - 1]);
-        const double pk = -ci[k] * inv;
-        rhstt[k] = (rhstt[k] - ai[k] * rhstt[k - 1]) * inv;
-        ci[k] = pk;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < ML; k++)
-      if (k == nsoil - 1) ci[k] = rhstt[k];
-#pragma unroll
-    for (int k = ML - 2; k >= 0; k--)
-      if (k <= nsoil - 2) ci[k] = ci[k] * ci[k + 1] + rhstt[k];
-    // the solution is added to sh2o; rhstt keeps the old values (sh2o0 of SStep)
-#pragma unroll
-    for (int k = 0; k < ML; k++) {
-      if (k < nsoil) {
-        rhstt[k] = sh2o[k];
-        sh2o[k] += ci[k];
-      }
-    }
-    // AdjSmProf: src/noah/noah.c:3081-3172 (ai holds sh2omid)
+    // SRT's coefficients, SStep (src/noah/noah.c:2437-2480) and the downward
+    // half of Rosr12 (:1572-1620) layer by layer: la becomes p, lb delta
+    const double pddum = s.infil[p];
+    double wdf = la[0][lane], wcnd = lb[0][lane];
+    double z0 = lz[0][lane], z1 = lz[1][lane], sh0 = lsh[0][lane], sh1 = lsh[1][lane];
+    double dsmdz = (sh0 - sh1) / (-0.5 * z1);
+    double ddz = 1.0 / (-0.5 * z1);
+    double pk, dk;
     {
-      double wplus = 0.0;
-#pragma unroll
-      for (int k = ML - 1; k >= 0; k--) {
-        if (k < nsoil) {
-          const double ddz = (k != 0) ? zsoil[k - 1] - zsoil[k] : -zsoil[0];
-          ai[k] = sh2o[k] + wplus / ddz;
-          const double stot = ai[k] + sice[k];
-          if (stot > smcmax) {
-            smc[k] = smcmax;
-            wplus = (stot - smcmax) * ddz;
-          } else {
-            const double sat = at(s.satdpth, k), sl = at(s.sldpth, k);
-            double stotmin = (sat * smcmax + (sl - sat) * (smcmin + SH2OMIN)) / sl;
-            stotmin = (stotmin > smcmax) ? smcmax : stotmin;
-            stotmin = (stotmin < smcmin + SH2OMIN) ? (smcmin + SH2OMIN) : stotmin;
-            if (stot < stotmin) {
-              smc[k] = stotmin;
-              wplus = (stot - stotmin) * ddz;
-            } else {
-              smc[k] = stot;
-              wplus = 0.0;
-            }
-          }
-          ai[k] = smc[k] - sice[k];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < ML; k++) {
-        if (k < nsoil) {
-          const double ddz = (k != 0) ? zsoil[k - 1] - zsoil[k] : -zsoil[0];
-          sh2o[k] = ai[k] + wplus / ddz;
-          const double stot = sh2o[k] + sice[k];
-          wplus = (stot > smcmax) ? (stot - smcmax) * ddz : 0.0;
-          smc[k] = (stot < smcmax) ? stot : smcmax;
-          smc[k] = (smc[k] > smcmin + SH2OMIN) ? smc[k] : (smcmin + SH2OMIN);
-          sh2o[k] = smc[k] - sice[k];
-          sh2o[k] = (sh2o[k] > 0.0) ? sh2o[k] : 0.0;
-        }
-      }
-      s.runoff3[p] = wplus / dt;
+      double bi = wdf * ddz / (-z0), ci = -bi;
+      double rhstt = (wdf * dsmdz + wcnd - pddum + e.edir[p] + at(e.et, 0)) / z0;
+      rhstt += at(s.runoff2_lyr, 0) / z0;
+      rhstt *= dt;
+      bi = 1.0 + bi * dt;
+      ci *= dt;
+      pk = -ci / bi;
+      dk = rhstt / bi;
+      la[0][lane] = pk;
+      lb[0][lane] = dk;
     }
-    // layer fluxes, bottom up (smflxv[nsoil - 1] stays 0)
-    double below = 0.0;
-#pragma unroll
-    for (int k = ML - 1; k >= 1; k--) {
-      if (k <= nsoil - 1) {
-        below = (sh2o[k] - rhstt[k]) * at(s.sldpth, k) / dt + at(s.runoff2_lyr, k) + at(e.et, k) + below;
-        at(s.smflxv, k - 1) = below;
+    for (int k = 1; k < nsoil; k++) {
+      const bool last = k == nsoil - 1;
+      const double denom2 = z0 - z1;
+      double wdf2 = 0.0, wcnd2 = 0.0, dsmdz2 = 0.0, ddz2 = 0.0, ci = 0.0, z2 = 0.0, sh2 = 0.0;
+      if (!last) {
+        z2 = lz[k + 1][lane];
+        sh2 = lsh[k + 1][lane];
+        const double denom = z0 - z2;
+        dsmdz2 = (sh1 - sh2) / (denom * 0.5);
+        wdf2 = la[k][lane];
+        wcnd2 = lb[k][lane];
+        ddz2 = 2.0 / denom;
+        ci = -wdf2 * ddz2 / denom2;
       }
+      double numer = (wdf2 * dsmdz2) + wcnd2 - (wdf * dsmdz) - wcnd + at(e.et, k);
+      numer += at(s.runoff2_lyr, k);
+      double rhstt = numer / (-denom2);
+      double ai = -wdf * ddz / denom2;
+      double bi = -(ai + ci);
+      rhstt *= dt;
+      ai *= dt;
+      bi = 1.0 + bi * dt;
+      ci = last ? 0.0 : ci * dt;
+      const double inv = 1.0 / (bi + ai * pk);
+      pk = -ci * inv;
+      dk = (rhstt - ai * dk) * inv;
+      la[k][lane] = pk;
+      lb[k][lane] = dk;
+      wdf = wdf2;
+      wcnd = wcnd2;
+      dsmdz = dsmdz2;
+      ddz = ddz2;
+      z0 = z1;
+      z1 = z2;
+      sh1 = sh2;
+    }
+    // the upward half of Rosr12, whose solution is added to sh2o, and
+    // AdjSmProf's upward pass (src/noah/noah.c:3081-3172): la becomes sh2omid
+    double wplus = 0.0, x = 0.0;
+    for (int k = nsoil - 1; k >= 0; k--) {
+      x = (k == nsoil - 1) ? lb[k][lane] : la[k][lane] * x + lb[k][lane];
+      const double ice = lic[k][lane];
+      const double ddzk = (k != 0) ? lz[k - 1][lane] - lz[k][lane] : -lz[0][lane];
+      const double mid = (lsh[k][lane] + x) + wplus / ddzk;
+      const double stot = mid + ice;
+      double smc;
+      if (stot > smcmax) {
+        smc = smcmax;
+        wplus = (stot - smcmax) * ddzk;
+      } else {
+        const double sat = lsat[k][lane], sl = at(s.sldpth, k);
+        double stotmin = (sat * smcmax + (sl - sat) * (smcmin + SH2OMIN)) / sl;
+        stotmin = (stotmin > smcmax) ? smcmax : stotmin;
+        stotmin = (stotmin < smcmin + SH2OMIN) ? (smcmin + SH2OMIN) : stotmin;
+        if (stot < stotmin) {
+          smc = stotmin;
+          wplus = (stot - stotmin) * ddzk;
+        } else {
+          smc = stot;
+          wplus = 0.0;
+        }
+      }
+      la[k][lane] = smc - ice;
+    }
+    // AdjSmProf's downward pass
+    for (int k = 0; k < nsoil; k++) {
+      const double ice = lic[k][lane];
+      const double ddzk = (k != 0) ? lz[k - 1][lane] - lz[k][lane] : -lz[0][lane];
+      double sh2o = la[k][lane] + wplus / ddzk;
+      const double stot = sh2o + ice;
+      wplus = (stot > smcmax) ? (stot - smcmax) * ddzk : 0.0;
+      double smc = (stot < smcmax) ? stot : smcmax;
+      smc = (smc > smcmin + SH2OMIN) ? smc : (smcmin + SH2OMIN);
+      sh2o = smc - ice;
+      sh2o = (sh2o > 0.0) ? sh2o : 0.0;
+      put(s.smc, k, smc);
+      put(s.sh2o, k, sh2o);
+      la[k][lane] = sh2o;
+    }
+    if (own) s.runoff3[p] = wplus / dt;
+    top = la[0][lane];
+    // layer fluxes, bottom up (smflxv[nsoil - 1] is 0)
+    double below = 0.0;
+    put(s.smflxv, nsoil - 1, 0.0);
+    for (int k = nsoil - 1; k >= 1; k--) {
+      below = (la[k][lane] - lsh[k][lane]) * at(s.sldpth, k) / dt + at(s.runoff2_lyr, k) + at(e.et, k) + below;
+      put(s.smflxv, k - 1, below);
     }
   }
 
-#pragma unroll
-  for (int k = 0; k < ML; k++) {
-    if (k < nsoil) {
-      at(s.smc, k) = smc[k];
-      at(s.sh2o, k) = sh2o[k];
-    }
-  }
   // what the next model step's RHS reads
-  e.sh2o0[p] = sh2o[0];
+  if (!own) return;
+  e.sh2o0[p] = top;
   e.fcr[p] = fcr;
   e.nwtbl[p] = nwtbl;
   const double ett = e.ett[p];
@@ -469,7 +475,7 @@ int download(pihm_noah_soil *s, const T *src, T *dst, int layers) {
 
 int launch(pihm_noah_soil *s, double dt, const double *y_dev) {
   pihm_ctx *c = s->ctx;
-  hipLaunchKernelGGL(k_noah_soil, dim3(div_up(s->ne, kBlock)), dim3(kBlock), 0, c->stream, s->ne, s->d, c->args.e,
+  hipLaunchKernelGGL(k_noah_soil, dim3(div_up(s->ne, kSoilCols)), dim3(kSoilCols * kSoilWaves), 0, c->stream, s->ne, s->d, c->args.e,
                      y_dev, dt);
   PIHM_HIP_TRY(hipGetLastError());
   return PIHM_OK;
