@@ -5,11 +5,12 @@
 // in the reference's operation order.  The soil column (smc, sh2o, at most 11
 // layers) is shared with the soil-water step and lives in HBM layer-major
 // ([k * ne + p]) so that a wavefront reads one layer of 64 neighbouring
-// elements together; the temperatures stc are stored the same way.  Inside
-// the thread the column is worked in private arrays.  The step ends by
+// elements together; the temperatures stc are stored the same way.  The
+// thread works on its column in LDS.  The step ends by
 // handing the RHS what it reads (pcpdrp, edir, ett, the layer transpiration,
-// sh2o[0]) and by refreshing GwTransp's share.  exp, log, log10, atan, sqrt
-// and pow are the device library's.
+// sh2o[0]) and by refreshing GwTransp's share.  Powers, and the logarithms of
+// the three loops that take most of the step, are xmath.hpp's; the rest are the
+// device library's.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -20,6 +21,7 @@
 #include "common.hpp"
 #include "ctx.hpp"
 #include "tsinterp.hpp"
+#include "xmath.hpp"
 
 using namespace pihm;
 
@@ -27,7 +29,6 @@ namespace {
 
 constexpr int ML = PIHM_NOAH_MAXLYR;
 // src/include/pihm_const.h:6-37,81
-constexpr double NPI = 3.14159265;
 constexpr double NGRAV = 9.80665;
 constexpr double NCP = 1004.0;
 constexpr double LVH2O = 2.501e6;
@@ -69,15 +70,29 @@ struct ColDev {
   double *pcpdrp, *edir, *ett, *et, *sh2o0;    // context step inputs and Noah hand-over
 };
 
+// One column's layers in LDS, layer k of 64 columns side by side.
+constexpr int kNoahBlock = 64;
+constexpr int NLAYARR = 7;
+struct Layers {
+  double *p;
+  __device__ double &operator[](int k) const { return p[k * kNoahBlock]; }
+};
+
+// ln of a positive number as a sum.
+struct LnPair {
+  double hi, lo;
+};
+
 // One element's working record: the reference's ps/ws/wf/es/ef fields the step
-// touches.  The layer arrays are the kernel's own locals: an array inside the
-// record, indexed at run time, would keep the whole record in scratch memory.
+// touches.  The layers are in LDS: an array inside the record, indexed at run
+// time, would keep the whole record in scratch memory.
 struct Col {
   int nsoil, nroot;
-  double *zsoil, *rtdis, *smc, *sh2o, *stc, *et;   // [ML]
+  Layers zsoil, smc, sh2o, stc, et, w1, w2;   // w1, w2: Transp's weights, then ShFlx's coefficients
+  LnPair lks;                                      // ln of the solids' conductivity
   // parameters
   double shdfac, cmcfactr, laimin, laimax, emissmin, emissmax, albedomin, albedomax, z0min, z0max, snup, cfactr;
-  double rgl, rsmin, rsmax, topt, hs, smcmax, smcmin, smcref, smcwlt, smcdry, quartz, alpha, beta, zlvl_wind;
+  double rgl, rsmin, rsmax, topt, hs, smcmax, smcmin, smcref, smcwlt, smcdry, alpha, beta, zlvl_wind;
   // carried
   double t1, sneqv, snowh, sndens, cmc, ch, cm, snotime1, albedo, emissi, q1;
   // forcing
@@ -107,7 +122,7 @@ __device__ __forceinline__ void cal_hum(Col &c, const NoahUni &u) {
 // CSnow: src/noah/noah.c:811-839
 __device__ __forceinline__ double c_snow(double dsnow) {
   const double UNIT = 0.11631;
-  const double cc = 0.328 * pow(10.0, 2.25 * dsnow);
+  const double cc = 0.328 * xpow(10.0, 2.25 * dsnow);
   return 2.0 * UNIT * cc;
 }
 
@@ -116,7 +131,7 @@ __device__ __forceinline__ void snow_new(Col &c, double newsn) {
   double snowhc = c.snowh * 100.0;
   const double newsnc = newsn * 100.0;
   const double tempc = c.sfctmp - 273.15;
-  const double dsnew = (tempc <= -15.0) ? 0.05 : 0.05 + 0.0017 * pow(tempc + 15.0, 1.5);
+  const double dsnew = (tempc <= -15.0) ? 0.05 : 0.05 + 0.0017 * xpow(tempc + 15.0, 1.5);
   const double hnewc = newsnc / dsnew;
   if (snowhc + hnewc < 0.001) c.sndens = (dsnew > c.sndens) ? dsnew : c.sndens;
   else c.sndens = (snowhc * c.sndens + hnewc * dsnew) / (snowhc + hnewc);
@@ -145,27 +160,73 @@ __device__ __forceinline__ void al_calc(Col &c, const NoahUni &u, double dt, int
     c.snotime1 = 0.0;
   } else {
     c.snotime1 += dt;
-    snoalb2 = snoalb1 * pow(SNACCA, pow(c.snotime1 / 86400.0, SNACCB));
+    snoalb2 = snoalb1 * xpow(SNACCA, xpow(c.snotime1 / 86400.0, SNACCB));
   }
   snoalb2 = (snoalb2 > c.alb) ? snoalb2 : c.alb;
   c.albedo = c.alb + c.sncovr * (snoalb2 - c.alb);
   c.albedo = (c.albedo > snoalb2) ? snoalb2 : c.albedo;
 }
 
-// TDfCnd: src/noah/noah.c:2520-2619
-__device__ __forceinline__ double tdf_cnd(double smc, double qz, double smcmax, double smcmin, double sh2o) {
-  const double THKICE = 2.2, THKQTZ = 7.7, THKW = 0.57;
+// ln x for any x: xmath's logarithm, a third of the library's instructions.
+__device__ __forceinline__ double ln_of(double x) {
+  if (x > 0.0 && x < HUGE_VAL) {
+    double lo;
+    return ln_pos(x, &lo);
+  }
+  return (x == 0.0) ? -HUGE_VAL : ((x < 0.0) ? NAN : x);
+}
+// Two of them in step.
+__device__ __forceinline__ void ln_of2(double a, double b, double *la, double *lb) {
+  if (a > 0.0 && a < HUGE_VAL && b > 0.0 && b < HUGE_VAL) {
+    const double x[2] = {a, b};
+    double hi[2], lo[2];
+    ln_pos_n<2>(x, hi, lo);
+    *la = hi[0];
+    *lb = hi[1];
+  } else {
+    *la = ln_of(a);
+    *lb = ln_of(b);
+  }
+}
+
+// a b + the pair (s, e), as a pair that carries the product's and the sum's
+// rounding.
+__device__ __forceinline__ void add_prod(double a, double b, double &s, double &e) {
+  const double p = a * b, t = s + p, z = t - s;
+  e += fma(a, b, -p) + ((s - (t - z)) + (p - z));
+  s = t;
+}
+
+// TDfCnd: src/noah/noah.c:2520-2619.  The solids' conductivity is quartz's
+// power times the other minerals', 7.7^q 2^(1-q), and the saturated one a
+// product of three powers: one exponential of the sum of their logarithms, the
+// sum carried as a pair.  lks is the solids' logarithm, one value per column.
+__device__ __forceinline__ LnPair ln_solids(double qz) {
+  const double LNQTZ = 2.0412203288596382, LNQTZ_LO = -3.402197230721298e-17;   // ln 7.7
+  const double LNO = 0.6931471805599453, LNO_LO = 2.3190468138462996e-17;       // ln 2
+  const double r = 1.0 - qz;
+  LnPair l{0.0, qz * LNQTZ_LO + r * LNO_LO};
+  add_prod(qz, LNQTZ, l.hi, l.lo);
+  add_prod(r, LNO, l.hi, l.lo);
+  return l;
+}
+__device__ __forceinline__ double tdf_cnd(double smc, const LnPair &lks, double smcmax, double smcmin, double sh2o) {
+  const double LNICE = 0.7884573603642703, LNICE_LO = -2.639344289064807e-17;   // ln 2.2
+  const double LNW = -0.5621189181535413, LNW_LO = 1.1409357209435452e-17;      // ln 0.57
   const double satratio = (smc - smcmin) / (smcmax - smcmin);
-  const double thko = 2.0;
-  const double thks = pow(THKQTZ, qz) * pow(thko, 1.0 - qz);
   const double xunfroz = sh2o / smc;
   const double xu = xunfroz * smcmax;
-  const double thksat = pow(thks, 1.0 - smcmax) * pow(THKICE, smcmax - xu) * pow(THKW, xu);
+  const double a = 1.0 - smcmax, b = smcmax - xu;
+  double hi = 0.0, lo = a * lks.lo + b * LNICE_LO + xu * LNW_LO;
+  add_prod(a, lks.hi, hi, lo);
+  add_prod(b, LNICE, hi, lo);
+  add_prod(xu, LNW, hi, lo);
+  const double thksat = exp_pair(hi, lo);
   const double gammd = (1.0 - smcmax) * 2700.0;
   const double thkdry = (0.135 * gammd + 64.7) / (2700.0 - 0.947 * gammd);
   double ake;
   if ((sh2o + 0.0005) < smc) ake = satratio;
-  else if (satratio > 0.1) ake = log10(satratio) + 1.0;
+  else if (satratio > 0.1) ake = ln_of(satratio) * 0.43429448190325183 + 1.0;   // log10
   else ake = 0.0;
   return ake * (thksat - thkdry) + thkdry;
 }
@@ -178,16 +239,15 @@ __device__ __forceinline__ double snow_z0(double sncovr, double z0brd, double sn
   return (1.0 - sncovr) * z0brd + sncovr * z0eff;
 }
 
-// Paulson's stability functions: src/noah/noah.c:3204-3222
-__device__ __forceinline__ double psp_mu(double xx) {
-  return -2.0 * log((xx + 1.0) * 0.5) - log((xx * xx + 1.0) * 0.5) + 2.0 * atan(xx) - NPI * 0.5;
-}
-__device__ __forceinline__ double psp_hu(double xx) { return -2.0 * log((xx * xx + 1.0) * 0.5); }
-
 // SfcDifOff: src/noah/noah.c:2862-3079 with iz0tlnd = 0 and Paulson's
-// functions (ilech = 0; the Lech branches are never taken)
+// functions (ilech = 0; the Lech branches are never taken; :3204-3222).  Only
+// differences of Paulson's functions at two heights are needed, and they are
+// added to the logarithm of a ratio of heights, so that the logarithms of a
+// pass are two, taken in step, and the arctangents one:
+//   mu(a) - mu(b) = ln [(b+1)^2 (b^2+1) / ((a+1)^2 (a^2+1))] + 2 atan((a-b)/(1+ab))
+//   hu(a) - hu(b) = 2 ln [(b^2+1) / (a^2+1)]          for a >= b >= 1
 __device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, double z0, double czil, double sfcspd, double t1v,
-                            double th2v, double &cm, double &ch) {
+                                            double th2v, double &cm, double &ch) {
   const double WWST = 1.2, VKRM = 0.40, EXCM = 0.001, BETA = 1.0 / 270.0;
   const double WOLD = 0.15;
   const int ITRMX = 5;
@@ -204,56 +264,59 @@ __device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, doubl
   double du2 = sfcspd * sfcspd;
   du2 = (du2 > EPSU2) ? du2 : EPSU2;
   const double btgh = btg * HPBL;
-  double wstar2 = (btgh * ch * dthv != 0.0) ? wwst2 * pow(fabs(btgh * ch * dthv), 2.0 / 3.0) : 0.0;
-  double ustar = sqrt(cm * sqrt(du2 + wstar2));
-  ustar = (ustar > EPSUST) ? ustar : EPSUST;
-  double zt = exp(zilfc * sqrt(ustar * z0)) * z0;
+  auto wstar2_of = [&](double chv) {
+    return (btgh * chv * dthv != 0.0) ? wwst2 * xpow(fabs(btgh * chv * dthv), 2.0 / 3.0) : 0.0;
+  };
+  auto ustar_of = [&](double cmv, double w) {
+    const double us = sqrt_pos(cmv * sqrt_pos(du2 + w));
+    return (us > EPSUST) ? us : EPSUST;
+  };
+  double wstar2 = wstar2_of(ch);
+  double ustar = ustar_of(cm, wstar2);
+  double zt = exp(zilfc * sqrt_pos(ustar * z0)) * z0;
   const double zslu = zlvl_wind + zu;
   double zslt = zlvl + zt;
-  const double rlogu = log(zslu / zu);
-  double rlogt = log(zslt / zt);
-  double rlmo = elfc * ch * dthv / pow(ustar, 3.0);
+  const double ratu = zslu / zu;
+  double ratt = fdiv(zslt, zt);
+  double rlmo = fdiv(elfc * ch * dthv, xpow(ustar, 3.0));
+#pragma unroll 1
   for (int itr = 0; itr < ITRMX; itr++) {
     double zetalt = zslt * rlmo;
     zetalt = zetalt > ZTMIN ? zetalt : ZTMIN;
-    rlmo = zetalt / zslt;
+    rlmo = fdiv(zetalt, zslt);
     double zetalu = zslu * rlmo;
     const double zetau = zu * rlmo;
     const double zetat = zt * rlmo;
-    double simm, simh;
+    double simm, simh, lu = ratu, lt = ratt;
     if (rlmo < 0.0) {
-      const double xlu4 = 1.0 - 16.0 * zetalu;
-      const double xlt4 = 1.0 - 16.0 * zetalt;
-      const double xu4 = 1.0 - 16.0 * zetau;
-      const double xt4 = 1.0 - 16.0 * zetat;
-      const double xlu = sqrt(sqrt(xlu4));
-      const double xlt = sqrt(sqrt(xlt4));
-      const double xu = sqrt(sqrt(xu4));
-      const double xt = sqrt(sqrt(xt4));
-      const double psmz = psp_mu(xu);
-      simm = psp_mu(xlu) - psmz + rlogu;
-      const double pshz = psp_hu(xt);
-      simh = psp_hu(xlt) - pshz + rlogt;
+      const double slu = sqrt_pos(1.0 - 16.0 * zetalu), su = sqrt_pos(1.0 - 16.0 * zetau);
+      const double xlu = sqrt_pos(slu), xu = sqrt_pos(su);
+      const double ru = fdiv((xu + 1.0) * (xu + 1.0) * (su + 1.0), (xlu + 1.0) * (xlu + 1.0) * (slu + 1.0));
+      const double rt = fdiv(sqrt_pos(1.0 - 16.0 * zetat) + 1.0, sqrt_pos(1.0 - 16.0 * zetalt) + 1.0);
+      simm = 2.0 * atan(fdiv(xlu - xu, 1.0 + xlu * xu));
+      simh = 0.0;
+      lu *= ru;
+      lt *= rt * rt;
     } else {
       zetalu = (zetalu < ZTMAX) ? zetalu : ZTMAX;
       zetalt = (zetalt < ZTMAX) ? zetalt : ZTMAX;
-      const double psmz = 5.0 * zetau;
-      simm = 5.0 * zetalu - psmz + rlogu;
-      const double pshz = 5.0 * zetat;
-      simh = 5.0 * zetalt - pshz + rlogt;
+      simm = 5.0 * zetalu - 5.0 * zetau;
+      simh = 5.0 * zetalt - 5.0 * zetat;
     }
-    ustar = sqrt(cm * sqrt(du2 + wstar2));
-    ustar = (ustar > EPSUST) ? ustar : EPSUST;
-    zt = exp(zilfc * sqrt(ustar * z0)) * z0;
+    ln_of2(lu, lt, &lu, &lt);
+    simm += lu;
+    simh += lt;
+    ustar = ustar_of(cm, wstar2);
+    zt = exp(zilfc * sqrt_pos(ustar * z0)) * z0;
     zslt = zlvl + zt;
-    rlogt = log(zslt / zt);
+    ratt = fdiv(zslt, zt);
     const double ustark = ustar * VKRM;
-    cm = (ustark / simm > cxch) ? ustark / simm : cxch;
-    ch = (ustark / simh > cxch) ? ustark / simh : cxch;
-    wstar2 = (btgh * ch * dthv != 0.0) ? wwst2 * pow(fabs(btgh * ch * dthv), 2.0 / 3.0) : 0.0;
-    const double rlmn = elfc * ch * dthv / pow(ustar, 3.0);
-    const double rlma = rlmo * WOLD + rlmn * wnew;
-    rlmo = rlma;
+    const double cmn = fdiv(ustark, simm), chn = fdiv(ustark, simh);
+    cm = (cmn > cxch) ? cmn : cxch;
+    ch = (chn > cxch) ? chn : cxch;
+    wstar2 = wstar2_of(ch);
+    const double rlmn = fdiv(elfc * ch * dthv, xpow(ustar, 3.0));
+    rlmo = rlmo * WOLD + rlmn * wnew;
   }
 }
 
@@ -292,26 +355,24 @@ __device__ __forceinline__ void can_res(Col &c) {
   const double ff = 0.55 * 2.0 * c.soldn / (c.rgl * c.proj_lai);
   double rcs = (ff + c.rsmin / c.rsmax) / (1.0 + ff);
   rcs = (rcs > 0.0001) ? rcs : 0.0001;
-  double rct = 1.0 - 0.0016 * pow(c.topt - c.sfctmp, 2.0);
+  const double dtopt = c.topt - c.sfctmp, t2 = c.sfctmp * c.sfctmp;
+  double rct = 1.0 - 0.0016 * (dtopt * dtopt);
   rct = (rct > 0.0001) ? rct : 0.0001;
   double rcq = 1.0 / (1.0 + c.hs * (c.q2sat - c.q2));
   rcq = (rcq > 0.01) ? rcq : 0.01;
-  double part[ML];
   double gx = (c.sh2o[0] - c.smcwlt) / (c.smcref - c.smcwlt);
   gx = (gx > 1.0) ? 1.0 : gx;
   gx = (gx < 0.0) ? 0.0 : gx;
-  part[0] = (c.zsoil[0] / c.zsoil[c.nroot - 1]) * gx;
+  double rcsoil = (c.zsoil[0] / c.zsoil[c.nroot - 1]) * gx;
   for (int k = 1; k < c.nroot; k++) {
     gx = (c.sh2o[k] - c.smcwlt) / (c.smcref - c.smcwlt);
     gx = (gx > 1.0) ? 1.0 : gx;
     gx = (gx < 0.0) ? 0.0 : gx;
-    part[k] = ((c.zsoil[k] - c.zsoil[k - 1]) / c.zsoil[c.nroot - 1]) * gx;
+    rcsoil += ((c.zsoil[k] - c.zsoil[k - 1]) / c.zsoil[c.nroot - 1]) * gx;
   }
-  double rcsoil = 0.0;
-  for (int k = 0; k < c.nroot; k++) rcsoil += part[k];
   rcsoil = (rcsoil > 0.0001) ? rcsoil : 0.0001;
   c.rc = c.rsmin / (c.proj_lai * rcs * rct * rcq * rcsoil);
-  const double rr = (4.0 * c.emissi * SIGMA * RD / NCP) * pow(c.sfctmp, 4.0) / (c.sfcprs * c.ch) + 1.0;
+  const double rr = (4.0 * c.emissi * SIGMA * RD / NCP) * (t2 * t2) / (c.sfcprs * c.ch) + 1.0;
   const double delta = (SLV / NCP) * c.dqsdt2;
   c.pc = (rr + delta) / (rr * (1.0 + c.rc * c.ch) + delta);
 }
@@ -321,7 +382,7 @@ __device__ __forceinline__ void d_evap(Col &c, const NoahUni &u) {
   const double sratio = (c.sh2o[0] - c.smcdry) / (c.smcmax - c.smcdry);
   double fx = 0.0;
   if (sratio > 0.0) {
-    fx = pow(sratio, u.fxexp);
+    fx = xpow(sratio, u.fxexp);
     fx = (fx > 1.0) ? 1.0 : fx;
     fx = (fx < 0.0) ? 0.0 : fx;
   }
@@ -332,9 +393,9 @@ __device__ __forceinline__ void d_evap(Col &c, const NoahUni &u) {
 __device__ __forceinline__ void transp(Col &c) {
   for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
   double etpa;
-  if (c.cmc != 0.0) etpa = c.shdfac * c.pc * c.etp * (1.0 - pow(c.cmc / c.cmcmax, c.cfactr));
+  if (c.cmc != 0.0) etpa = c.shdfac * c.pc * c.etp * (1.0 - xpow(c.cmc / c.cmcmax, c.cfactr));
   else etpa = c.shdfac * c.pc * c.etp;
-  double gx[ML];
+  const Layers &gx = c.w1;
   double sgx = 0.0;
   for (int i = 0; i < c.nroot; i++) {
     gx[i] = (c.smc[i] - c.smcwlt) / (c.smcref - c.smcwlt);
@@ -345,7 +406,7 @@ __device__ __forceinline__ void transp(Col &c) {
   sgx /= (double)c.nroot;
   double denom = 0.0;
   for (int i = 0; i < c.nroot; i++) {
-    const double rtx = c.rtdis[i] + gx[i] - sgx;
+    const double rtx = c.w2[i] + gx[i] - sgx;
     gx[i] *= ((rtx > 0.0) ? rtx : 0.0);
     denom += gx[i];
   }
@@ -365,7 +426,7 @@ __device__ __forceinline__ void evapo(Col &c, const NoahUni &u, double dt) {
       transp(c);
       for (int k = 0; k < c.nsoil; k++) c.ett += c.et[k];
       if (c.cmc > 0.0)
-        c.ec = c.shdfac * pow((c.cmc / c.cmcmax > 1.0) ? 1.0 : c.cmc / c.cmcmax, c.cfactr) * c.etp;
+        c.ec = c.shdfac * xpow((c.cmc / c.cmcmax > 1.0) ? 1.0 : c.cmc / c.cmcmax, c.cfactr) * c.etp;
       else
         c.ec = 0.0;
       const double cmc2ms = c.cmc / dt;
@@ -395,14 +456,14 @@ __device__ __forceinline__ void pcp_drp(Col &c, double prcp, double dt) {
 }
 
 // TBnd: src/noah/noah.c:2482-2518
-__device__ __forceinline__ double t_bnd(double tu, double tb, const double *zsoil, double zbot, int k, int nsoil) {
+__device__ __forceinline__ double t_bnd(double tu, double tb, const Layers &zsoil, double zbot, int k, int nsoil) {
   const double zup = (k == 0) ? 0.0 : zsoil[k - 1];
   const double zb = (k == nsoil - 1) ? 2.0 * zbot - zsoil[k] : zsoil[k + 1];
   return tu + (tb - tu) * (zup - zsoil[k]) / (zup - zb);
 }
 
 // TmpAvg: src/noah/noah.c:2621-2723
-__device__ __forceinline__ double tmp_avg(double tup, double tm, double tdn, const double *zsoil, int k) {
+__device__ __forceinline__ double tmp_avg(double tup, double tm, double tdn, const Layers &zsoil, int k) {
   const double dz = (k == 0) ? -zsoil[0] : zsoil[k - 1] - zsoil[k];
   const double dzh = dz * 0.5;
   double tavg;
@@ -455,15 +516,18 @@ __device__ __forceinline__ double fr_h2o(double tkelv, double smc, double sh2o, 
   swl = (swl > smc - SH2OMIN) ? (smc - SH2OMIN) : swl;
   swl = (swl < 0.0) ? 0.0 : swl;
   int nlog = 0, kcount = 0;
-  double mx = 0.0;
+  const double mx = beta / (1.0 - beta);
+  const double range = smcmax - smcmin, ibeta = 1.0 / beta, kd = 1.0 / (beta - 1.0) / range;
+  double la, lt;
+  ln_of2(NGRAV / alpha / LSUBF, -(tkelv - TFREEZ) / tkelv, &la, &lt);
   while (nlog < 10 && kcount == 0) {
     nlog++;
-    const double satn = (smc - swl - smcmin) / (smcmax - smcmin);
-    mx = beta / (1.0 - beta);
-    const double df = log(NGRAV / alpha / LSUBF) + 1.0 / beta * log(pow(satn, mx) - 1.0) +
-                      2.0 * log(1.0 + CK * swl) - log(-(tkelv - TFREEZ) / tkelv);
-    const double denom = 1.0 / (beta - 1.0) / (smcmax - smcmin) * pow(satn, mx - 1.0) / (pow(satn, mx) - 1.0) +
-                         2.0 * CK / (1.0 + CK * swl);
+    const double satn = (smc - swl - smcmin) / range;
+    const double pw = xpow(satn, mx);          // satn^(mx-1) below is pw / satn
+    double lp, lc;
+    ln_of2(pw - 1.0, 1.0 + CK * swl, &lp, &lc);
+    const double df = la + ibeta * lp + 2.0 * lc - lt;
+    const double denom = kd * (pw / satn) / (pw - 1.0) + 2.0 * CK / (1.0 + CK * swl);
     double swlk = swl - df / denom;
     swlk = (swlk > smc - SH2OMIN) ? (smc - SH2OMIN) : swlk;
     swlk = (swlk < 0.0) ? 0.0 : swlk;
@@ -473,7 +537,7 @@ __device__ __forceinline__ double fr_h2o(double tkelv, double smc, double sh2o, 
   }
   double freew = smc - swl;
   if (kcount == 0) {
-    double fk = pow(pow(-(tkelv - TFREEZ) / tkelv * alpha * LSUBF / NGRAV, beta), 1.0 / mx) * (smcmax - smcmin) -
+    double fk = xpow(xpow(-(tkelv - TFREEZ) / tkelv * alpha * LSUBF / NGRAV, beta), 1.0 / mx) * (smcmax - smcmin) -
                 smcmin;
     fk = (fk < SH2OMIN) ? SH2OMIN : fk;
     freew = (fk < smc) ? fk : smc;
@@ -503,117 +567,80 @@ __device__ __forceinline__ void sh_flx(Col &c, const NoahUni &u, double dt, doub
   const double CH2O = 4.2e6;
   const int nsoil = c.nsoil;
   const double csoil_loc = u.csoil;
-  double ai[ML], bi[ML], ci[ML], rhsts[ML];
-  // HRT: top layer
-  double hcpct = c.sh2o[0] * CH2O + (1.0 - c.smcmax) * csoil_loc + (c.smcmax - c.smc[0]) * NCP +
-                 (c.smc[0] - c.sh2o[0]) * CPICE;
-  double ddz = 1.0 / (-0.5 * c.zsoil[1]);
-  ai[0] = 0.0;
-  ci[0] = (df1 * ddz) / (c.zsoil[0] * hcpct);
-  bi[0] = -ci[0] + df1 / (0.5 * c.zsoil[0] * c.zsoil[0] * hcpct * zz1);
-  double dtsdz = (c.stc[0] - c.stc[1]) / (-0.5 * c.zsoil[1]);
-  c.ssoil = df1 * (c.stc[0] - yy) / (0.5 * c.zsoil[0] * zz1);
-  double denom = c.zsoil[0] * hcpct;
-  rhsts[0] = (df1 * dtsdz - c.ssoil) / denom;
-  double qtot = -1.0 * rhsts[0] * denom;
-  double sice = c.smc[0] - c.sh2o[0];
-  const double tsurf = (yy + (zz1 - 1.0) * c.stc[0]) / zz1;
-  double tbk = t_bnd(c.stc[0], c.stc[1], c.zsoil, u.zbot, 0, nsoil);
-  if ((sice > 0.0) || (c.stc[0] < TFREEZ) || (tsurf < TFREEZ) || (tbk < TFREEZ)) {
-    const double tavg = tmp_avg(tsurf, c.stc[0], tbk, c.zsoil, 0);
-    const double tsnsr = snk_src(c, tavg, 0, dt, qtot);
-    rhsts[0] -= tsnsr / denom;
-  }
-  // HRT: the layers below
-  double ddz2 = 0.0, df1k = df1, dtsdz2 = 0.0, tbk1 = 0.0;
-  for (int k = 1; k < nsoil; k++) {
-    hcpct = c.sh2o[k] * CH2O + (1.0 - c.smcmax) * csoil_loc + (c.smcmax - c.smc[k]) * NCP +
-            (c.smc[k] - c.sh2o[k]) * CPICE;
-    double df1n;
-    if (k != nsoil - 1) {
-      df1n = tdf_cnd(c.smc[k], c.quartz, c.smcmax, c.smcmin, c.sh2o[k]);
-      denom = 0.5 * (c.zsoil[k - 1] - c.zsoil[k + 1]);
-      dtsdz2 = (c.stc[k] - c.stc[k + 1]) / denom;
-      ddz2 = 2.0 / (c.zsoil[k - 1] - c.zsoil[k + 1]);
-      ci[k] = -df1n * ddz2 / ((c.zsoil[k - 1] - c.zsoil[k]) * hcpct);
-      tbk1 = t_bnd(c.stc[k], c.stc[k + 1], c.zsoil, u.zbot, k, nsoil);
+  const Layers &ci = c.w1, &rhsts = c.w2;   // Rosr12's p and delta
+  // HRT, the top layer and those below in one loop, so that the sink term's
+  // code is there once and a layer's branch is taken by all columns together
+  double ddz = 0.0, df1k = df1, dtsdz = 0.0, tup = 0.0, pk = 0.0, dk = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < nsoil; k++) {
+    const double smc = c.smc[k], sh2o = c.sh2o[k], stc = c.stc[k];
+    const double hcpct = sh2o * CH2O + (1.0 - c.smcmax) * csoil_loc + (c.smcmax - smc) * NCP + (smc - sh2o) * CPICE;
+    double denom, tdn, ak, bk, ck, rk;
+    if (k == 0) {
+      ddz = 1.0 / (-0.5 * c.zsoil[1]);
+      ak = 0.0;
+      ck = (df1 * ddz) / (c.zsoil[0] * hcpct);
+      bk = -ck + df1 / (0.5 * c.zsoil[0] * c.zsoil[0] * hcpct * zz1);
+      dtsdz = (stc - c.stc[1]) / (-0.5 * c.zsoil[1]);
+      c.ssoil = df1 * (stc - yy) / (0.5 * c.zsoil[0] * zz1);
+      denom = c.zsoil[0] * hcpct;
+      rk = (df1 * dtsdz - c.ssoil) / denom;
+      tup = (yy + (zz1 - 1.0) * stc) / zz1;
+      tdn = t_bnd(stc, c.stc[1], c.zsoil, u.zbot, 0, nsoil);
     } else {
-      df1n = tdf_cnd(c.smc[k], c.quartz, c.smcmax, c.smcmin, c.sh2o[k]);
-      denom = 0.5 * (c.zsoil[k - 1] + c.zsoil[k]) - u.zbot;
-      dtsdz2 = (c.stc[k] - u.tbot) / denom;
-      ci[k] = 0.0;
-      tbk1 = t_bnd(c.stc[k], u.tbot, c.zsoil, u.zbot, k, nsoil);
+      const bool last = k == nsoil - 1;
+      const double zu = c.zsoil[k - 1], zk = c.zsoil[k], tn = last ? u.tbot : c.stc[k + 1];
+      const double df1n = tdf_cnd(smc, c.lks, c.smcmax, c.smcmin, sh2o);
+      double ddz2 = ddz;                       // the last layer's goes unread
+      if (last) {
+        denom = 0.5 * (zu + zk) - u.zbot;
+        ck = 0.0;
+      } else {
+        denom = 0.5 * (zu - c.zsoil[k + 1]);
+        ddz2 = 2.0 / (zu - c.zsoil[k + 1]);
+        ck = -df1n * ddz2 / ((zu - zk) * hcpct);
+      }
+      const double dtsdz2 = (stc - tn) / denom;
+      tdn = t_bnd(stc, tn, c.zsoil, u.zbot, k, nsoil);
+      denom = (zk - zu) * hcpct;
+      rk = (df1n * dtsdz2 - df1k * dtsdz) / denom;
+      ak = -df1k * ddz / ((zu - zk) * hcpct);
+      bk = -(ak + ck);
+      df1k = df1n;
+      dtsdz = dtsdz2;
+      ddz = ddz2;
     }
-    denom = (c.zsoil[k] - c.zsoil[k - 1]) * hcpct;
-    rhsts[k] = (df1n * dtsdz2 - df1k * dtsdz) / denom;
-    qtot = -1.0 * denom * rhsts[k];
-    sice = c.smc[k] - c.sh2o[k];
-    const double tavg = tmp_avg(tbk, c.stc[k], tbk1, c.zsoil, k);
-    if ((sice > 0.0) || (c.stc[k] < TFREEZ) || (tbk < TFREEZ) || (tbk1 < TFREEZ)) {
+    if ((smc - sh2o > 0.0) || (stc < TFREEZ) || (tup < TFREEZ) || (tdn < TFREEZ)) {
+      const double qtot = -1.0 * denom * rk;
+      const double tavg = tmp_avg(tup, stc, tdn, c.zsoil, k);
       const double tsnsr = snk_src(c, tavg, k, dt, qtot);
-      rhsts[k] = rhsts[k] - tsnsr / denom;
+      rk -= tsnsr / denom;
     }
-    ai[k] = -df1k * ddz / ((c.zsoil[k - 1] - c.zsoil[k]) * hcpct);
-    bi[k] = -(ai[k] + ci[k]);
-    tbk = tbk1;
-    df1k = df1n;
-    dtsdz = dtsdz2;
-    ddz = ddz2;
-  }
-  // HStep and Rosr12 in place, layer by layer: ci becomes p, rhsts becomes
-  // delta; each entry is read before it is overwritten, so the arithmetic is
-  // the reference's, which works on copies
-  {
-    double bk = 1.0 + bi[0] * dt, ck = (nsoil == 1) ? 0.0 : ci[0] * dt;
-    ci[0] = -ck / bk;
-    rhsts[0] = (rhsts[0] * dt) / bk;
-    for (int k = 1; k < nsoil; k++) {
-      const double ak = ai[k] * dt;
-      bk = 1.0 + bi[k] * dt;
-      ck = (k == nsoil - 1) ? 0.0 : ci[k] * dt;
-      const double inv = 1.0 / (bk + ak * ci[k - 1]);
-      ci[k] = -ck * inv;
-      rhsts[k] = (rhsts[k] * dt - ak * rhsts[k - 1]) * inv;
+    tup = tdn;
+    // HStep and the downward half of Rosr12
+    ak *= dt;
+    bk = 1.0 + bk * dt;
+    ck = (k == nsoil - 1) ? 0.0 : ck * dt;
+    if (k == 0) {
+      pk = -ck / bk;
+      dk = (rk * dt) / bk;
+    } else {
+      const double inv = 1.0 / (bk + ak * pk);
+      pk = -ck * inv;
+      dk = (rk * dt - ak * dk) * inv;
     }
-    ci[nsoil - 1] = rhsts[nsoil - 1];
-    for (int k = nsoil - 2; k >= 0; k--) ci[k] = ci[k] * ci[k + 1] + rhsts[k];
+    ci[k] = pk;
+    rhsts[k] = dk;
   }
-  for (int k = 0; k < nsoil; k++) c.stc[k] += ci[k];
+  // the upward half, added to the temperatures
+  double xk = rhsts[nsoil - 1];
+  c.stc[nsoil - 1] += xk;
+  for (int k = nsoil - 2; k >= 0; k--) {
+    xk = ci[k] * xk + rhsts[k];
+    c.stc[k] += xk;
+  }
   c.t1 = (yy + (zz1 - 1.0) * c.stc[0]) / zz1;
   c.ssoil = df1 * (c.stc[0] - c.t1) / (0.5 * c.zsoil[0]);
-}
-
-// NoPac: src/noah/noah.c:1343-1449
-__device__ __forceinline__ void no_pac(Col &c, const NoahUni &u, double dt, double t24) {
-  double prcpf = c.prcp;
-  c.dew = 0.0;
-  c.edir = 0.0;
-  c.ec = 0.0;
-  for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
-  c.ett = 0.0;
-  if (c.etp > 0.0) {
-    evapo(c, u, dt);
-    c.eta = c.etns;
-  } else {
-    c.dew = -c.etp;
-    prcpf += c.dew;
-  }
-  pcp_drp(c, prcpf, dt);
-  if (c.etp <= 0.0) {
-    c.beta_ = 0.0;
-    c.eta = c.etp;
-    if (c.etp < 0.0) c.beta_ = 1.0;
-  } else {
-    c.beta_ = c.eta / c.etp;
-  }
-  double df1 = tdf_cnd(c.smc[0], c.quartz, c.smcmax, c.smcmin, c.sh2o[0]);
-  df1 *= exp(u.sbeta * c.shdfac);
-  const double yynum = c.fdown - c.emissi * SIGMA * t24;
-  const double yy = c.sfctmp + (yynum / c.rch + c.th2 - c.sfctmp - c.beta_ * c.epsca) / c.rr;
-  const double zz1 = df1 / (-0.5 * c.zsoil[0] * c.rch * c.rr) + 1.0;
-  sh_flx(c, u, dt, yy, zz1, df1);
-  c.flx1 = CPH2O * c.prcp * 1000.0 * (c.t1 - c.sfctmp);
-  c.flx3 = 0.0;
 }
 
 // SnowPack: src/noah/noah.c:2100-2200
@@ -642,15 +669,10 @@ __device__ __forceinline__ void snow_pack(double esd, double dtsec, double &snow
   snowh = snowhc * 0.01;
 }
 
-// SnoPac: src/noah/noah.c:1813-2098
-__device__ __forceinline__ void sno_pac(Col &c, const NoahUni &u, int snowng, double dt, double t24, double prcpf, double df1) {
-  const double ESDMIN = 1.0e-6, SNOEXP = 2.0;
-  c.dew = 0.0;
-  c.edir = 0.0;
-  c.ec = 0.0;
-  for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
-  c.ett = 0.0;
-  c.esnow = 0.0;
+// SnoPac (src/noah/noah.c:1813-2098) up to PcpDrp, Evapo apart; returns the
+// water that reaches the canopy.
+__device__ __forceinline__ double sno_pac(Col &c, int snowng, double dt, double t24, double prcpf, double df1) {
+  const double ESDMIN = 1.0e-6;
   double esnow2 = 0.0, etanrg;
   c.beta_ = 1.0;
   if (c.etp <= 0.0) {
@@ -661,7 +683,6 @@ __device__ __forceinline__ void sno_pac(Col &c, const NoahUni &u, int snowng, do
     etanrg = c.etp * 1000.0 * ((1.0 - c.sncovr) * LVH2O + c.sncovr * LSUBS);
   } else {
     if (c.sncovr < 1.0) {
-      evapo(c, u, dt);
       c.edir *= (1.0 - c.sncovr);
       c.ec *= (1.0 - c.sncovr);
       for (int k = 0; k < c.nsoil; k++) c.et[k] = c.et[k] * (1.0 - c.sncovr);
@@ -697,7 +718,7 @@ __device__ __forceinline__ void sno_pac(Col &c, const NoahUni &u, int snowng, do
     ex = 0.0;
     c.snomlt = 0.0;
   } else {
-    c.t1 = TFREEZ * pow(c.sncovr, SNOEXP) + t12 * (1.0 - pow(c.sncovr, SNOEXP));
+    c.t1 = TFREEZ * (c.sncovr * c.sncovr) + t12 * (1.0 - c.sncovr * c.sncovr);
     c.beta_ = 1.0;
     c.ssoil = df1 * (c.t1 - c.stc[0]) / dtot;
     if (c.sneqv - esnow2 <= ESDMIN) {
@@ -725,12 +746,56 @@ __device__ __forceinline__ void sno_pac(Col &c, const NoahUni &u, int snowng, do
     }
     prcpf += ex;
   }
+  return prcpf;
+}
+
+// NoPac (src/noah/noah.c:1343-1449) and SnoPac.  Columns with and without snow
+// share wavefronts, so what both do - Evapo, PcpDrp and ShFlx, most of the
+// work - stands outside the branch on the snow.
+__device__ __forceinline__ void pac(Col &c, const NoahUni &u, bool snow, int snowng, double dt, double t24, double prcpf,
+                                    double df1) {
+  c.dew = 0.0;
+  c.edir = 0.0;
+  c.ec = 0.0;
+  for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
+  c.ett = 0.0;
+  c.esnow = 0.0;
+  if (c.etp > 0.0 && (!snow || c.sncovr < 1.0)) evapo(c, u, dt);
+  if (snow) {
+    prcpf = sno_pac(c, snowng, dt, t24, prcpf, df1);
+  } else {
+    prcpf = c.prcp;
+    if (c.etp > 0.0) {
+      c.eta = c.etns;
+    } else {
+      c.dew = -c.etp;
+      prcpf += c.dew;
+    }
+  }
   pcp_drp(c, prcpf, dt);
-  const double zz1 = 1.0;
-  const double yy = c.stc[0] - 0.5 * c.ssoil * c.zsoil[0] * zz1 / df1;
-  const double t11 = c.t1;
-  const double ssoil1 = c.ssoil;
+  double yy, zz1 = 1.0;
+  const double t11 = c.t1, ssoil1 = c.ssoil;
+  if (snow) {
+    yy = c.stc[0] - 0.5 * c.ssoil * c.zsoil[0] * zz1 / df1;
+  } else {
+    if (c.etp <= 0.0) {
+      c.beta_ = 0.0;
+      c.eta = c.etp;
+      if (c.etp < 0.0) c.beta_ = 1.0;
+    } else {
+      c.beta_ = c.eta / c.etp;
+    }
+    // NoPac's conductivity is the one SFlx has for bare ground
+    const double yynum = c.fdown - c.emissi * SIGMA * t24;
+    yy = c.sfctmp + (yynum / c.rch + c.th2 - c.sfctmp - c.beta_ * c.epsca) / c.rr;
+    zz1 = df1 / (-0.5 * c.zsoil[0] * c.rch * c.rr) + 1.0;
+  }
   sh_flx(c, u, dt, yy, zz1, df1);
+  if (!snow) {
+    c.flx1 = CPH2O * c.prcp * 1000.0 * (c.t1 - c.sfctmp);
+    c.flx3 = 0.0;
+    return;
+  }
   c.t1 = t11;
   c.ssoil = ssoil1;
   if (c.sneqv > 0.0) {
@@ -804,7 +869,7 @@ __device__ __forceinline__ void s_flx(Col &c, const NoahUni &u, double dt) {
     c.sncovr = (c.sncovr < 0.98) ? c.sncovr : 0.98;
     al_calc(c, u, dt, snowng);
   }
-  double df1 = tdf_cnd(c.smc[0], c.quartz, c.smcmax, c.smcmin, c.sh2o[0]);
+  double df1 = tdf_cnd(c.smc[0], c.lks, c.smcmax, c.smcmin, c.sh2o[0]);
   df1 *= exp(u.sbeta * shdfac);
   if (c.sncovr > 0.97) df1 = c.sncond;
   const double dsoil = -(0.5 * c.zsoil[0]);
@@ -827,14 +892,9 @@ __device__ __forceinline__ void s_flx(Col &c, const NoahUni &u, double dt) {
   penman(c, t24, t2v, snowng, frzgra);
   if (shdfac > 0.0) can_res(c);
   else c.rc = 0.0;
-  c.esnow = 0.0;
-  if (c.sneqv == 0.0) {
-    no_pac(c, u, dt, t24);
-    c.eta_kinematic = c.eta * 1000.0;
-  } else {
-    sno_pac(c, u, snowng, dt, t24, prcpf, df1);
-    c.eta_kinematic = (c.esnow + c.etns) * 1000.0;
-  }
+  const bool snow = !(c.sneqv == 0.0);
+  pac(c, u, snow, snowng, dt, t24, prcpf, df1);
+  c.eta_kinematic = snow ? (c.esnow + c.etns) * 1000.0 : c.eta * 1000.0;
   c.q1 = c.q2 + c.eta_kinematic * NCP / c.rch;
   c.sheat = -(c.ch * NCP * c.sfcprs) / (RD * t2v) * (c.th2 - c.t1);
   c.ef_edir = c.edir * 1000.0 * LVH2O;
@@ -859,24 +919,33 @@ __global__ __launch_bounds__(kBlock) void k_noah_meteo(int nstation, int nrec, c
 // Noah(): src/noah/noah.c:3-55, one element per thread.
 //
 // What bounds it: one column's chain of dependent FP64 work (the whole step is
-// one wavefront's latency up to some 20,000 columns), and at 100,000 columns
-// the chain times the few wavefronts a SIMD holds.  So the functions are
-// inlined, which lets the column's record live in registers (256, two
-// wavefronts per SIMD) with only the layer arrays and the largest branches'
-// overflow in scratch memory, and a workgroup is one wavefront, which spreads
-// 20,000 columns over every CU.  Measured (us per step, 6,000 / 20,011 /
-// 100,000 columns): 122 / 139 / 233 with calls and the record in scratch;
-// inlined 74.9 / 85.3 / 181.8 at one wavefront per SIMD, 80.9 / 101.1 / 170.8
-// at two, 94.8 / 124.7 / 208.1 at three; two and the heat solve in place
-// 77.9 / 92.8 / 147.7.
-constexpr int kNoahBlock = 64;
-__global__ __launch_bounds__(kNoahBlock, 2) void k_noah(int ne, int nstation, NoahDev d, NoahUni u, ColDev s, double dt) {
+// one wavefront's latency up to some 60,000 columns), and at 100,000 columns
+// two such chains one after the other, since the layers' 39 KB of LDS leave a
+// SIMD one wavefront.  So:
+// - every function is inlined and the column's record lives in registers (242,
+//   nothing in scratch memory); the layer arrays, indexed at run time, are in
+//   LDS, where they cost neither registers nor scratch;
+// - the branches that columns of one wavefront take differently (snow or none,
+//   the top layer or one below) hold only what differs;
+// - the powers, and the logarithms of the exchange coefficients' fixed point,
+//   of the supercooled water's Newton iteration and of the layers'
+//   conductivities, are the shorter ones of xmath.hpp, and fewer.
+// Measured (us per step, 6,000 / 20,011 / 100,000 columns): 122 / 139 / 233
+// with calls and the record in scratch; 77.9 / 92.8 / 147.7 inlined (256
+// registers and 960 B of scratch); 53.3 / 60.5 / 125.5 with the shared branches
+// and the shorter functions at 474 registers, 66.2 / 87.2 / 139.7 at 256;
+// 41.9 / 47.9 / 92.5 with the layers in LDS.  Against the step in 80-bit
+// arithmetic on 100,000 columns its errors are the former kernel's to a few
+// per cent (exchange coefficient: 7.5e-16 in the mean, before and now).
+__global__ __launch_bounds__(kNoahBlock, 1) void k_noah(int ne, int nstation, NoahDev d, NoahUni u, ColDev s, double dt) {
   const int p = blockIdx.x * kNoahBlock + threadIdx.x;
   if (p >= ne) return;
   auto at = [ne, p](double *f, int k) -> double & { return f[(long)k * ne + p]; };
-  double zsoil[ML], rtdis[ML], smc[ML], sh2o[ML], stc[ML], et[ML];
+  __shared__ double lay[NLAYARR][ML][kNoahBlock];
   Col c;
-  c.zsoil = zsoil; c.rtdis = rtdis; c.smc = smc; c.sh2o = sh2o; c.stc = stc; c.et = et;
+  Layers *const arr[] = {&c.zsoil, &c.smc, &c.sh2o, &c.stc, &c.et, &c.w1, &c.w2};
+#pragma unroll
+  for (int k = 0; k < NLAYARR; k++) arr[k]->p = &lay[k][0][threadIdx.x];
   c.nsoil = s.nsoil[p];
   c.nroot = d.nroot[p];
   for (int k = 0; k < ML; k++) {
@@ -885,12 +954,11 @@ __global__ __launch_bounds__(kNoahBlock, 2) void k_noah(int ne, int nstation, No
     c.stc[k] = 0.0;
     c.et[k] = 0.0;
     c.zsoil[k] = 0.0;
-    c.rtdis[k] = 0.0;
   }
   // DefSldpth's depths and RootDist (src/noah/lsm_func.c:86-205)
   c.zsoil[0] = -at(s.sldpth, 0);
   for (int k = 1; k < c.nsoil; k++) c.zsoil[k] = -at(s.sldpth, k) + c.zsoil[k - 1];
-  for (int j = 0; j < c.nroot; j++) c.rtdis[j] = -at(s.sldpth, j) / c.zsoil[c.nroot - 1];
+  for (int j = 0; j < c.nroot; j++) c.w2[j] = -at(s.sldpth, j) / c.zsoil[c.nroot - 1];
   for (int k = 0; k < c.nsoil; k++) {
     c.smc[k] = at(s.smc, k);
     c.sh2o[k] = at(s.sh2o, k);
@@ -901,7 +969,7 @@ __global__ __launch_bounds__(kNoahBlock, 2) void k_noah(int ne, int nstation, No
   c.albedomax = d.albedomax[p]; c.z0min = d.z0min[p]; c.z0max = d.z0max[p]; c.snup = d.snup[p];
   c.cfactr = d.cfactr[p]; c.rgl = d.rgl[p]; c.rsmin = d.rsmin[p]; c.rsmax = d.rsmax[p]; c.topt = d.topt[p];
   c.hs = d.hs[p]; c.smcref = d.smcref[p]; c.smcwlt = d.smcwlt[p]; c.smcdry = d.smcdry[p];
-  c.quartz = d.quartz[p]; c.zlvl_wind = d.zlvl_wind[p];
+  c.lks = ln_solids(d.quartz[p]); c.zlvl_wind = d.zlvl_wind[p];
   c.smcmax = s.smcmax[p]; c.smcmin = s.smcmin[p]; c.alpha = s.alpha[p]; c.beta = s.beta[p];
   c.t1 = at(d.sc, 0); c.sneqv = at(d.sc, 1); c.snowh = at(d.sc, 2); c.sndens = at(d.sc, 3);
   c.cmc = at(d.sc, 4); c.ch = at(d.sc, 5); c.cm = at(d.sc, 6); c.snotime1 = at(d.sc, 7);
