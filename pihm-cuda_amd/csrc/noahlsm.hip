@@ -167,7 +167,7 @@ __device__ __forceinline__ void al_calc(Col &c, const NoahUni &u, double dt, int
   c.albedo = (c.albedo > snoalb2) ? snoalb2 : c.albedo;
 }
 
-// ln x for any x: xmath's logarithm, a third of the library's instructions.
+// ln x for any x, xmath's logarithm on its main path.
 __device__ __forceinline__ double ln_of(double x) {
   if (x > 0.0 && x < HUGE_VAL) {
     double lo;
