@@ -105,12 +105,15 @@ struct Round {
 // per-member totals of its reductions (a second launch, one workgroup per
 // member with a reduction).
 // after_ops, when not null, is recorded between the operation kernel and the
-// reduction kernel (timing of the operation kernel alone).
-void launch_ops(const Dev &d, const Round &r, hipStream_t st, hipEvent_t after_ops = nullptr);
+// reduction kernel (timing of the operation kernel alone).  With sig and flag
+// the reduction kernel also ends the tick (launch_signal's work); returns
+// whether it does, which takes a round with reductions.
+bool launch_ops(const Dev &d, const Round &r, hipStream_t st, hipEvent_t after_ops = nullptr, unsigned *sig = nullptr,
+                unsigned *flag = nullptr);
 constexpr int kTuneNG = 4;
 constexpr int kTuneG[kTuneNG] = {1, 2, 4, 8};
-// One-lane kernel writing ++(*ctr) to *flag (host memory) after the work queued before it.
-void launch_signal(unsigned *ctr, volatile unsigned *flag, hipStream_t st);
+// One-lane kernel writing ++sig[0] to *flag (host memory) after the work queued before it.
+void launch_signal(unsigned *sig, unsigned *flag, hipStream_t st);
 
 }  // namespace ens
 }  // namespace pihm

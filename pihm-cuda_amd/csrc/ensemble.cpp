@@ -717,12 +717,16 @@ struct pihm_ensemble {
   std::vector<Task<int>> tops; // running model-step loops
   long ticks = 0, op_launches = 0, rhs_launches = 0;
   // the operation kernel's launches timed with HIP events (the first kEvPairs
-  // of each tick) and their algorithmic bytes
-  static constexpr int kEvPairs = 8;
+  // of the first tick of a run and of every kEvTicks-th after it) and their
+  // algorithmic bytes.  A pair of events costs a tick some 8 us (24 members,
+  // two launches a tick: 29.0 ms a run with every tick timed, 24.8 with one in
+  // 32), so most ticks go without.
+  static constexpr int kEvPairs = 8, kEvTicks = 16;
+  long next_timed = 0;
   hipEvent_t ev_ops[2 * kEvPairs] = {};
   long ops_timed = 0;
   double ops_bytes = 0.0, ops_ms = 0.0;
-  unsigned *sig_ctr = nullptr;           // device tick count
+  unsigned *sig_ctr = nullptr;           // device: ticks so far, workgroups done (k_ens_final)
   volatile unsigned *sig_flag = nullptr; // pinned host copy
   unsigned sig_expect = 0;
   int ops_g = 1;               // chunks per workgroup of k_ens_ops (pihm_ens_autotune)
@@ -894,6 +898,8 @@ int pihm_ensemble::flush() {
   std::memcpy(stage_h, buf.data(), buf.size());
   PIHM_HIP_TRY(hipMemcpyAsync(stage_d, stage_h, buf.size(), hipMemcpyHostToDevice, st));
   int ntimed = 0;
+  const bool time_tick = ticks >= next_timed;
+  bool signalled = false;
   double timed_bytes[kEvPairs];
   for (const auto &r : plans) {
     if (r.rhs) {
@@ -914,17 +920,19 @@ int pihm_ensemble::flush() {
       rd.nred = r.nred;
       rd.nchunks = r.nblocks;
       rd.g = ops_g;
-      const bool timed = ntimed < kEvPairs && ev_ops[2 * ntimed];
+      const bool timed = time_tick && ntimed < kEvPairs && ev_ops[2 * ntimed];
       if (timed) PIHM_HIP_TRY(hipEventRecord(ev_ops[2 * ntimed], st));
-      launch_ops(dev, rd, st, timed ? ev_ops[2 * ntimed + 1] : nullptr);
+      const bool last = &r == &plans.back();
+      signalled = launch_ops(dev, rd, st, timed ? ev_ops[2 * ntimed + 1] : nullptr, last ? sig_ctr : nullptr,
+                             (unsigned *)sig_flag);
       PIHM_HIP_TRY(hipGetLastError());
       if (timed) timed_bytes[ntimed++] = r.bytes;
       op_launches++;
     }
   }
-  // wait for the tick: spin on the count the signal kernel writes to host
+  // wait for the tick: spin on the count that its last launch writes to host
   // memory, handing over to the runtime's wait after 2 ms
-  launch_signal(sig_ctr, sig_flag, st);
+  if (!signalled) launch_signal(sig_ctr, (unsigned *)sig_flag, st);
   PIHM_HIP_TRY(hipGetLastError());
   const unsigned want = ++sig_expect;
   const auto t0 = std::chrono::steady_clock::now();
@@ -945,6 +953,7 @@ int pihm_ensemble::flush() {
       ops_timed++;
     }
   }
+  if (ntimed > 0) next_timed = ticks + kEvTicks;
   ticks++;
   return PIHM_OK;
 }
@@ -1055,10 +1064,10 @@ int ens_alloc(pihm_ctx *c, const int *nrec_cap, const int *nst_cap, const pihm_r
     return fail(PIHM_ERR_HIP);
   std::memset(e->result, 0, (size_t)nmem * kRes * sizeof(double));
   if (hipHostMalloc((void **)&e->mnan, nmem * sizeof(int), hipHostMallocCoherent) != hipSuccess) return fail(PIHM_ERR_HIP);
-  if (hipMalloc((void **)&e->sig_ctr, sizeof(unsigned)) != hipSuccess) return fail(PIHM_ERR_HIP);
+  if (hipMalloc((void **)&e->sig_ctr, 2 * sizeof(unsigned)) != hipSuccess) return fail(PIHM_ERR_HIP);
   for (auto &ev : e->ev_ops)
     if (hipEventCreate(&ev) != hipSuccess) return fail(PIHM_ERR_HIP);
-  if (hipMemset(e->sig_ctr, 0, sizeof(unsigned)) != hipSuccess) return fail(PIHM_ERR_HIP);
+  if (hipMemset(e->sig_ctr, 0, 2 * sizeof(unsigned)) != hipSuccess) return fail(PIHM_ERR_HIP);
   {
     unsigned *f = nullptr;
     if (hipHostMalloc((void **)&f, sizeof(unsigned), hipHostMallocCoherent) != hipSuccess) return fail(PIHM_ERR_HIP);
@@ -1155,6 +1164,7 @@ void ens_start(pihm_ensemble *e, int k, long ke) {
 // Returns the number of members that finished or failed, or an error < 0.
 static int ens_advance(pihm_ensemble *e, long max_ticks, bool stop_on_finish, int *nfailed) {
   int nfin = 0, nfail = 0;
+  e->next_timed = e->ticks;
   for (long t = 0; t < max_ticks; t++) {
     bool any = false;
     for (int k = 0; k < e->nmem; k++) {

@@ -73,7 +73,8 @@ __device__ __forceinline__ Ix ix_of(const RhsArgs &a, int member) {
 template <bool B>
 __device__ __forceinline__ void flag_nan(const RhsArgs &a, const Ix &ix) {
   *a.nanflag = 1;
-  if (B && a.mnan) a.mnan[ix.m] = 1;
+  // host memory, read when the tick's last launch says so
+  if (B && a.mnan) __hip_atomic_store(&a.mnan[ix.m], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 template <bool B>
 __device__ __forceinline__ Ix ix_elem(const RhsArgs &a, int p) { return ix_of<B>(a, B ? a.emem[p] : 0); }
