@@ -89,7 +89,9 @@ void pihm_gpu_backend_destroy(pihm_gpu_backend *b);
 int  pihm_gpu_backend_get(pihm_gpu_backend *b, pihm_backend *out);
 
 /* One call: device vector, backend and driver for a whole run.
- * y_inout is the state in caller order. */
+ * y_inout is the state in caller order.  The context keeps the run's device
+ * vectors (22 of the state's length) for its next run and frees them with
+ * itself, here and in the other pihm_run_gpu_* calls. */
 int pihm_run_gpu(pihm_ctx *ctx, const pihm_forcing *forc, const pihm_run_config *cfg,
                  double *y_inout, pihm_run_stats *stats);
 
