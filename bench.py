@@ -328,7 +328,7 @@ def _producers(mesh, seed):
 def producers_run(mesh, seed, iters=200):
     """The per-step producers on the device at the 200,000-triangle workload, timed with
     HIP events: one land-surface step (k_meteo + k_intcp_snow_et) and one boundary-series
-    apply (k_bc_interp + k_bc_scatter)."""
+    apply (k_bc)."""
     L = _lib.lib()
     h, lsm, bc, bc_bytes = _producers(mesh, seed)
     ms_l, ms_b = C.c_double(), C.c_double()
