@@ -1596,8 +1596,9 @@ int ctx_load(pihm_ctx *c, int k, const pihm_mesh_desc *m) {
                   E.alpha, E.beta, E.porosity, E.dmac, E.kmac, E.kmacv,
                   E.areafh, E.rough, E.rzd};
   for (int f = 0; f < 17; f++) {
-    if (es[f] == m->kmach) {
-      // EffKh's conductivity with macropores (src/lat_flow.c:258), static
+    if (ed[f] == E.kmac) {
+      // EffKh's conductivity with macropores (src/lat_flow.c:258), static; known
+      // by where it goes: the caller's arrays may be one and the same
       for (int lp = 0; lp < n; lp++) {
         const int i = order[lp];
         hd[lp] = m->kmach[i] * m->areafv[i] + m->ksath[i] * (1.0 - m->areafv[i]);
