@@ -10,10 +10,12 @@
  * definitions are used and the ones below are skipped.
  *
  * Data lives in device memory (HBM).  Reductions (dot product, norms, min)
- * are deterministic: a fixed-shape two-pass tree (wavefront shuffles inside a
- * block, then one block over the block partials in index order), so the same
- * input gives the same bits on every call and for every launch timing.  They
- * return a host double, which implies a stream synchronisation.
+ * are deterministic: a fixed-shape two-pass tree (inside a block, then one
+ * block over the block partials in index order), so the same input gives the
+ * same bits on every call and for every launch timing.  They return a host
+ * double and wait for it: when one returns, everything queued on the vector's
+ * stream before it is done, and so is the vector that N_VInvTest_Hip and
+ * N_VConstrMask_Hip store.
  */
 #ifndef PIHM_NVECTOR_H
 #define PIHM_NVECTOR_H

@@ -400,9 +400,16 @@ bool reduce_wait(N_Vector v, const RedArgs &a, double *out) {
   for (int k = 0; k < a.nvec; k++) out[k] = a.work.result[k];
   return true;
 }
+// The two tests also store a vector, which has to be written when they return:
+// their second pass stays a launch of its own at every length.  The last
+// workgroup of a single launch would announce the sum while other wavefronts'
+// stores are on their way, and caches are written back when a kernel ends.
+constexpr bool red_stores(int kind) { return kind == R_INVTEST || kind == R_CONSTR; }
+
 template <int KIND>
 bool reduce(N_Vector v, RedArgs &a, double *out) {
   a.work = X(v)->w;
+  if constexpr (red_stores(KIND)) a.work.ticket = nullptr;
   launch_reduce<KIND>(a, red_blocks(a.n), S(v));
   return reduce_wait(v, a, out);
 }
