@@ -419,7 +419,13 @@ __device__ __forceinline__ LatOut elem_lateral(const RhsArgs &a, int p, const Ix
     den[j] = sqrt_pos(avg_sf) * (0.5 * (me.rough + nr.rough));
     ovl[j] = 0.0;
   }
-  if (hs[0] > 0.0 || hs[1] > 0.0 || hs[2] > 0.0) {
+  // a dry face's flux is zero, unless 0 times its edge and gradient over its
+  // roughness is no number, which the reference reports; the three in one test
+  // each (an overflow or underflow here only takes the long way)
+  const bool sound = den[0] * den[1] * den[2] > 0.0 &&
+                     fabs(in.edge[0] * gh[0] + in.edge[1] * gh[1] + in.edge[2] * gh[2]) < HUGE_VAL;
+  const bool flow = hs[0] > 0.0 || hs[1] > 0.0 || hs[2] > 0.0 || !sound;
+  if (flow) {
     // OverLandFlow: src/lat_flow.c:279-283 (literal exponent 0.6666667)
     const double ex[3] = {0.6666667, 0.6666667, 0.6666667};
     double pw[3];
