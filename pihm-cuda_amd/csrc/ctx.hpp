@@ -149,7 +149,7 @@ namespace pihm {
 // What pihm_ctx_poll_nan's kernel hands to the host.
 struct NanReport {
   int flag;
-  volatile unsigned count;
+  volatile unsigned seq;         // the number of the report
 };
 // Capacity of one slot of a context: the largest mesh it can hold.
 struct SlotCap {
@@ -212,9 +212,9 @@ struct pihm_ctx {
   pihm::RhsArgs args;            // pointers filled at creation
   void *arena;                   // one device allocation for everything
   size_t arena_bytes;
-  int *nanflag_dev;              // the flag, then the count of its reports
+  int *nanflag_dev;
   pihm::NanReport *nan_host;     // pinned (coherent)
-  unsigned nan_expect;           // reports awaited so far
+  unsigned nan_seq;              // the last report asked for
   double *stage_host;            // scratch for host-side permutations
   int noah;                      // RHS with the reference's _NOAH_ branches
   void *noah_arena;              // the Noah fields of ElemDev

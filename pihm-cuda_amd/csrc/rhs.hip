@@ -1401,7 +1401,7 @@ int ctx_alloc(const std::vector<SlotCap> &caps, int surf_mode, int riv_mode, pih
   c->stream = nullptr; c->nan_check = 1; c->record = 0; c->ncalls = 0;
   c->arena = nullptr;
   c->nan_host = nullptr;
-  c->nan_expect = 0;
+  c->nan_seq = 0;
   c->rhs_path = PIHM_RHS_TWO_KERNELS;
   c->one_launch_ok = 0;
   c->tiles = TileArgs{};
@@ -1446,7 +1446,7 @@ int ctx_alloc(const std::vector<SlotCap> &caps, int surf_mode, int riv_mode, pih
   ar.add(&A.rec.sub, 3L * ne);
   ar.add(&A.rec.infil, ne);
   ar.add(&A.rec.rechg, ne);
-  ar.add(&c->nanflag_dev, 2);   // the flag and the count of its reports
+  ar.add(&c->nanflag_dev, 1);
   ar.add(&c->mem_dev, nmem);
   int32_t *emem_dev = nullptr, *rmem_dev = nullptr;
   ar.add(&emem_dev, ne);
@@ -1460,7 +1460,7 @@ int ctx_alloc(const std::vector<SlotCap> &caps, int surf_mode, int riv_mode, pih
   if (rc) { pihm_ctx_destroy(c); return rc; }
   ar.carve((char *)c->arena);
   c->nan_host->flag = 0;
-  c->nan_host->count = 0;
+  c->nan_host->seq = 0;
   // empty slots: empty upstream lists, boundary codes
   std::vector<int32_t> rm(nr1, 0), ub(nr1, 0);
   for (int k = 0; k < nmem; k++)
@@ -2217,41 +2217,41 @@ int pihm_rhs_launch_compact(pihm_ctx *c, const MemberIO *mio, int *mnan, const i
   return PIHM_OK;
 }
 
-// Hands the NaN flag to the host and clears it: the flag, then the running
-// count of reports, to coherent host memory.
-__global__ void k_nan_report(int *flag, unsigned *ctr, int *host_flag, volatile unsigned *host_count) {
+// Hands the NaN flag to the host and clears it: the flag, then the number of
+// the report, to coherent host memory.
+__global__ void k_nan_report(int *flag, int *host_flag, volatile unsigned *host_seq, unsigned seq) {
   if (threadIdx.x != 0) return;
   const int v = *flag;
-  const unsigned n = *ctr + 1u;
-  *ctr = n;
   if (v) *flag = 0;
   __hip_atomic_store(host_flag, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the flag has reached the host before its count
-  *host_count = n;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the flag has reached the host before its number
+  *host_seq = seq;
 }
 
 // Reads and clears the sticky NaN flag; everything queued on the stream before
-// the call is done when it returns.  The host spins on the report's count and
+// the call is done when it returns.  The host spins on the report's number and
 // after 2 ms falls back to the runtime's wait, which also reports errors: 19.9 us
 // for an evaluation of 535 triangles with its check, 24.9 with a copy of the
-// flag and the runtime's wait.
+// flag and the runtime's wait.  Every report has a number of its own, given by
+// the host whether or not the launch succeeds, so none is taken for another;
+// an error that an earlier call left with the thread is not this launch's.
 extern "C" int pihm_ctx_poll_nan(pihm_ctx *c) {
   if (!c) return PIHM_ERR_ARG;
   NanReport *h = c->nan_host;
-  hipLaunchKernelGGL(k_nan_report, dim3(1), dim3(64), 0, c->stream, c->nanflag_dev, (unsigned *)(c->nanflag_dev + 1),
-                     &h->flag, &h->count);
-  PIHM_HIP_TRY(hipGetLastError());
-  const unsigned want = c->nan_expect + 1u;
+  unsigned want = ++c->nan_seq;
+  int *flag = c->nanflag_dev, *host_flag = &h->flag;
+  volatile unsigned *host_seq = &h->seq;
+  void *args[] = {&flag, &host_flag, &host_seq, &want};
+  PIHM_HIP_TRY(hipLaunchKernel((const void *)k_nan_report, dim3(1), dim3(64), args, 0, c->stream));
   const auto t0 = std::chrono::steady_clock::now();
-  for (unsigned it = 1; h->count != want; it++) {
+  for (unsigned it = 1; h->seq != want; it++) {
     if ((it & 255u) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
       PIHM_HIP_TRY(hipStreamSynchronize(c->stream));
-      if (h->count != want) return PIHM_ERR_HIP;
+      if (h->seq != want) return PIHM_ERR_HIP;
       break;
     }
     __builtin_ia32_pause();
   }
-  c->nan_expect = want;
   std::atomic_thread_fence(std::memory_order_acquire);
   return h->flag ? PIHM_ERR_NAN : PIHM_OK;
 }
