@@ -1,8 +1,9 @@
 // bc.hip - boundary-condition time series applied on the device.
 //
-// One launch on the context's stream per apply: one thread per element edge and
-// river segment, which interpolates its series if it has one (IntrplForc,
-// src/forcing.c:482-530; ApplyElemBc, :127-177; ApplyRiverBc, :214-244).
+// One thread per element edge and river segment, which interpolates its series
+// if it has one (IntrplForc, src/forcing.c:482-530; ApplyElemBc, :127-177;
+// ApplyRiverBc, :214-244); where a great many have one, a launch of one thread
+// per series interpolates them first.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -27,9 +28,7 @@ struct BcSeries {
 // code > 0: series code-1 (head); code < 0: series -code-1 (flux); 0: unchanged.
 // Element edges first (edge-major, device order), then river segments.  The few
 // entries that have a series interpolate it themselves, beside the many that
-// only read their code: 4.9 us at 200,000 triangles, bound by the codes and one
-// bisection's loads, where a launch that interpolated each series and one that
-// scattered them took 4.7 + 4.8.
+// only read their code: bound by the codes and one bisection's loads.
 __global__ __launch_bounds__(kBlock) void k_bc(long n_edge, int nr, const int32_t *code_e, const int32_t *code_r,
                                                BcSeries se, BcSeries sr, double t, double *ebc, double *rbc) {
   const long i = (long)blockIdx.x * kBlock + threadIdx.x;
@@ -41,6 +40,39 @@ __global__ __launch_bounds__(kBlock) void k_bc(long n_edge, int nr, const int32_
   const long k = (c > 0 ? c : -c) - 1;
   ts_interp<1>(s.ft + k * s.nrec, s.v + k * s.nrec, s.nrec, t, edge ? ebc + i : rbc + (i - n_edge), 1);
 }
+
+// Above kBcDirect entries with a series, in two launches: every series' value
+// into a table, element series first, then the entries from the table (bound by
+// the codes and the values written, whatever the length of the series).
+__global__ __launch_bounds__(kBlock) void k_bc_interp(int nts_e, int nts_r, BcSeries se, BcSeries sr, double t,
+                                                      double *val) {
+  const int k = blockIdx.x * kBlock + threadIdx.x;
+  if (k >= nts_e + nts_r) return;
+  const BcSeries s = k < nts_e ? se : sr;
+  const long q = k < nts_e ? k : k - nts_e;
+  ts_interp<1>(s.ft + q * s.nrec, s.v + q * s.nrec, s.nrec, t, val + k, 1);
+}
+__global__ __launch_bounds__(kBlock) void k_bc_scatter(long n_edge, int nr, const int32_t *code_e,
+                                                       const int32_t *code_r, int nts_e, const double *val,
+                                                       double *ebc, double *rbc) {
+  const long i = (long)blockIdx.x * kBlock + threadIdx.x;
+  if (i >= n_edge + nr) return;
+  const bool edge = i < n_edge;
+  const int c = edge ? code_e[i] : code_r[i - n_edge];
+  if (c == 0) return;
+  const double v = val[(edge ? 0 : nts_e) + (c > 0 ? c : -c) - 1];
+  if (edge) ebc[i] = v;
+  else rbc[i - n_edge] = v;
+}
+
+// Entries with a series up to which they interpolate it themselves.  Measured
+// (us per apply, one launch / two; series of 1,000 and of 20,000 records):
+// the outer edges and the river segments of 200,000 triangles, 6,306 of 605,000
+// entries, 4.7 / 5.8 and 6.1 / 6.8; a tenth of the edges drawn at random, 6,487
+// of 60,533 entries 4.3 / 5.4 and 5.2 / 6.5, 19,462 of 181,500 5.0 / 5.7 and
+// 6.8 / 6.5, 32,630 of 302,500 6.3 / 5.8 and 8.7 / 6.7, 65,114 of 605,000
+// 10.9 / 6.6 and 15.6 / 7.5; all of 605,000 19.8 / 6.8 and 35.5 / 7.8.
+constexpr long kBcDirect = 16384;
 
 bool times_increase(const pihm_ts *s) {
   for (int k = 0; k < s->nts; k++)
@@ -57,7 +89,8 @@ struct pihm_bc {
   long n_edge;
   int nr;
   int32_t *code_e, *code_r;
-  double *ft_e, *v_e, *ft_r, *v_r;
+  double *ft_e, *v_e, *ft_r, *v_r, *val;
+  long ncoded;          // edges and segments with a series
   double t_lo, t_hi;    // the time range every series covers
   void *arena;
 };
@@ -100,6 +133,9 @@ int pihm_bc_create(pihm_ctx *ctx, const int32_t *elem_type, const pihm_ts *ets, 
   b->nts_r = nts_r;
   b->nrec_r = nts_r ? rts->nrec : 0;
   b->n_edge = 3L * ne;
+  b->ncoded = 0;
+  for (const int32_t c : ce) b->ncoded += c != 0;
+  for (const int32_t c : cr) b->ncoded += c != 0;
   b->nr = nr;
   b->t_lo = -HUGE_VAL;
   b->t_hi = HUGE_VAL;
@@ -111,7 +147,8 @@ int pihm_bc_create(pihm_ctx *ctx, const int32_t *elem_type, const pihm_ts *ets, 
       }
   auto al = [](size_t n) { return (n + 255) & ~size_t(255); };
   const size_t se = (size_t)b->nts_e * b->nrec_e * sizeof(double), sr = (size_t)b->nts_r * b->nrec_r * sizeof(double);
-  const size_t total = al(3L * ne * 4) + al(cr.size() * 4) + 2 * al(se) + 2 * al(sr);
+  const size_t total = al(3L * ne * 4) + al(cr.size() * 4) + 2 * al(se) + 2 * al(sr) +
+                       al((nts_e + nts_r + 1) * sizeof(double));
   if (hipMalloc(&b->arena, total) != hipSuccess) { delete b; return PIHM_ERR_HIP; }
   char *base = (char *)b->arena;
   b->code_e = (int32_t *)base; base += al(3L * ne * 4);
@@ -119,7 +156,8 @@ int pihm_bc_create(pihm_ctx *ctx, const int32_t *elem_type, const pihm_ts *ets, 
   b->ft_e = (double *)base; base += al(se);
   b->v_e = (double *)base; base += al(se);
   b->ft_r = (double *)base; base += al(sr);
-  b->v_r = (double *)base;
+  b->v_r = (double *)base; base += al(sr);
+  b->val = (double *)base;
   bool ok = hipMemcpy(b->code_e, ce.data(), 3L * ne * 4, hipMemcpyHostToDevice) == hipSuccess &&
             hipMemcpy(b->code_r, cr.data(), cr.size() * 4, hipMemcpyHostToDevice) == hipSuccess;
   if (ok && se)
@@ -142,9 +180,17 @@ void pihm_bc_destroy(pihm_bc *b) {
 static void launch_apply(pihm_bc *b, double t) {
   pihm_ctx *c = b->ctx;
   const long n = b->n_edge + b->nr;
-  hipLaunchKernelGGL(k_bc, dim3((unsigned)div_up(n, (long)kBlock)), dim3(kBlock), 0, c->stream, b->n_edge, b->nr,
-                     b->code_e, b->code_r, BcSeries{b->nrec_e, b->ft_e, b->v_e}, BcSeries{b->nrec_r, b->ft_r, b->v_r},
-                     t, c->args.e.ebc, c->args.r.bc);
+  const dim3 grid((unsigned)div_up(n, (long)kBlock));
+  const BcSeries se{b->nrec_e, b->ft_e, b->v_e}, sr{b->nrec_r, b->ft_r, b->v_r};
+  if (b->ncoded <= kBcDirect || std::isnan(t)) {   // no interval holds a NaN: the entries stay, the table may be empty
+    hipLaunchKernelGGL(k_bc, grid, dim3(kBlock), 0, c->stream, b->n_edge, b->nr, b->code_e, b->code_r, se, sr, t,
+                       c->args.e.ebc, c->args.r.bc);
+    return;
+  }
+  hipLaunchKernelGGL(k_bc_interp, dim3(div_up(b->nts_e + b->nts_r, kBlock)), dim3(kBlock), 0, c->stream, b->nts_e,
+                     b->nts_r, se, sr, t, b->val);
+  hipLaunchKernelGGL(k_bc_scatter, grid, dim3(kBlock), 0, c->stream, b->n_edge, b->nr, b->code_e, b->code_r, b->nts_e,
+                     b->val, c->args.e.ebc, c->args.r.bc);
 }
 
 int pihm_bc_apply(pihm_bc *b, double t) {
