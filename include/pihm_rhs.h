@@ -266,6 +266,9 @@ int  pihm_ctx_get_fluxes(pihm_ctx *ctx, double *ovlflow, double *subsurf,
  * src/river_flow.c:520-583); it lets tests bound the device results against
  * the host libm and check that host and device return the same bits. */
 int  pihm_math_pow(int n, const double *x, const double *y, double *out, int on_device);
+/* The same for the land surface's power, which keeps the accuracy of a C
+ * library's pow (a little over half an ulp), and with y NULL for its logarithm. */
+int  pihm_math_fine(int n, const double *x, const double *y, double *out, int on_device);
 
 #ifdef __cplusplus
 }

@@ -8,9 +8,9 @@
 // elements together; the temperatures stc are stored the same way.  The
 // thread works on its column in LDS.  The step ends by
 // handing the RHS what it reads (pcpdrp, edir, ett, the layer transpiration,
-// sh2o[0]) and by refreshing GwTransp's share.  Powers, and the logarithms of
-// the three loops that take most of the step, are xmath.hpp's; the rest are the
-// device library's.
+// sh2o[0]) and by refreshing GwTransp's share.  Powers and logarithms are
+// xmath.hpp's fine ones, as accurate as the device library's; exp and atan are
+// the device library's.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -78,18 +78,13 @@ struct Layers {
   __device__ double &operator[](int k) const { return p[k * kNoahBlock]; }
 };
 
-// ln of a positive number as a sum.
-struct LnPair {
-  double hi, lo;
-};
-
 // One element's working record: the reference's ps/ws/wf/es/ef fields the step
 // touches.  The layers are in LDS: an array inside the record, indexed at run
 // time, would keep the whole record in scratch memory.
 struct Col {
   int nsoil, nroot;
   Layers zsoil, smc, sh2o, stc, et, w1, w2;   // w1, w2: Transp's weights, then ShFlx's coefficients
-  LnPair lks;                                      // ln of the solids' conductivity
+  double ksolid;                                      // the solids' factor of the saturated conductivity
   // parameters
   double shdfac, cmcfactr, laimin, laimax, emissmin, emissmax, albedomin, albedomax, z0min, z0max, snup, cfactr;
   double rgl, rsmin, rsmax, topt, hs, smcmax, smcmin, smcref, smcwlt, smcdry, alpha, beta, zlvl_wind;
@@ -122,7 +117,7 @@ __device__ __forceinline__ void cal_hum(Col &c, const NoahUni &u) {
 // CSnow: src/noah/noah.c:811-839
 __device__ __forceinline__ double c_snow(double dsnow) {
   const double UNIT = 0.11631;
-  const double cc = 0.328 * xpow(10.0, 2.25 * dsnow);
+  const double cc = 0.328 * pow_fine(10.0, 2.25 * dsnow);
   return 2.0 * UNIT * cc;
 }
 
@@ -131,7 +126,7 @@ __device__ __forceinline__ void snow_new(Col &c, double newsn) {
   double snowhc = c.snowh * 100.0;
   const double newsnc = newsn * 100.0;
   const double tempc = c.sfctmp - 273.15;
-  const double dsnew = (tempc <= -15.0) ? 0.05 : 0.05 + 0.0017 * xpow(tempc + 15.0, 1.5);
+  const double dsnew = (tempc <= -15.0) ? 0.05 : 0.05 + 0.0017 * pow_fine(tempc + 15.0, 1.5);
   const double hnewc = newsnc / dsnew;
   if (snowhc + hnewc < 0.001) c.sndens = (dsnew > c.sndens) ? dsnew : c.sndens;
   else c.sndens = (snowhc * c.sndens + hnewc * dsnew) / (snowhc + hnewc);
@@ -160,73 +155,58 @@ __device__ __forceinline__ void al_calc(Col &c, const NoahUni &u, double dt, int
     c.snotime1 = 0.0;
   } else {
     c.snotime1 += dt;
-    snoalb2 = snoalb1 * xpow(SNACCA, xpow(c.snotime1 / 86400.0, SNACCB));
+    snoalb2 = snoalb1 * pow_fine(SNACCA, pow_fine(c.snotime1 / 86400.0, SNACCB));
   }
   snoalb2 = (snoalb2 > c.alb) ? snoalb2 : c.alb;
   c.albedo = c.alb + c.sncovr * (snoalb2 - c.alb);
   c.albedo = (c.albedo > snoalb2) ? snoalb2 : c.albedo;
 }
 
-// ln x for any x, xmath's logarithm on its main path.
-__device__ __forceinline__ double ln_of(double x) {
-  if (x > 0.0 && x < HUGE_VAL) {
-    double lo;
-    return ln_pos(x, &lo);
-  }
-  return (x == 0.0) ? -HUGE_VAL : ((x < 0.0) ? NAN : x);
-}
-// Two of them in step.
+// Two logarithms in step.
 __device__ __forceinline__ void ln_of2(double a, double b, double *la, double *lb) {
   if (a > 0.0 && a < HUGE_VAL && b > 0.0 && b < HUGE_VAL) {
     const double x[2] = {a, b};
     double hi[2], lo[2];
-    ln_pos_n<2>(x, hi, lo);
+    ln_fine_n<2>(x, hi, lo);
     *la = hi[0];
     *lb = hi[1];
   } else {
-    *la = ln_of(a);
-    *lb = ln_of(b);
+    *la = ln_fine(a);
+    *lb = ln_fine(b);
   }
 }
 
-// a b + the pair (s, e), as a pair that carries the product's and the sum's
-// rounding.
-__device__ __forceinline__ void add_prod(double a, double b, double &s, double &e) {
-  const double p = a * b, t = s + p, z = t - s;
-  e += fma(a, b, -p) + ((s - (t - z)) + (p - z));
-  s = t;
+// log10 x of a positive number, as ln x / ln 10.
+__device__ __forceinline__ double log10_of(double x) {
+  const double M = 0.43429448190325182, M_LO = 1.0983196502167651e-17;   // 1 / ln 10
+  if (!(x < HUGE_VAL)) return x;
+  const double xs[1] = {x};
+  double h[1], l[1];
+  ln_fine_n<1>(xs, h, l);
+  const double p = h[0] * M;
+  return p + (fma(h[0], M, -p) + (h[0] * M_LO + l[0] * M));
 }
 
-// TDfCnd: src/noah/noah.c:2520-2619.  The solids' conductivity is quartz's
-// power times the other minerals', 7.7^q 2^(1-q), and the saturated one a
-// product of three powers: one exponential of the sum of their logarithms, the
-// sum carried as a pair.  lks is the solids' logarithm, one value per column.
-__device__ __forceinline__ LnPair ln_solids(double qz) {
-  const double LNQTZ = 2.0412203288596382, LNQTZ_LO = -3.402197230721298e-17;   // ln 7.7
-  const double LNO = 0.6931471805599453, LNO_LO = 2.3190468138462996e-17;       // ln 2
-  const double r = 1.0 - qz;
-  LnPair l{0.0, qz * LNQTZ_LO + r * LNO_LO};
-  add_prod(qz, LNQTZ, l.hi, l.lo);
-  add_prod(r, LNO, l.hi, l.lo);
-  return l;
+// TDfCnd: src/noah/noah.c:2520-2619.  The saturated conductivity is a product of
+// three powers.  The solids' is the same in every layer of a column; the ice's
+// and the water's have constant bases, whose logarithms are constants.
+__device__ __forceinline__ double solids_power(double qz, double smcmax) {
+  return pow_fine(pow_fine(7.7, qz) * pow_fine(2.0, 1.0 - qz), 1.0 - smcmax);
 }
-__device__ __forceinline__ double tdf_cnd(double smc, const LnPair &lks, double smcmax, double smcmin, double sh2o) {
+__device__ __forceinline__ double tdf_cnd(double smc, double ksolid, double smcmax, double smcmin, double sh2o) {
   const double LNICE = 0.7884573603642703, LNICE_LO = -2.639344289064807e-17;   // ln 2.2
   const double LNW = -0.5621189181535413, LNW_LO = 1.1409357209435452e-17;      // ln 0.57
   const double satratio = (smc - smcmin) / (smcmax - smcmin);
   const double xunfroz = sh2o / smc;
   const double xu = xunfroz * smcmax;
-  const double a = 1.0 - smcmax, b = smcmax - xu;
-  double hi = 0.0, lo = a * lks.lo + b * LNICE_LO + xu * LNW_LO;
-  add_prod(a, lks.hi, hi, lo);
-  add_prod(b, LNICE, hi, lo);
-  add_prod(xu, LNW, hi, lo);
-  const double thksat = exp_pair(hi, lo);
+  double il, wl;
+  const double ih = mul_pair(smcmax - xu, LNICE, LNICE_LO, &il), wh = mul_pair(xu, LNW, LNW_LO, &wl);
+  const double thksat = ksolid * exp_fine(ih, il) * exp_fine(wh, wl);
   const double gammd = (1.0 - smcmax) * 2700.0;
   const double thkdry = (0.135 * gammd + 64.7) / (2700.0 - 0.947 * gammd);
   double ake;
   if ((sh2o + 0.0005) < smc) ake = satratio;
-  else if (satratio > 0.1) ake = ln_of(satratio) * 0.43429448190325183 + 1.0;   // log10
+  else if (satratio > 0.1) ake = log10_of(satratio) + 1.0;
   else ake = 0.0;
   return ake * (thksat - thkdry) + thkdry;
 }
@@ -265,7 +245,7 @@ __device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, doubl
   du2 = (du2 > EPSU2) ? du2 : EPSU2;
   const double btgh = btg * HPBL;
   auto wstar2_of = [&](double chv) {
-    return (btgh * chv * dthv != 0.0) ? wwst2 * xpow(fabs(btgh * chv * dthv), 2.0 / 3.0) : 0.0;
+    return (btgh * chv * dthv != 0.0) ? wwst2 * pow_fine(fabs(btgh * chv * dthv), 2.0 / 3.0) : 0.0;
   };
   auto ustar_of = [&](double cmv, double w) {
     const double us = sqrt_pos(cmv * sqrt_pos(du2 + w));
@@ -278,7 +258,7 @@ __device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, doubl
   double zslt = zlvl + zt;
   const double ratu = zslu / zu;
   double ratt = fdiv(zslt, zt);
-  double rlmo = fdiv(elfc * ch * dthv, xpow(ustar, 3.0));
+  double rlmo = fdiv(elfc * ch * dthv, cube(ustar));
 #pragma unroll 1
   for (int itr = 0; itr < ITRMX; itr++) {
     double zetalt = zslt * rlmo;
@@ -315,7 +295,7 @@ __device__ __forceinline__ void sfc_dif_off(double zlvl, double zlvl_wind, doubl
     cm = (cmn > cxch) ? cmn : cxch;
     ch = (chn > cxch) ? chn : cxch;
     wstar2 = wstar2_of(ch);
-    const double rlmn = fdiv(elfc * ch * dthv, xpow(ustar, 3.0));
+    const double rlmn = fdiv(elfc * ch * dthv, cube(ustar));
     rlmo = rlmo * WOLD + rlmn * wnew;
   }
 }
@@ -355,7 +335,7 @@ __device__ __forceinline__ void can_res(Col &c) {
   const double ff = 0.55 * 2.0 * c.soldn / (c.rgl * c.proj_lai);
   double rcs = (ff + c.rsmin / c.rsmax) / (1.0 + ff);
   rcs = (rcs > 0.0001) ? rcs : 0.0001;
-  const double dtopt = c.topt - c.sfctmp, t2 = c.sfctmp * c.sfctmp;
+  const double dtopt = c.topt - c.sfctmp;
   double rct = 1.0 - 0.0016 * (dtopt * dtopt);
   rct = (rct > 0.0001) ? rct : 0.0001;
   double rcq = 1.0 / (1.0 + c.hs * (c.q2sat - c.q2));
@@ -372,7 +352,7 @@ __device__ __forceinline__ void can_res(Col &c) {
   }
   rcsoil = (rcsoil > 0.0001) ? rcsoil : 0.0001;
   c.rc = c.rsmin / (c.proj_lai * rcs * rct * rcq * rcsoil);
-  const double rr = (4.0 * c.emissi * SIGMA * RD / NCP) * (t2 * t2) / (c.sfcprs * c.ch) + 1.0;
+  const double rr = (4.0 * c.emissi * SIGMA * RD / NCP) * fourth(c.sfctmp) / (c.sfcprs * c.ch) + 1.0;
   const double delta = (SLV / NCP) * c.dqsdt2;
   c.pc = (rr + delta) / (rr * (1.0 + c.rc * c.ch) + delta);
 }
@@ -382,7 +362,7 @@ __device__ __forceinline__ void d_evap(Col &c, const NoahUni &u) {
   const double sratio = (c.sh2o[0] - c.smcdry) / (c.smcmax - c.smcdry);
   double fx = 0.0;
   if (sratio > 0.0) {
-    fx = xpow(sratio, u.fxexp);
+    fx = pow_fine(sratio, u.fxexp);
     fx = (fx > 1.0) ? 1.0 : fx;
     fx = (fx < 0.0) ? 0.0 : fx;
   }
@@ -393,7 +373,7 @@ __device__ __forceinline__ void d_evap(Col &c, const NoahUni &u) {
 __device__ __forceinline__ void transp(Col &c) {
   for (int k = 0; k < c.nsoil; k++) c.et[k] = 0.0;
   double etpa;
-  if (c.cmc != 0.0) etpa = c.shdfac * c.pc * c.etp * (1.0 - xpow(c.cmc / c.cmcmax, c.cfactr));
+  if (c.cmc != 0.0) etpa = c.shdfac * c.pc * c.etp * (1.0 - pow_fine(c.cmc / c.cmcmax, c.cfactr));
   else etpa = c.shdfac * c.pc * c.etp;
   const Layers &gx = c.w1;
   double sgx = 0.0;
@@ -426,7 +406,7 @@ __device__ __forceinline__ void evapo(Col &c, const NoahUni &u, double dt) {
       transp(c);
       for (int k = 0; k < c.nsoil; k++) c.ett += c.et[k];
       if (c.cmc > 0.0)
-        c.ec = c.shdfac * xpow((c.cmc / c.cmcmax > 1.0) ? 1.0 : c.cmc / c.cmcmax, c.cfactr) * c.etp;
+        c.ec = c.shdfac * pow_fine((c.cmc / c.cmcmax > 1.0) ? 1.0 : c.cmc / c.cmcmax, c.cfactr) * c.etp;
       else
         c.ec = 0.0;
       const double cmc2ms = c.cmc / dt;
@@ -523,7 +503,7 @@ __device__ __forceinline__ double fr_h2o(double tkelv, double smc, double sh2o, 
   while (nlog < 10 && kcount == 0) {
     nlog++;
     const double satn = (smc - swl - smcmin) / range;
-    const double pw = xpow(satn, mx);          // satn^(mx-1) below is pw / satn
+    const double pw = pow_fine(satn, mx);          // satn^(mx-1) below is pw / satn
     double lp, lc;
     ln_of2(pw - 1.0, 1.0 + CK * swl, &lp, &lc);
     const double df = la + ibeta * lp + 2.0 * lc - lt;
@@ -537,7 +517,7 @@ __device__ __forceinline__ double fr_h2o(double tkelv, double smc, double sh2o, 
   }
   double freew = smc - swl;
   if (kcount == 0) {
-    double fk = xpow(xpow(-(tkelv - TFREEZ) / tkelv * alpha * LSUBF / NGRAV, beta), 1.0 / mx) * (smcmax - smcmin) -
+    double fk = pow_fine(pow_fine(-(tkelv - TFREEZ) / tkelv * alpha * LSUBF / NGRAV, beta), 1.0 / mx) * (smcmax - smcmin) -
                 smcmin;
     fk = (fk < SH2OMIN) ? SH2OMIN : fk;
     freew = (fk < smc) ? fk : smc;
@@ -590,7 +570,7 @@ __device__ __forceinline__ void sh_flx(Col &c, const NoahUni &u, double dt, doub
     } else {
       const bool last = k == nsoil - 1;
       const double zu = c.zsoil[k - 1], zk = c.zsoil[k], tn = last ? u.tbot : c.stc[k + 1];
-      const double df1n = tdf_cnd(smc, c.lks, c.smcmax, c.smcmin, sh2o);
+      const double df1n = tdf_cnd(smc, c.ksolid, c.smcmax, c.smcmin, sh2o);
       double ddz2 = ddz;                       // the last layer's goes unread
       if (last) {
         denom = 0.5 * (zu + zk) - u.zbot;
@@ -869,7 +849,7 @@ __device__ __forceinline__ void s_flx(Col &c, const NoahUni &u, double dt) {
     c.sncovr = (c.sncovr < 0.98) ? c.sncovr : 0.98;
     al_calc(c, u, dt, snowng);
   }
-  double df1 = tdf_cnd(c.smc[0], c.lks, c.smcmax, c.smcmin, c.sh2o[0]);
+  double df1 = tdf_cnd(c.smc[0], c.ksolid, c.smcmax, c.smcmin, c.sh2o[0]);
   df1 *= exp(u.sbeta * shdfac);
   if (c.sncovr > 0.97) df1 = c.sncond;
   const double dsoil = -(0.5 * c.zsoil[0]);
@@ -922,21 +902,21 @@ __global__ __launch_bounds__(kBlock) void k_noah_meteo(int nstation, int nrec, c
 // one wavefront's latency up to some 60,000 columns), and at 100,000 columns
 // two such chains one after the other, since the layers' 39 KB of LDS leave a
 // SIMD one wavefront.  So:
-// - every function is inlined and the column's record lives in registers (242,
+// - every function is inlined and the column's record lives in registers (231,
 //   nothing in scratch memory); the layer arrays, indexed at run time, are in
 //   LDS, where they cost neither registers nor scratch;
 // - the branches that columns of one wavefront take differently (snow or none,
 //   the top layer or one below) hold only what differs;
-// - the powers, and the logarithms of the exchange coefficients' fixed point,
-//   of the supercooled water's Newton iteration and of the layers'
-//   conductivities, are the shorter ones of xmath.hpp, and fewer.
+// - the powers and logarithms are xmath.hpp's fine ones, and fewer than the
+//   reference's.
 // Measured (us per step, 6,000 / 20,011 / 100,000 columns): 122 / 139 / 233
 // with calls and the record in scratch; 77.9 / 92.8 / 147.7 inlined (256
-// registers and 960 B of scratch); 53.3 / 60.5 / 125.5 with the shared branches
-// and the shorter functions at 474 registers, 66.2 / 87.2 / 139.7 at 256;
-// 41.9 / 47.9 / 92.5 with the layers in LDS.  Against the step in 80-bit
-// arithmetic on 100,000 columns its errors are the former kernel's to a few
-// per cent (exchange coefficient: 7.5e-16 in the mean, before and now).
+// registers and 960 B of scratch); with the shared branches and xmath.hpp's
+// short functions 53.3 / 60.5 / 125.5 at 474 registers, 66.2 / 87.2 / 139.7 at
+// 256, 41.7 / 47.6 / 92.5 with the layers in LDS; 43.8 / 49.7 / 96.5 with the
+// fine ones.  Those err by at most 0.66 ulp (power) and 0.52 (logarithm) over
+// the step's ranges, the device library's by 1.3 and 0.63, the short power by up
+// to 18.6.
 __global__ __launch_bounds__(kNoahBlock, 1) void k_noah(int ne, int nstation, NoahDev d, NoahUni u, ColDev s, double dt) {
   const int p = blockIdx.x * kNoahBlock + threadIdx.x;
   if (p >= ne) return;
@@ -969,7 +949,7 @@ __global__ __launch_bounds__(kNoahBlock, 1) void k_noah(int ne, int nstation, No
   c.albedomax = d.albedomax[p]; c.z0min = d.z0min[p]; c.z0max = d.z0max[p]; c.snup = d.snup[p];
   c.cfactr = d.cfactr[p]; c.rgl = d.rgl[p]; c.rsmin = d.rsmin[p]; c.rsmax = d.rsmax[p]; c.topt = d.topt[p];
   c.hs = d.hs[p]; c.smcref = d.smcref[p]; c.smcwlt = d.smcwlt[p]; c.smcdry = d.smcdry[p];
-  c.lks = ln_solids(d.quartz[p]); c.zlvl_wind = d.zlvl_wind[p];
+  c.ksolid = solids_power(d.quartz[p], s.smcmax[p]); c.zlvl_wind = d.zlvl_wind[p];
   c.smcmax = s.smcmax[p]; c.smcmin = s.smcmin[p]; c.alpha = s.alpha[p]; c.beta = s.beta[p];
   c.t1 = at(d.sc, 0); c.sneqv = at(d.sc, 1); c.snowh = at(d.sc, 2); c.sndens = at(d.sc, 3);
   c.cmc = at(d.sc, 4); c.ch = at(d.sc, 5); c.cm = at(d.sc, 6); c.snotime1 = at(d.sc, 7);

@@ -2388,21 +2388,25 @@ extern "C" int pihm_ctx_time_kernels(pihm_ctx *c, const double *y, double *ydot,
 }
 
 // ---------------------------------------------------------------------------
-// the flux functions' power routine, exposed for its accuracy tests
+// the flux functions' power routine and the land surface's functions, exposed
+// for their accuracy tests
 // ---------------------------------------------------------------------------
 
 namespace {
-__global__ __launch_bounds__(kBlock) void k_math_pow(int n, const double *x, const double *y, double *out) {
-  const int i = blockIdx.x * kBlock + threadIdx.x;
-  if (i < n) out[i] = xpow(x[i], y[i]);
+enum MathFn { M_POW = 0, M_POW_FINE, M_LN_FINE };
+__host__ __device__ inline double math_fn(int fn, double x, double y) {
+  return fn == M_POW ? xpow(x, y) : (fn == M_POW_FINE ? pow_fine(x, y) : ln_fine(x));
 }
-}  // namespace
+__global__ __launch_bounds__(kBlock) void k_math(int n, int fn, const double *x, const double *y, double *out) {
+  const int i = blockIdx.x * kBlock + threadIdx.x;
+  if (i < n) out[i] = math_fn(fn, x[i], y[i]);
+}
 
-extern "C" int pihm_math_pow(int n, const double *x, const double *y, double *out, int on_device) {
+int math_run(int fn, int n, const double *x, const double *y, double *out, int on_device) {
   if (n < 0 || (n > 0 && (!x || !y || !out))) return PIHM_ERR_ARG;
   if (n == 0) return PIHM_OK;
   if (!on_device) {
-    for (int i = 0; i < n; i++) out[i] = xpow(x[i], y[i]);
+    for (int i = 0; i < n; i++) out[i] = math_fn(fn, x[i], y[i]);
     return PIHM_OK;
   }
   double *d = nullptr;
@@ -2411,12 +2415,20 @@ extern "C" int pihm_math_pow(int n, const double *x, const double *y, double *ou
   hipError_t e = hipMemcpy(d, x, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(d + n, y, bytes, hipMemcpyHostToDevice);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_math_pow, dim3(div_up(n, kBlock)), dim3(kBlock), 0, 0, n, d, d + n, d + 2L * n);
+    hipLaunchKernelGGL(k_math, dim3(div_up(n, kBlock)), dim3(kBlock), 0, 0, n, fn, d, d + n, d + 2L * n);
     e = hipGetLastError();
   }
   if (e == hipSuccess) e = hipMemcpy(out, d + 2L * n, bytes, hipMemcpyDeviceToHost);
   (void)hipFree(d);
   return e == hipSuccess ? PIHM_OK : PIHM_ERR_HIP;
+}
+}  // namespace
+
+extern "C" int pihm_math_pow(int n, const double *x, const double *y, double *out, int on_device) {
+  return math_run(M_POW, n, x, y, out, on_device);
+}
+extern "C" int pihm_math_fine(int n, const double *x, const double *y, double *out, int on_device) {
+  return y ? math_run(M_POW_FINE, n, x, y, out, on_device) : math_run(M_LN_FINE, n, x, x, out, on_device);
 }
 
 // Average device time of one whole RHS evaluation (both kernels back to

@@ -271,4 +271,108 @@ PIHM_HD void xpow_n(const double (&x)[K], const double (&y)[K], double (&r)[K]) 
   for (int k = 0; k < K; k++) r[k] = (x[k] > 0.0 && x[k] < HUGE_VAL) ? r[k] : x[k];
 }
 
+// ---------------------------------------------------------------------------
+// The same two functions as the device library has them, to a little over half
+// an ulp, for the land-surface step, whose powers and logarithms were the
+// library's: what the short ones above leave out, the rounding of the
+// logarithm's quotient and of the exponential's sums, is carried along (some
+// 15 operations more for a power).
+
+// ln x = hi + lo for finite x > 0, the pair to about 3e-18 of its size.
+template <int K>
+PIHM_HD void ln_fine_n(const double (&x)[K], double (&hi)[K], double (&lo)[K]) {
+  double q[K], ql[K], s[K], p[K], de[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    int e;
+    double m = split_exp(x[k], &e);
+    if (m < 0.70710678118654752440) {
+      m = m + m;
+      e -= 1;
+    }
+    const double n = m - 1.0, d = m + 1.0, dl = m - (d - 1.0);   // n is exact, d + dl = m + 1
+    q[k] = log_ratio(m);                                         // n / d, rounded
+    // the rest of n / (d + dl); 1 / (m + 1) is (1 - q) / 2 as well as it needs to be
+    ql[k] = fma(-q[k], dl, fma(-q[k], d, n)) * fma(-0.5, q[k], 0.5);
+    s[k] = q[k] * q[k];
+    de[k] = (double)e;
+  }
+#define PIHM_STEP(c) { const double cc = coef(c); for (int k = 0; k < K; k++) p[k] = fma(p[k], s[k], cc); }
+  { const double cc = coef(1.0 / 21.0); for (int k = 0; k < K; k++) p[k] = cc; }
+  PIHM_STEP(1.0 / 19.0) PIHM_STEP(1.0 / 17.0) PIHM_STEP(1.0 / 15.0) PIHM_STEP(1.0 / 13.0) PIHM_STEP(1.0 / 11.0)
+  PIHM_STEP(1.0 / 9.0) PIHM_STEP(1.0 / 7.0) PIHM_STEP(1.0 / 5.0) PIHM_STEP(1.0 / 3.0)
+#undef PIHM_STEP
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const double f2 = q[k] + q[k], fl = ql[k] + ql[k];
+    // beyond 2 q: the series' other terms, at most a hundredth of it, and ql's share 2 ql / (1 - s)
+    const double t = fma(f2 * s[k], p[k], fma(fl, s[k], fl));
+    const double a = de[k] * kLn2Hi;               // exact
+    const double h = a + f2, l = (a - h) + f2;     // exact: |a| >= |f2| or a == 0
+    const double r = l + fma(de[k], kLn2Lo, t);
+    hi[k] = h + r;
+    lo[k] = (h - hi[k]) + r;
+  }
+}
+
+// e^(hi + lo) for any hi, |lo| <= ulp(hi).
+PIHM_HD double exp_fine(double hi, double lo) {
+  if (!(fabs(hi) < 1000.0)) return hi > 0.0 ? HUGE_VAL : (hi < 0.0 ? 0.0 : hi);   // the last: NaN
+  const double kk = rint(hi * 1.44269504088896340736);
+  const double r0 = fma(-kk, kLn2Hi, hi);          // exact
+  double rl = fma(-kk, kLn2Lo, lo);
+  const double r = r0 + rl;                        // |r| <= ln2 / 2 + 1e-10
+  rl = (r0 - r) + rl;
+  double p = coef(1.0 / 6227020800.0);
+#define PIHM_STEP(c) p = fma(p, r, coef(c));
+  PIHM_STEP(1.0 / 479001600.0) PIHM_STEP(1.0 / 39916800.0) PIHM_STEP(1.0 / 3628800.0) PIHM_STEP(1.0 / 362880.0)
+  PIHM_STEP(1.0 / 40320.0) PIHM_STEP(1.0 / 5040.0) PIHM_STEP(1.0 / 720.0) PIHM_STEP(1.0 / 120.0)
+  PIHM_STEP(1.0 / 24.0) PIHM_STEP(1.0 / 6.0)
+#undef PIHM_STEP
+  const double h = 1.0 + r, l = (1.0 - h) + r;     // exact
+  const double u = fma(rl, h, (r * r) * fma(p, r, 0.5));
+  return ldexp(h + (l + u), (int)kk);
+}
+
+// ln x for any x.
+PIHM_HD double ln_fine(double x) {
+  if (x > 0.0 && x < HUGE_VAL) {
+    const double xs[1] = {x};
+    double h[1], l[1];
+    ln_fine_n<1>(xs, h, l);
+    return h[0];                                   // h + l rounded
+  }
+  return (x == 0.0) ? -HUGE_VAL : ((x < 0.0) ? NAN : x);
+}
+
+// x^y as the C library's, special arguments included.
+PIHM_HD double pow_fine(double x, double y) {
+  double ax = x, r = 0.0;
+  bool neg = false, main_path = x > 0.0 && x < HUGE_VAL && fabs(y) < HUGE_VAL;
+  if (!main_path && !(x == 0.0 && y > 0.0 && !signbit(x))) {
+    ax = 0.0;
+    r = pow_special(x, y, &ax, &neg);
+    main_path = ax > 0.0;
+  }
+  if (main_path) {
+    const double xs[1] = {ax};
+    double h[1], l[1], tlo;
+    ln_fine_n<1>(xs, h, l);
+    const double thi = mul_pair(y, h[0], l[0], &tlo);
+    r = exp_fine(thi, tlo);
+    if (neg) r = -r;
+  }
+  return r;
+}
+
+// x^3 and x^4, a rounding apart from the exact product's rounding.
+PIHM_HD double cube(double x) {
+  const double s = x * x, c = s * x;
+  return c + fma(fma(x, x, -s), x, fma(s, x, -c));
+}
+PIHM_HD double fourth(double x) {
+  const double s = x * x, q = s * s;
+  return q + fma(2.0 * s, fma(x, x, -s), fma(s, s, -q));
+}
+
 }  // namespace pihm
