@@ -35,8 +35,8 @@ BYTES_PER_SEG = 200      # ... per river segment
 # FETCH_SIZE x 2.000 (262,157 KiB read back for 524,288 KiB copied), WRITE_SIZE x 1.000.
 # One launch (k_rhs_tile): 36,630.0 x 2 + 4,821.8 KiB.  Two kernels (k_prep + k_flux):
 # (13,766.3 + 28,852.0) x 2 + (12,919.4 + 4,818.1) KiB.
-RHS_TRAFFIC_BYTES = {"one launch": (36630.0 * 2.0 + 4821.8) * 1024,
-                     "two kernels": ((13766.3 + 28852.0) * 2.0 + (12919.4 + 4818.1)) * 1024}
+RHS_TRAFFIC_BYTES = {"one launch": (36751.0 * 2.0 + 4821.9) * 1024,
+                     "two kernels": ((13773.9 + 28262.4) * 2.0 + (12919.4 + 4818.1)) * 1024}
 RHS_KERNELS = {"one launch": "one RHS evaluation (k_rhs_tile: one launch, tile records in LDS)",
                "two kernels": "one RHS evaluation (k_prep + k_flux, back to back)"}
 # Land-surface step (k_intcp_snow_et), algorithmic bytes per element: 15 FP64 parameters
@@ -215,7 +215,8 @@ def _ops_roofline(a, b):
     if n <= 0 or ms <= 0.0:
         return None
     gbps = by / (ms * 1e-3) / 1e9
-    return {"kernel": "k_ens_ops (every ready member's queued vector operations, one launch)",
+    return {"kernel": "k_ens_ops (every ready member's queued vector operations, one launch), sampled: "
+                      "the first launches of a run's first tick and of every 16th after it",
             "launches_timed": n, "bytes_per_launch": by / n, "us_per_launch": ms * 1e3 / n,
             "achieved": gbps, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": gbps / HBM_PEAK_GBS}
 
@@ -351,17 +352,17 @@ def producers_run(mesh, seed, iters=200):
                                   "traffic": LSM_TRAFFIC_BYTES}},
         "bc_apply": {"ms": ms_b.value, "algorithmic_bytes": bc_bytes,
                      "achieved_GBps": bc_bytes / (ms_b.value * 1e-3) / 1e9,
-                     "note": "two launches over 600k edge codes: launch-latency bound"},
+                     "note": "one launch over 600k edge codes: launch-latency bound"},
     }
 
 
 NOAH_EXTRA_BYTES_PER_ELEM = 32   # smcmin, sh2o[0], fcr, gwet read by the _NOAH_ branches
 # HBM bytes per launch at the 100,000-triangle mesh from the FETCH_SIZE and WRITE_SIZE passes
 # (FETCH_SIZE x 2, calibrated on the copy kernel): one Noah RHS on the one-launch path
-# (k_rhs_tile with the _NOAH_ branches: 18,711.1 x 2 + 2,411.0 KiB), one soil-water step
-# (28,417.5 x 2 + 46,484.4 KiB)
-NOAH_RHS_TRAFFIC_BYTES = (18711.1 * 2.0 + 2411.0) * 1024
-NOAH_SOIL_TRAFFIC_BYTES = (28417.5 * 2.0 + 46484.4) * 1024
+# (k_rhs_tile with the _NOAH_ branches: 18,708.1 x 2 + 2,411.0 KiB), one soil-water step
+# (28,417.8 x 2 + 46,484.4 KiB)
+NOAH_RHS_TRAFFIC_BYTES = (18708.1 * 2.0 + 2411.0) * 1024
+NOAH_SOIL_TRAFFIC_BYTES = (28417.8 * 2.0 + 46484.4) * 1024
 # algorithmic bytes of the soil-water step per element: reads 4 layer fields (sldpth, smc, sh2o, et;
 # 352 B), 12 FP64 scalars and 2 int32 (104 B); writes 5 layer fields (satdpth, runoff2_lyr, smflxv,
 # smc, sh2o; 440 B), 4 FP64 scalars and nwtbl (36 B)
@@ -425,7 +426,7 @@ def noah_rhs_run(seed, iters=200, coupled=True):
                          "ms_per_step": soil_ms, "layers": MAXLYR, "algorithmic_bytes": soil_bytes,
                          "achieved_GBps": soil_bytes / (soil_ms * 1e-3) / 1e9,
                          "traffic": NOAH_SOIL_TRAFFIC_BYTES,
-                         "note": "once per model step; one thread per element column"},
+                         "note": "once per model step; four wavefronts per 64 element columns"},
            "note": "per-LSM-step values (edir, ett, per-layer et) held fixed: the RHS and the soil-water "
                    "step alone; the coupled run with the Noah step is the flux_pihm object"}
     if not coupled:
@@ -596,7 +597,7 @@ def physical_cores():
 # 200,000-triangle workload (SQ_INSTS_VALU / SQ_WAVES, the same profile passes as the traffic).
 # A wavefront's FP64 instruction occupies a SIMD for 4 cycles (16 lanes per cycle); the chip
 # has 1,024 SIMDs at 2.4 GHz.
-RHS_VALU = {"one launch": [(1175.2, 3382)], "two kernels": [(229.9, 3320), (1174.2, 3192)]}
+RHS_VALU = {"one launch": [(1226.2, 3382)], "two kernels": [(229.9, 3320), (1183.1, 3192)]}
 SIMDS, CLOCK_MHZ = 1024, 2400.0
 
 

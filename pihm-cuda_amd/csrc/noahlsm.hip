@@ -1,8 +1,11 @@
 // noahlsm.hip - the Noah land-surface step of the _NOAH_ build on the device.
 //
 // One thread per element runs Noah() (src/noah/noah.c:3-55): the humidity
-// terms, the moisture clamps and SFlx (:166-609) with every routine it calls,
-// in the reference's operation order.  The soil column (smc, sh2o, at most 11
+// terms, the moisture clamps and SFlx (:166-609) with every routine it calls.
+// Sums and products keep the reference's operation order but for Paulson's
+// functions, whose differences are one logarithm (sfc_dif_off), FrH2O's second
+// power, which is the first over its base, and whole-number powers, which are
+// products rounded once.  The soil column (smc, sh2o, at most 11
 // layers) is shared with the soil-water step and lives in HBM layer-major
 // ([k * ne + p]) so that a wavefront reads one layer of 64 neighbouring
 // elements together; the temperatures stc are stored the same way.  The

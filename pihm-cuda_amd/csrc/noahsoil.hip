@@ -1,16 +1,17 @@
 // noahsoil.hip - the _NOAH_ build's soil-water step after each model step.
 //
-// One thread per element runs the element's soil column in the reference's
-// order: Summary's FindWaterTable and CalcLatFlx (src/update.c:37-43), then
-// NoahHydrol (src/noah/noah.c:57-94): FindWaterTable again, the moisture
+// Each element's soil column: Summary's FindWaterTable and CalcLatFlx
+// (src/update.c:37-43), then NoahHydrol (src/noah/noah.c:57-94): the moisture
 // clamps, and SmFlx with SRT, SStep, Rosr12 and AdjSmProf.  The layer arrays
-// live in HBM layer-major ([k * ne + p]) so that the threads of a wavefront
-// read one layer of 64 neighbouring elements together; inside the thread the
-// column (at most 11 layers) is worked in private arrays.  Every expression
-// keeps the reference's operation order; powers use xpow (as the RHS does) and
-// exp is the device library's.  At the end the thread leaves in the context
-// what the next model step's RHS reads: sh2o[0], fcr, nwtbl and GwTransp's
-// share (src/noah/lsm_func.c:163-185) for the new water-table layer.
+// live in HBM layer-major ([k * ne + p]) so that a wavefront reads one layer of
+// 64 neighbouring elements together; four wavefronts work on 64 columns (at
+// most 11 layers each) in LDS.  The water table, the lateral split, the clamps
+// and the solve keep the reference's operation order.  The conductivity and
+// the retention curve's slope share their powers (kr_slope), which are xpow's,
+// as in the RHS; the ice factor's cube is two products, and exp is the device
+// library's.  At the end the step leaves in the context what the next model
+// step's RHS reads: sh2o[0], fcr, nwtbl and GwTransp's share
+// (src/noah/lsm_func.c:163-185) for the new water-table layer.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -131,7 +132,10 @@ __device__ __forceinline__ void wdf_cnd(double *wdf, double *wcnd, double smc, c
 // divisions, and 932 B per column of memory.  Measured (us per step, 6,000 /
 // 20,011 / 100,000 columns of 11 layers): 42.4 / 46.8 / 104.6 with one thread
 // per column, the column in registers (316 VGPRs, one wavefront per SIMD) and
-// five powers per layer; 32.5 / 37.0 / 85.2 with the powers shared; this form 17.8 / 22.6 / 52.0.
+// five powers per layer; 32.5 / 37.0 / 85.2 with the powers shared; this form
+// 17.8 / 22.6 / 52.0.  The compiler reserves 100 B of scratch per lane for it
+// (the water table's two layer arrays and arguments); a build without any took
+// 17.8 / 22.7 / 52.3.
 constexpr int kSoilCols = 64, kSoilWaves = 4;
 
 __global__ __launch_bounds__(kSoilCols * kSoilWaves, 4) void k_noah_soil(int ne, SoilDev s, ElemDev e,

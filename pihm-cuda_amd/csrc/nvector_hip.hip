@@ -5,10 +5,10 @@
 // a == b and a*(x-y) when a == -b, (a*x)+(b*y) otherwise, which equals every
 // special case of the serial version bit for bit.
 //
-// Reductions run in two launches: each workgroup reduces a fixed, strided set
-// of entries (wavefront shuffles, then LDS) and writes its partial; one
-// workgroup then adds the partials in workgroup order and writes the result
-// to pinned host memory.  The summation tree depends
+// Reductions: each workgroup reduces a fixed, strided set of entries (lane
+// moves inside a wavefront, then LDS) and writes its partial; one workgroup, the
+// last to finish or a second launch's (redux.hpp), then combines the partials in
+// workgroup order and writes the result to pinned host memory.  The tree depends
 // only on the length, so results are reproducible bit for bit.
 #include <hip/hip_runtime.h>
 

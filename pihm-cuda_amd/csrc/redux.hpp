@@ -15,11 +15,19 @@
 //
 // Both passes are bound by latency.  The second pass took 5.7 us a launch in
 // the 200,000-triangle run with one slot's butterfly after the other through
-// the LDS, 2.8-3.7 us with the slots in step and lane moves (lanes.hpp).  The
-// line at 64 workgroups (32,768 entries): at 18,000 entries (36 workgroups) an
-// hour of a 6,000-triangle run takes 68.3 ms with the second launch and 63.2
-// with the ticket; at 1,024 workgroups their tickets queue up on one address
-// and 20 minutes at 200,000 triangles take 108 ms against 89.
+// the LDS, 2.8-3.7 us with the slots in step and lane moves (lanes.hpp).
+//
+// The line at 64 workgroups (32,768 entries) is on the safe side.  A dot product
+// and the Arnoldi step's six sums, from the call to the result (us, two launches
+// / one), by workgroups:
+//     36: 11.3 / 9.3, 13.9 / 12.3     64: 11.3 / 9.5, 14.1 / 12.4
+//    119: 11.4 / 10.0, 14.0 / 12.9   160: 11.3 / 10.5, 14.1 / 13.4
+//    256: 11.4 / 11.6, 14.2 / 14.6   512: 11.3 / 14.7, 14.7 / 17.5
+//   1024: 11.4 / 20.7, 16.4 / 24.2
+// Every further workgroup's ticket waits its turn at one address, about 10 ns
+// each: the single launch is ahead up to some 200 workgroups, and whole runs say
+// the same (20,011 triangles, 119 workgroups: 25.5 / 23.1 ms for 12 minutes;
+// 60,000, 355: 21.6 / 21.7 for 8; 200,000, 1,024: 10.1 / 11.9 for 4).
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cfloat>

@@ -1060,15 +1060,16 @@ __device__ __forceinline__ double tile_sfmag(const RhsArgs &a, int s, long q, co
 //
 // What bounds it: at 200,000 triangles the phases run one after the other on
 // every SIMD, memory (about 14 us of the time, 430 B per element) and then the
-// FP64 issue of the fluxes; on small meshes the one wavefront of a SIMD walks
-// its chain of dependent operations alone.  Measured (us per evaluation, wet
+// fluxes, whose chains of dependent FP64 operations three wavefronts do not
+// hide (1,226 vector instructions a wavefront are 6.7 us of a SIMD's issue); on
+// small meshes the one wavefront of a SIMD walks its chain alone.  Measured (us per evaluation, wet
 // state, 535 / 6,000 / 20,011 / 100,000 / 200,000 triangles): 14.5 / 15.3 /
 // 15.3 / 20.3 / 31.0 with one edge after the other and the compiler's
 // divisions; 11.7 / 12.6 / 12.6 / 16.9 / 27.3 with the faces and powers in
 // step, divisions that share reciprocals, and nothing spilled (157 VGPRs,
 // three wavefronts per SIMD).  Held to 128 VGPRs for a fourth wavefront it
-// spills, and a kernel with any scratch memory costs more than the wavefront
-// gives (28.1 against 25.3 in an otherwise equal pair).  Tiles of 64 / 256
+// spills, and the scratch memory costs more than the wavefront gives (28.1
+// against 25.3 in an otherwise equal pair).  Tiles of 64 / 256
 // elements: 7% / 12% slower at 20,011, equal / 4% slower at 200,000.
 //
 // The river blocks read their own copy of the arguments (ra): with one copy
@@ -2230,9 +2231,12 @@ __global__ void k_nan_report(int *flag, int *host_flag, volatile unsigned *host_
 
 // Reads and clears the sticky NaN flag; everything queued on the stream before
 // the call is done when it returns.  The host spins on the report's number and
-// after 2 ms falls back to the runtime's wait, which also reports errors: 19.9 us
-// for an evaluation of 535 triangles with its check, 24.9 with a copy of the
-// flag and the runtime's wait.  Every report has a number of its own, given by
+// after 2 ms falls back to the runtime's wait, which also reports errors.  In a
+// row of evaluations of 535 triangles each takes 19.6 us with its check, 24.9
+// with a copy of the flag and the runtime's wait.  The launches are retired by
+// the caller's next wait of the runtime, which then takes as much longer: one
+// evaluation and one such wait are 31.2 us either way.  A program whose next
+// waits spin too (the reductions here) keeps the gain.  Every report has a number of its own, given by
 // the host whether or not the launch succeeds, so none is taken for another;
 // an error that an earlier call left with the thread is not this launch's.
 extern "C" int pihm_ctx_poll_nan(pihm_ctx *c) {
