@@ -703,8 +703,9 @@ __device__ __forceinline__ ChanSide chan_side(const RiverDev &R, const double *y
   c.stage = clamp0(ys[r]);
   c.zbed = R.zbed[r];
   c.total_h = c.stage + c.zbed;
-  c.perim = riv_perim(R.ord[r], c.stage, R.coeff[r]);
-  c.crossa = riv_cs_area(R.ord[r], c.stage, R.coeff[r]);
+  const Section s = riv_section(R.ord[r], c.stage, R.coeff[r]);
+  c.perim = s.perim;
+  c.crossa = s.area;
   c.rough = R.rough[r];
   c.length = R.length[r];
   return c;
@@ -749,8 +750,8 @@ __device__ __forceinline__ void river_out(const RhsArgs &a, const double *ys, co
         const double total_h = stage + zbed;
         const double distance = 0.5 * length;
         const double grad_h = (total_h - bcv) / distance;
-        const double perim = riv_perim(ord, stage, coeff);
-        const double crossa = riv_cs_area(ord, stage, coeff);
+        const Section sec = riv_section(ord, stage, coeff);
+        const double perim = sec.perim, crossa = sec.area;
         const double avg_h = (perim == 0.0) ? 0.0 : (crossa / perim);
         flux = overland_flow(avg_h, grad_h, grad_h, crossa, R.rough[r]);
       } else {
@@ -767,8 +768,8 @@ __device__ __forceinline__ void river_out(const RhsArgs &a, const double *ys, co
         const double total_h = stage + zbed;
         const double distance = 0.5 * length;
         const double grad_h = (total_h - bcv) / distance;
-        const double perim = riv_perim(ord, stage, coeff);
-        const double crossa = riv_cs_area(ord, stage, coeff);
+        const Section sec = riv_section(ord, stage, coeff);
+        const double perim = sec.perim, crossa = sec.area;
         const double avg_h = (perim == 0.0) ? 0.0 : (crossa / perim);
         q = overland_flow(avg_h, grad_h, grad_h, crossa, R.rough[r]);
         break;
@@ -777,13 +778,13 @@ __device__ __forceinline__ void river_out(const RhsArgs &a, const double *ys, co
       case ZERO_DPTH_GRAD: {
         const double distance = 0.5 * length;
         const double grad_h = (zbed - (R.node_zmax[r] - R.depth[r])) / distance;
-        const double perim = riv_perim(ord, stage, coeff);
-        const double crossa = riv_cs_area(ord, stage, coeff);
+        const Section sec = riv_section(ord, stage, coeff);
+        const double perim = sec.perim, crossa = sec.area;
         q = sqrt(grad_h) * crossa * ((perim > 0.0) ? xpow(crossa / perim, 2.0 / 3.0) : 0.0) / R.rough[r];
         break;
       }
       default: {  // CRIT_DPTH (other codes rejected at creation)
-        const double crossa = riv_cs_area(ord, stage, coeff);
+        const double crossa = riv_section(ord, stage, coeff).area;
         q = crossa * sqrt(GRAV * stage);
         break;
       }
